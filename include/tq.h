@@ -261,23 +261,39 @@ int tq_gemv_w4g128_tiled(const uint16_t* x_bf16, int64_t m, const uint8_t* packe
 /* Prefill-shaped W8A8: activations already quantized per row (use
  * tq_quantize_i8_rowwise on X).  acc[i,j] = sum_p qa[i,p]*qw[j,p] (int32,
  * bit-exact); y = fma(f32(acc) * sa[i], sw[j], bias[j] or 0).  acc may be NULL.
- * Any M, N, K.  The MFMA kernels serve N % 16 == 0 and K % 16 == 0 (M <= 16 with
- * K % 64 == 0 and K <= 8192: a skinny kernel of N/16 blocks, 16 weight rows each;
- * the LDS-DMA kernel K % 128 == 0) with 16-byte aligned qa, qw, sw, bias, y and
- * acc; other cases take a shape-general kernel. */
+ * Any M, N, K and any alignment of the codes, all on the i8 MFMA.  M <= 16 with
+ * N % 16 == 0, K % 64 == 0 and K <= 8192 (16-byte aligned operands): a skinny
+ * kernel of N/16 blocks, 16 weight rows each; the LDS-DMA kernel's 128 x 256 tiles
+ * where K % 128 == 0 and they fill the chip; register-staged tiles otherwise. */
 int tq_gemm_w8a8(const int8_t* qa, const float* sa, const int8_t* qw, const float* sw,
                  const float* bias, int64_t m, int64_t n, int64_t k, int32_t* acc,
                  float* y, tq_stream_t stream);
 
+/* The same with a workspace (device memory, 8-byte aligned, at least
+ * tq_gemm_w8a8_workspace_bytes(M, N, K) bytes, contents need not be initialised):
+ * where the output tiles leave compute units idle, K is split over blocks, whose
+ * int32 partial sums meet there (the same acc and y, bit for bit). */
+int64_t tq_gemm_w8a8_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tq_gemm_w8a8_ws(const int8_t* qa, const float* sa, const int8_t* qw, const float* sw,
+                    const float* bias, int64_t m, int64_t n, int64_t k, int32_t* acc,
+                    void* workspace, int64_t workspace_bytes, float* y, tq_stream_t stream);
+
 /* Prefill-shaped FP8 W8A8 (both operands per-row E4M3, tq_quantize_fp8_rowwise):
  * y[i,j] = fma(f32(sum_p e4m3(qa[i,p]) * e4m3(qw[j,p])) * sa[i], sw[j], bias[j] or 0);
  * products exact, f32 accumulation.  The reference value is Linear over the
- * dequantized operands (linear.rs:111-121, tensor_ops.rs:379-410).  Any M, N,
- * K.  The FP8 MFMA kernels serve K % 128 == 0 and N % 16 == 0 with 16-byte
- * aligned qa, qw, sw, bias and y (M <= 16 with K <= 8192: a skinny kernel of N/16
- * blocks); other cases take a shape-general kernel. */
+ * dequantized operands (linear.rs:111-121, tensor_ops.rs:379-410).  Any M, N, K
+ * and alignment.  The FP8 MFMA kernels serve K % 128 == 0 and N % 16 == 0 with
+ * 16-byte aligned qa, qw, sw, bias and y (M <= 16 with K <= 8192: a skinny kernel of
+ * N/16 blocks); other cases widen the codes to bf16 (exact) for the bf16 MFMA. */
 int tq_gemm_fp8(const uint8_t* qa, const float* sa, const uint8_t* qw, const float* sw,
                 const float* bias, int64_t m, int64_t n, int64_t k, float* y, tq_stream_t stream);
+
+/* The same with a workspace, as tq_gemm_w8a8_ws (f32 or f64 partial sums, added in
+ * a fixed order). */
+int64_t tq_gemm_fp8_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tq_gemm_fp8_ws(const uint8_t* qa, const float* sa, const uint8_t* qw, const float* sw,
+                   const float* bias, int64_t m, int64_t n, int64_t k, void* workspace,
+                   int64_t workspace_bytes, float* y, tq_stream_t stream);
 
 /* Prefill-shaped W4A16: x bf16 [M, K], INT4 g128 weights, f32 accumulation with
  * the group scale applied to each 128-long partial sum; y f32 [M, N].

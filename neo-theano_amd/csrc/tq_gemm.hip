@@ -12,7 +12,7 @@
 // the byte-to-lane assignment that suits its loads; integer accumulation makes
 // the order invisible in the result.
 //
-// Two kernels:
+// Three kernels:
 //  * k_gemm_w8a8_dma (K % 128 == 0): one 256-thread block per 128 (m) x 256 (n)
 //    tile.  K advances in 128-byte stages through a 3-deep LDS ring filled by
 //    global_load_lds_dwordx4 (global -> LDS without registers; one instruction
@@ -24,137 +24,26 @@
 //    instructions of the stage after next interleaved with it, so that neither
 //    LDS latency nor a full memory queue idles the matrix core.  The epilogue
 //    goes through LDS to write 512-byte row segments.
-//  * k_gemm_w8a8 (any K % 16 == 0): 128 x 128 tiles of v_mfma_i32_16x16x64_i8
-//    with register-staged LDS loads.
+//  * k_gemm_tile (tq_gemm_tile.h; any M, N, K, any alignment): smaller tiles, K
+//    split over blocks where they leave CUs idle, for the M and N that do not fill
+//    the chip with 128 x 256 tiles and the shapes the LDS DMA cannot load.  Which
+//    one runs is tile_plan's estimate: at M = 64, N = 4096, K = 14336 the tiles
+//    take 15 us against 70 us for sixteen DMA blocks; at M = 2048, N = K = 4096
+//    the DMA kernel's 36 us stand against 51 us.
 #include "tq_internal.h"
 
 namespace tq {
 namespace {
 
-constexpr int kBlock = 256;
-constexpr int kTileN = 128;   // weight rows per block
-constexpr int kTileM = 128;   // activation rows per block
-constexpr int kTileK = 128;   // bytes of K per stage
-constexpr int kLdsRow = kTileK + 16;
-
 __device__ __forceinline__ i32x4 mfma_i8(i32x4 a, i32x4 b, i32x4 c) {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
-
-// Block tile order: an XCD receives every 8th block; renumber so that the 8
-// blocks resident on one XCD at a time share weight tiles (column-major over m).
-__device__ __forceinline__ void tile_of(int64_t bid, int64_t tiles_m, int64_t* tn, int64_t* tm) {
-    *tn = bid / tiles_m;
-    *tm = bid % tiles_m;
-}
-
-__global__ __launch_bounds__(kBlock, 2) void k_gemm_w8a8(const int8_t* __restrict__ qa,
-                                                         const float* __restrict__ sa,
-                                                         const int8_t* __restrict__ qw,
-                                                         const float* __restrict__ sw,
-                                                         const float* __restrict__ bias, int64_t m,
-                                                         int64_t n, int64_t k,
-                                                         int32_t* __restrict__ acc_out,
-                                                         float* __restrict__ y) {
-    __shared__ __attribute__((aligned(16))) int8_t lds_w[kTileN * kLdsRow];
-    __shared__ __attribute__((aligned(16))) int8_t lds_a[kTileM * kLdsRow];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wn = wave >> 1, wm = wave & 1;  // 2 x 2 waves, each 64 n x 64 m
-    const int64_t tiles_m = (m + kTileM - 1) / kTileM;
-    int64_t tn, tm;
-    tile_of(blockIdx.x, tiles_m, &tn, &tm);
-    const int64_t n0 = tn * kTileN, m0 = tm * kTileM;
-
-    // global -> register staging: thread t moves 16 B chunks (row t/8 + 32i, col 16*(t%8))
-    const int ld_row = tid >> 3, ld_col = (tid & 7) * 16;
-    i32x4 pw[4], pa[4];
-    auto load_stage = [&](int64_t k0) {
-        const bool kval = k0 + ld_col < k;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t rn = n0 + ld_row + 32 * i, rm = m0 + ld_row + 32 * i;
-            pw[i] = (kval && rn < n) ? *reinterpret_cast<const i32x4*>(qw + rn * k + k0 + ld_col)
-                                     : i32x4{0, 0, 0, 0};
-            pa[i] = (kval && rm < m) ? *reinterpret_cast<const i32x4*>(qa + rm * k + k0 + ld_col)
-                                     : i32x4{0, 0, 0, 0};
-        }
-    };
-    auto store_stage = [&]() {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            *reinterpret_cast<i32x4*>(lds_w + (ld_row + 32 * i) * kLdsRow + ld_col) = pw[i];
-            *reinterpret_cast<i32x4*>(lds_a + (ld_row + 32 * i) * kLdsRow + ld_col) = pa[i];
-        }
-    };
-
-    i32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
-
-    const int64_t ksteps = (k + kTileK - 1) / kTileK;
-    load_stage(0);
-    store_stage();
-    __syncthreads();
-
-    // MFMA operand rows: lane l reads row (l % 16) of a 16-row sub-tile, bytes
-    // [16 * (l / 16), +16) of each 64-byte K step.
-    const int op_row = lane & 15, op_k = (lane >> 4) * 16;
-    for (int64_t ks = 0; ks < ksteps; ++ks) {
-        if (ks + 1 < ksteps) load_stage((ks + 1) * kTileK);
-#pragma unroll
-        for (int kk = 0; kk < kTileK; kk += 64) {
-            i32x4 a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = *reinterpret_cast<const i32x4*>(lds_w + (wn * 64 + i * 16 + op_row) * kLdsRow + kk + op_k);
-                b[i] = *reinterpret_cast<const i32x4*>(lds_a + (wm * 64 + i * 16 + op_row) * kLdsRow + kk + op_k);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = mfma_i8(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
-        if (ks + 1 < ksteps) {
-            store_stage();
-            __syncthreads();
-        }
-    }
-
-    // epilogue: lane holds D[n = 4*(l/16) + r][m = l % 16] of each 16x16 tile
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t nb = n0 + wn * 64 + i * 16 + (lane >> 4) * 4;
-        if (nb >= n) continue;
-        const f32x4 swv = *reinterpret_cast<const f32x4*>(sw + nb);
-        f32x4 bv = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (bias) bv = *reinterpret_cast<const f32x4*>(bias + nb);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t mm = m0 + wm * 64 + j * 16 + (lane & 15);
-            if (mm >= m) continue;
-            const i32x4 c = acc[i][j];
-            if (acc_out) *reinterpret_cast<i32x4*>(acc_out + mm * n + nb) = c;
-            const float s_row = sa[mm];
-            f32x4 o;
-            o.x = fmaf(static_cast<float>(c.x) * s_row, swv.x, bv.x);
-            o.y = fmaf(static_cast<float>(c.y) * s_row, swv.y, bv.y);
-            o.z = fmaf(static_cast<float>(c.z) * s_row, swv.z, bv.z);
-            o.w = fmaf(static_cast<float>(c.w) * s_row, swv.w, bv.w);
-            *reinterpret_cast<f32x4*>(y + mm * n + nb) = o;
-        }
-    }
-}
-
 
 }  // namespace
 }  // namespace tq
 
 #include "tq_gemm_dma.h"
+#include "tq_gemm_tile.h"
 
 namespace tq {
 namespace {
@@ -399,29 +288,66 @@ __global__ __launch_bounds__(kSkinnyBlock) void k_gemm_fp8_skinny(const int8_t* 
 }  // namespace
 }  // namespace tq
 
-using namespace tq;
+namespace tq {
+namespace {
 
-extern "C" int tq_gemm_w8a8(const int8_t* qa, const float* sa, const int8_t* qw, const float* sw,
-                            const float* bias, int64_t m, int64_t n, int64_t k, int32_t* acc,
-                            float* y, tq_stream_t stream) {
-    TQ_REQUIRE(m >= 0 && n >= 0 && k >= 0, "tq_gemm_w8a8: negative shape");
+// Decode batches (M <= 16) of the operands the MFMA kernels' vectors take run the
+// skinny kernels: K <= 8192, runs of up to 8 64-byte chunks per wave, whose loads
+// all fit the registers.
+bool i8_vectors(const void* qa, const void* qw, const void* sw, const void* bias, const void* y, const void* acc,
+                int64_t n, int64_t k) {
+    return k > 0 && n % 16 == 0 && k % 16 == 0 && aligned(qa, 16) && aligned(qw, 16) && aligned(sw, 16) &&
+           aligned(y, 16) && (!acc || aligned(acc, 16)) && (!bias || aligned(bias, 16));
+}
+bool i8_skinny(int64_t m, int64_t n, int64_t k) {
+    return m <= 16 && k % 64 == 0 && k <= 8192 && n < (int64_t(1) << 31);
+}
+bool fp8_skinny(int64_t m, int64_t k) { return m <= 16 && k <= 8192; }
+
+// ns per 128-byte stage of the DMA kernels' 128 x 256 tiles (M = 2048, N = K = 4096)
+constexpr int kDmaStageI8 = 1000, kDmaStageF8 = 950;
+
+TileArgs a8_args(const void* qa, const float* sa, const void* qw, const float* sw, const float* bias, int64_t m,
+                 int64_t n, int64_t k, int32_t* acc, float* y, void* part) {
+    TileArgs p{};
+    p.a = qa;
+    p.w = qw;
+    p.sa = sa;
+    p.sw = sw;
+    p.bias = bias;
+    p.m = static_cast<int>(m);
+    p.n = static_cast<int>(n);
+    p.k = static_cast<int>(k);
+    p.lda = p.k;
+    p.acc = acc;
+    p.y = y;
+    p.part = part;
+    return p;
+}
+
+// Bytes of partial sums the largest plan of these sizes may take (the operands'
+// alignment, which picks among the kernels, is not known here).
+template <class T>
+int64_t a8_part_bytes(int64_t m, int64_t n, int64_t k) {
+    if (m <= 0 || n <= 0 || k <= 0 || !tile_fits(m, n, k)) return 0;
+    return tile_plan<T>(m, n, k, 0, true).part_bytes;
+}
+
+int gemm_w8a8(const int8_t* qa, const float* sa, const int8_t* qw, const float* sw, const float* bias, int64_t m,
+              int64_t n, int64_t k, int32_t* acc, void* ws, int64_t ws_bytes, float* y, hipStream_t st,
+              const char* what) {
+    TQ_REQUIRE(m >= 0 && n >= 0 && k >= 0, "%s: negative shape", what);
     if (m == 0 || n == 0) return TQ_OK;
-    TQ_REQUIRE(sa && sw && y && (k == 0 || (qa && qw)), "tq_gemm_w8a8: null pointer");
+    TQ_REQUIRE(sa && sw && y && (k == 0 || (qa && qw)), "%s: null pointer", what);
     TQ_REQUIRE(aligned(sa, 4) && aligned(sw, 4) && aligned(y, 4) && (!acc || aligned(acc, 4)) &&
                    (!bias || aligned(bias, 4)),
-               "tq_gemm_w8a8: misaligned pointer");
-    // the MFMA kernels tile N by 16 rows, K by 16-byte vectors, and store 16-byte vectors
-    if (k == 0 || n % 16 != 0 || k % 16 != 0 || !aligned(qa, 16) || !aligned(qw, 16) || !aligned(sw, 16) ||
-        !aligned(y, 16) || (acc && !aligned(acc, 16)) || (bias && !aligned(bias, 16)))
-        return launch_gemm_w8a8_generic(qa, sa, qw, sw, bias, m, n, k, acc, y, as_hip(stream));
-    // decode batches: the skinny kernel, N / 16 blocks (K <= 8192: runs of up to 8
-    // chunks per wave, whose loads all fit the registers)
-    if (m <= 16 && k % 64 == 0 && k <= 8192 && n < (int64_t(1) << 31)) {
+               "%s: misaligned pointer", what);
+    const bool vec = i8_vectors(qa, qw, sw, bias, y, acc, n, k);
+    if (vec && i8_skinny(m, n, k)) {
         const int64_t cpw = ((k >> 6) + kSkinnyWaves - 1) / kSkinnyWaves;
         const unsigned grid = static_cast<unsigned>(n / 16);
         const int mi = static_cast<int>(m), ni = static_cast<int>(n);
-#define TQ_SKINNY(P) \
-    k_gemm_w8a8_skinny<P><<<grid, kSkinnyBlock, 0, as_hip(stream)>>>(qa, sa, qw, sw, bias, mi, ni, k, acc, y)
+#define TQ_SKINNY(P) k_gemm_w8a8_skinny<P><<<grid, kSkinnyBlock, 0, st>>>(qa, sa, qw, sw, bias, mi, ni, k, acc, y)
         if (cpw <= 1)
             TQ_SKINNY(1);
         else if (cpw <= 2)
@@ -431,59 +357,96 @@ extern "C" int tq_gemm_w8a8(const int8_t* qa, const float* sa, const int8_t* qw,
         else
             TQ_SKINNY(8);
 #undef TQ_SKINNY
-        return check_launch("tq_gemm_w8a8");
+        return check_launch(what);
     }
-    if (k % kDmaBK == 0 && m < (int64_t(1) << 31) && n < (int64_t(1) << 31) && k < (int64_t(1) << 31)) {
-        const int64_t tm = (m + kDmaBM - 1) / kDmaBM, tn = (n + kDmaBN - 1) / kDmaBN;
-        if (tm * tn < (int64_t(1) << 31)) {
-            k_gemm_w8a8_dma<false><<<static_cast<unsigned>(tm * tn), 256, 0, as_hip(stream)>>>(
-                qa, sa, qw, sw, bias, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), acc, y,
-                static_cast<int>(tm), static_cast<int>(tn));
-            return check_launch("tq_gemm_w8a8");
-        }
+    if (!tile_fits(m, n, k)) return launch_gemm_w8a8_generic(qa, sa, qw, sw, bias, m, n, k, acc, y, st);
+    const TilePlan plan = tile_plan<GemmI8>(m, n, k, vec && k % kDmaBK == 0 ? kDmaStageI8 : 0, ws != nullptr);
+    if (plan.shape == kTileDma) {
+        const int tm = static_cast<int>((m + kDmaBM - 1) / kDmaBM), tn = static_cast<int>((n + kDmaBN - 1) / kDmaBN);
+        k_gemm_w8a8_dma<false><<<static_cast<unsigned>(tm * tn), 256, 0, st>>>(
+            qa, sa, qw, sw, bias, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), acc, y, tm, tn);
+        return check_launch(what);
     }
-    const int64_t tiles = ((m + kTileM - 1) / kTileM) * ((n + kTileN - 1) / kTileN);
-    TQ_REQUIRE(tiles < (int64_t(1) << 31), "tq_gemm_w8a8: problem too large");
-    k_gemm_w8a8<<<static_cast<unsigned>(tiles), kBlock, 0, as_hip(stream)>>>(qa, sa, qw, sw, bias, m, n, k, acc,
-                                                                             y);
-    return check_launch("tq_gemm_w8a8");
+    TQ_REQUIRE(ws_bytes >= plan.part_bytes && aligned(ws, 8), "%s: workspace of %lld bytes, %lld needed", what,
+               (long long)ws_bytes, (long long)plan.part_bytes);
+    return launch_tile<GemmI8>(plan, a8_args(qa, sa, qw, sw, bias, m, n, k, acc, y, ws), st, what);
 }
 
-extern "C" int tq_gemm_fp8(const uint8_t* qa, const float* sa, const uint8_t* qw, const float* sw,
-                           const float* bias, int64_t m, int64_t n, int64_t k, float* y, tq_stream_t stream) {
-    TQ_REQUIRE(m >= 0 && n >= 0 && k >= 0, "tq_gemm_fp8: negative shape");
+int gemm_fp8(const uint8_t* qa, const float* sa, const uint8_t* qw, const float* sw, const float* bias, int64_t m,
+             int64_t n, int64_t k, void* ws, int64_t ws_bytes, float* y, hipStream_t st, const char* what) {
+    TQ_REQUIRE(m >= 0 && n >= 0 && k >= 0, "%s: negative shape", what);
     if (m == 0 || n == 0) return TQ_OK;
-    TQ_REQUIRE(sa && sw && y && (k == 0 || (qa && qw)), "tq_gemm_fp8: null pointer");
+    TQ_REQUIRE(sa && sw && y && (k == 0 || (qa && qw)), "%s: null pointer", what);
     TQ_REQUIRE(aligned(sa, 4) && aligned(sw, 4) && aligned(y, 4) && (!bias || aligned(bias, 4)),
-               "tq_gemm_fp8: misaligned pointer");
-    // the MFMA kernel takes K in 128-byte stages, stores 4 consecutive n per lane
-    // (N % 16 == 0) and loads 16-byte vectors
-    const bool fast = k > 0 && k % kDmaBK == 0 && n % 16 == 0 && aligned(qa, 16) && aligned(qw, 16) &&
-                      aligned(sw, 16) && aligned(y, 16) && (!bias || aligned(bias, 16)) &&
-                      m < (int64_t(1) << 31) && n < (int64_t(1) << 31) && k < (int64_t(1) << 31);
-    if (fast && m <= 16 && k <= 8192) {  // decode batches: the skinny kernel, N / 16 blocks
+               "%s: misaligned pointer", what);
+    // the fp8 MFMAs take K in 128-byte stages, N in 16s and 16-byte vectors; they
+    // round inside their sums (1.5e-5 of y at any K), so operands outside that form
+    // stay on exact products with f32 and f64 sums (4.7e-8)
+    const bool native = i8_vectors(qa, qw, sw, bias, y, nullptr, n, k) && k % kDmaBK == 0;
+    if (native && n < (int64_t(1) << 31) && fp8_skinny(m, k)) {
         const int64_t cpw = ((k >> 7) + kSkinnyWaves - 1) / kSkinnyWaves;
         const unsigned grid = static_cast<unsigned>(n / 16);
         const auto* a = reinterpret_cast<const int8_t*>(qa);
         const auto* w = reinterpret_cast<const int8_t*>(qw);
         const int mi = static_cast<int>(m), ni = static_cast<int>(n);
         if (cpw <= 1)
-            k_gemm_fp8_skinny<1><<<grid, kSkinnyBlock, 0, as_hip(stream)>>>(a, sa, w, sw, bias, mi, ni, k, y);
+            k_gemm_fp8_skinny<1><<<grid, kSkinnyBlock, 0, st>>>(a, sa, w, sw, bias, mi, ni, k, y);
         else if (cpw <= 2)
-            k_gemm_fp8_skinny<2><<<grid, kSkinnyBlock, 0, as_hip(stream)>>>(a, sa, w, sw, bias, mi, ni, k, y);
+            k_gemm_fp8_skinny<2><<<grid, kSkinnyBlock, 0, st>>>(a, sa, w, sw, bias, mi, ni, k, y);
         else
-            k_gemm_fp8_skinny<4><<<grid, kSkinnyBlock, 0, as_hip(stream)>>>(a, sa, w, sw, bias, mi, ni, k, y);
-        return check_launch("tq_gemm_fp8");
+            k_gemm_fp8_skinny<4><<<grid, kSkinnyBlock, 0, st>>>(a, sa, w, sw, bias, mi, ni, k, y);
+        return check_launch(what);
     }
-    if (fast) {
-        const int64_t tm = (m + kDmaBM - 1) / kDmaBM, tn = (n + kDmaBN - 1) / kDmaBN;
-        if (tm * tn < (int64_t(1) << 31)) {
-            k_gemm_fp8_dma<<<static_cast<unsigned>(tm * tn), 256, 0, as_hip(stream)>>>(
-                reinterpret_cast<const int8_t*>(qa), sa, reinterpret_cast<const int8_t*>(qw), sw, bias,
-                static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), y, static_cast<int>(tm),
-                static_cast<int>(tn));
-            return check_launch("tq_gemm_fp8");
-        }
+    if (!tile_fits(m, n, k)) return launch_gemm_fp8_generic(qa, sa, qw, sw, bias, m, n, k, y, st);
+    const TileArgs args = a8_args(qa, sa, qw, sw, bias, m, n, k, nullptr, y, ws);
+    const TilePlan plan = native ? tile_plan<GemmF8>(m, n, k, kDmaStageF8, ws != nullptr)
+                                 : tile_plan<GemmF8b>(m, n, k, 0, ws != nullptr);
+    if (plan.shape == kTileDma) {
+        const int tm = static_cast<int>((m + kDmaBM - 1) / kDmaBM), tn = static_cast<int>((n + kDmaBN - 1) / kDmaBN);
+        k_gemm_fp8_dma<<<static_cast<unsigned>(tm * tn), 256, 0, st>>>(
+            reinterpret_cast<const int8_t*>(qa), sa, reinterpret_cast<const int8_t*>(qw), sw, bias,
+            static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), y, tm, tn);
+        return check_launch(what);
     }
-    return launch_gemm_fp8_generic(qa, sa, qw, sw, bias, m, n, k, y, as_hip(stream));
+    TQ_REQUIRE(ws_bytes >= plan.part_bytes && aligned(ws, 8), "%s: workspace of %lld bytes, %lld needed", what,
+               (long long)ws_bytes, (long long)plan.part_bytes);
+    return native ? launch_tile<GemmF8>(plan, args, st, what) : launch_tile<GemmF8b>(plan, args, st, what);
 }
+
+}  // namespace
+}  // namespace tq
+
+using namespace tq;
+
+extern "C" {
+
+int tq_gemm_w8a8(const int8_t* qa, const float* sa, const int8_t* qw, const float* sw, const float* bias, int64_t m,
+                 int64_t n, int64_t k, int32_t* acc, float* y, tq_stream_t stream) {
+    return gemm_w8a8(qa, sa, qw, sw, bias, m, n, k, acc, nullptr, 0, y, as_hip(stream), "tq_gemm_w8a8");
+}
+
+int64_t tq_gemm_w8a8_workspace_bytes(int64_t m, int64_t n, int64_t k) { return a8_part_bytes<GemmI8>(m, n, k); }
+
+int tq_gemm_w8a8_ws(const int8_t* qa, const float* sa, const int8_t* qw, const float* sw, const float* bias,
+                    int64_t m, int64_t n, int64_t k, int32_t* acc, void* workspace, int64_t workspace_bytes, float* y,
+                    tq_stream_t stream) {
+    return gemm_w8a8(qa, sa, qw, sw, bias, m, n, k, acc, workspace, workspace_bytes, y, as_hip(stream),
+                     "tq_gemm_w8a8_ws");
+}
+
+int tq_gemm_fp8(const uint8_t* qa, const float* sa, const uint8_t* qw, const float* sw, const float* bias, int64_t m,
+                int64_t n, int64_t k, float* y, tq_stream_t stream) {
+    return gemm_fp8(qa, sa, qw, sw, bias, m, n, k, nullptr, 0, y, as_hip(stream), "tq_gemm_fp8");
+}
+
+int64_t tq_gemm_fp8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    return std::max(a8_part_bytes<GemmF8>(m, n, k), a8_part_bytes<GemmF8b>(m, n, k));
+}
+
+int tq_gemm_fp8_ws(const uint8_t* qa, const float* sa, const uint8_t* qw, const float* sw, const float* bias,
+                   int64_t m, int64_t n, int64_t k, void* workspace, int64_t workspace_bytes, float* y,
+                   tq_stream_t stream) {
+    return gemm_fp8(qa, sa, qw, sw, bias, m, n, k, workspace, workspace_bytes, y, as_hip(stream), "tq_gemm_fp8_ws");
+}
+
+}  // extern "C"

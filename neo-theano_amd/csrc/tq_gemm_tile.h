@@ -1,0 +1,701 @@
+// tq_gemm_tile.h -- one register-staged MFMA GEMM for the 8-bit Linears the
+// LDS-DMA kernels do not serve, over operand traits:
+//
+//   y[m, n] = epilogue(sum_k A[m, k] * W[n, k])       A, W K-contiguous ("NT")
+//
+//  * GemmI8: A and W INT8 codes, int32 sums (exact).
+//  * GemmW8: A f32, W INT8 codes, on the i8 matrix cores: every row of A is a
+//    fixed-point number of 31 bits below its own largest magnitude, held as four
+//    balanced base-256 digits in four int8 rows (k_split_rows), so the sums of
+//    digits times codes are exact integers and the only errors are 2^-31 of the
+//    row's largest value per element and the final rounding: closer to the exact
+//    sum than f32 FMAs, at four i8 MFMAs per product (two bf16 ones' time).
+//  * GemmF8: A and W e4m3 codes on the fp8 matrix cores.
+//  * GemmF8b: the same codes widened to bf16 (exact products, f32 sums).
+//  * GemmF8W: A f32, W e4m3 codes, on the bf16 matrix cores.  Every f32
+//    activation is split exactly into three bf16 planes (8 + 8 + 8 significand
+//    bits, by truncation) and every code is exact in bf16, so each product is
+//    exact and only the f32 sums round.
+//
+// The bf16 forms add their running sums into a second set of accumulators every
+// kFlushStages stages (in f64 for GemmF8b), so that a sum's rounding grows with
+// the square root of a run's length and not of K: relative errors at K = 14336 are
+// 1.2e-7 (GemmF8W) and 4.7e-8 (GemmF8b), against 2.8e-7 and 7.2e-8 for a wave's f32
+// FMAs per output.
+//
+// Any M, N, K and any alignment of A, W and their rows (element-aligned
+// pointers): global loads are 8 to 32 bytes per lane at byte (codes) or 4-byte
+// (f32) alignment, which global memory instructions take on this target; the
+// last, partial K stage loads element by element; rows past M or N re-read the
+// last row and are not stored.
+#pragma once
+
+#include <algorithm>
+
+#include "tq_internal.h"
+
+namespace tq {
+namespace {
+
+typedef __bf16 tile_bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// Vectors at the alignment of their elements.
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
+typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
+
+// high halves of a and b as one dword (a low)
+__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
+    return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
+__device__ __forceinline__ uint32_t f32_bits(float v) { return __builtin_bit_cast(uint32_t, v); }
+
+// ---- sources: global elements -> registers (Raw) -> 16-byte LDS chunks ----
+// kElems elements make one chunk of each of kPlanes planes.
+
+// f32 -> three bf16 planes.  hi = x truncated to 8 significand bits, then the
+// (exact) residual twice more: hi + mid + lo == x.  An infinity is its own hi;
+// its residual must be 0, not inf - inf; a NaN stays NaN in mid and lo.
+struct SrcF32 {
+    typedef float elem_t;
+    static constexpr int kElems = 8, kPlanes = 3;
+    struct Raw {
+        f32x4 a, b;
+    };
+    __device__ static Raw load(const elem_t* p) {
+        return Raw{*reinterpret_cast<const f32x4_a4*>(p), *reinterpret_cast<const f32x4_a4*>(p + 4)};
+    }
+    __device__ static Raw load_part(const elem_t* p, int n) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = i < n ? p[i] : 0.0f;
+        return Raw{f32x4{v[0], v[1], v[2], v[3]}, f32x4{v[4], v[5], v[6], v[7]}};
+    }
+    __device__ static void planes(const Raw& r, u32x4 (&out)[kPlanes]) {
+        const float v[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+        uint32_t h[8], m[8], l[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            h[i] = f32_bits(v[i]) & 0xFFFF0000u;
+            const float hf = __uint_as_float(h[i]);
+            const float r1 = v[i] == hf ? 0.0f : v[i] - hf;
+            m[i] = f32_bits(r1) & 0xFFFF0000u;
+            l[i] = f32_bits(r1 - __uint_as_float(m[i]));  // at most 8 significant bits are left
+        }
+        out[0] = u32x4{pack_hi(h[0], h[1]), pack_hi(h[2], h[3]), pack_hi(h[4], h[5]), pack_hi(h[6], h[7])};
+        out[1] = u32x4{pack_hi(m[0], m[1]), pack_hi(m[2], m[3]), pack_hi(m[4], m[5]), pack_hi(m[6], m[7])};
+        out[2] = u32x4{pack_hi(l[0], l[1]), pack_hi(l[2], l[3]), pack_hi(l[4], l[5]), pack_hi(l[6], l[7])};
+    }
+};
+
+// 8 byte codes per chunk: the value of each as bf16 (exact).
+struct ValI8 {
+    typedef int8_t code_t;
+    __device__ static float value(uint32_t w, int b) { return static_cast<float>(static_cast<int8_t>(w >> (8 * b))); }
+};
+struct ValFp8 {
+    typedef uint8_t code_t;
+    template <int kB>
+    __device__ static float get(uint32_t w) { return __builtin_amdgcn_cvt_f32_fp8(static_cast<int>(w), kB); }
+    __device__ static float value(uint32_t w, int b) {
+        return b == 0 ? get<0>(w) : b == 1 ? get<1>(w) : b == 2 ? get<2>(w) : get<3>(w);
+    }
+};
+template <class Val>
+struct SrcBf16 {
+    typedef typename Val::code_t elem_t;
+    static constexpr int kElems = 8, kPlanes = 1;
+    struct Raw {
+        u32x2 v;
+    };
+    __device__ static Raw load(const elem_t* p) { return Raw{*reinterpret_cast<const u32x2_a1*>(p)}; }
+    __device__ static Raw load_part(const elem_t* p, int n) {
+        uint32_t w[2] = {0u, 0u};
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (i < n) w[i >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(p[i])) << (8 * (i & 3));
+        return Raw{u32x2{w[0], w[1]}};
+    }
+    __device__ static void planes(const Raw& r, u32x4 (&out)[1]) {
+        uint32_t f[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = f32_bits(Val::value(i < 4 ? r.v.x : r.v.y, i & 3));
+        out[0] = u32x4{pack_hi(f[0], f[1]), pack_hi(f[2], f[3]), pack_hi(f[4], f[5]), pack_hi(f[6], f[7])};
+    }
+};
+
+// 16 byte codes per chunk, as they are.
+template <class T>
+struct SrcBytes {
+    typedef T elem_t;
+    static constexpr int kElems = 16, kPlanes = 1;
+    struct Raw {
+        u32x4 v;
+    };
+    __device__ static Raw load(const elem_t* p) { return Raw{*reinterpret_cast<const u32x4_a1*>(p)}; }
+    __device__ static Raw load_part(const elem_t* p, int n) {
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (i < n) w[i >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(p[i])) << (8 * (i & 3));
+        return Raw{u32x4{w[0], w[1], w[2], w[3]}};
+    }
+    __device__ static void planes(const Raw& r, u32x4 (&out)[1]) { out[0] = r.v; }
+};
+
+// ---- operand traits ----
+// kFragChunks 16-byte chunks per lane and MFMA; an MFMA step covers twice that
+// many chunks of a row (one share per lane half).
+struct OpBf16 {
+    typedef f32x16 Acc;
+    static constexpr bool kFlush = true, kDigits = false;
+    static constexpr int kFragChunks = 1;
+    typedef u32x4 Frag;
+    __device__ static Frag frag(const u32x4 (&c)[1]) { return c[0]; }
+    __device__ static Acc mfma(Frag a, Frag b, Acc c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(tile_bf16x8, a),
+                                                       __builtin_bit_cast(tile_bf16x8, b), c, 0, 0, 0);
+    }
+};
+struct GemmF8W : OpBf16 {
+    typedef SrcF32 A;
+    typedef SrcBf16<ValFp8> W;
+    typedef float part_t;
+    static constexpr bool kRowScale = false;
+    static constexpr int kFlushStages = 8;
+};
+struct GemmF8b : OpBf16 {
+    typedef SrcBf16<ValFp8> A;
+    typedef SrcBf16<ValFp8> W;
+    typedef double part_t;
+    static constexpr bool kRowScale = true;
+    static constexpr int kFlushStages = 4;
+};
+struct GemmI8 {
+    typedef SrcBytes<int8_t> A;
+    typedef SrcBytes<int8_t> W;
+    typedef i32x16 Acc;
+    typedef int32_t part_t;
+    static constexpr bool kRowScale = true, kFlush = false, kDigits = false;
+    static constexpr int kFragChunks = 1;
+    typedef i32x4 Frag;
+    __device__ static Frag frag(const u32x4 (&c)[1]) { return __builtin_bit_cast(i32x4, c[0]); }
+    __device__ static Acc mfma(Frag a, Frag b, Acc c) {
+        return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+    }
+};
+// Rows 4 m .. 4 m + 3 of A are the digits of row m (lowest first).
+struct GemmW8 : GemmI8 {
+    typedef int64_t part_t;
+    static constexpr bool kRowScale = false, kDigits = true;
+};
+struct GemmF8 {
+    typedef SrcBytes<uint8_t> A;
+    typedef SrcBytes<uint8_t> W;
+    typedef f32x16 Acc;
+    typedef float part_t;
+    static constexpr bool kRowScale = true, kFlush = false, kDigits = false;
+    static constexpr int kFragChunks = 2;
+    typedef i32x8 Frag;
+    __device__ static Frag frag(const u32x4 (&c)[2]) {
+        return i32x8{static_cast<int>(c[0].x), static_cast<int>(c[0].y), static_cast<int>(c[0].z),
+                     static_cast<int>(c[0].w), static_cast<int>(c[1].x), static_cast<int>(c[1].y),
+                     static_cast<int>(c[1].z), static_cast<int>(c[1].w)};
+    }
+    __device__ static Acc mfma(Frag a, Frag b, Acc c) {
+        // cbsz = blgp = 0: both operands FP8 E4M3; scales 0 select the unscaled MFMA
+        return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+    }
+};
+
+// Fixed point of a row (kDigits): value = digits * 2^(e - 29) with 2^e <= the
+// row's largest magnitude < 2^(e + 1); a row holding an infinity or a NaN has no
+// such e and its outputs are summed directly in f32.
+constexpr int kNotFinite = INT32_MAX;
+
+struct TileArgs {
+    const void* a;      // A [m, lda] (kDigits: [4 m, lda] digit rows)
+    const void* w;      // W [n, k]
+    const float* sa;    // row scales [m] (kRowScale)
+    const int* ea;      // row exponents [m] (kDigits)
+    const float* x;     // the f32 activations [m, k] (kDigits, rows that are not finite)
+    const float* sw;    // column scales [n]
+    const float* bias;  // [n] or null
+    int m, n, k, lda;   // m counts outputs' rows
+    int tiles_m, tiles_n, split;
+    int32_t* acc;  // int32 sums [m, n] or null (GemmI8)
+    float* y;      // [m, n]
+    void* part;    // split > 1: partial sums [split][m][n]
+};
+
+__device__ __forceinline__ int64_t join_digits(int d0, int d1, int d2, int d3) {
+    return ((static_cast<int64_t>(d3) * 256 + d2) * 256 + d1) * 256 + d0;
+}
+
+// y[mm, nn] from its sum
+template <class T>
+__device__ __forceinline__ void tile_store(const TileArgs& p, typename T::part_t v, int mm, int nn, float sw, float b) {
+    const int64_t o = static_cast<int64_t>(mm) * p.n + nn;
+    if constexpr (T::kDigits) {
+        const int e = p.ea[mm];
+        if (e != kNotFinite) {
+            p.y[o] = static_cast<float>(fma(static_cast<double>(v), ldexp(static_cast<double>(sw), e - 29),
+                                            static_cast<double>(b)));
+        } else {
+            const float* x = p.x + static_cast<int64_t>(mm) * p.k;
+            const int8_t* w = static_cast<const int8_t*>(p.w) + static_cast<int64_t>(nn) * p.k;
+            float sum = 0.0f;
+            for (int k = 0; k < p.k; ++k) sum = fmaf(x[k], static_cast<float>(w[k]), sum);
+            p.y[o] = fmaf(sw, sum, b);
+        }
+    } else if constexpr (T::kRowScale) {
+        if constexpr (__is_same(typename T::part_t, int32_t))
+            if (p.acc) p.acc[o] = v;
+        p.y[o] = fmaf(static_cast<float>(v) * p.sa[mm], sw, b);
+    } else {
+        p.y[o] = fmaf(sw, v, b);
+    }
+}
+
+constexpr int kTileRow = 128;  // bytes of K per row and stage: 8 chunks
+__device__ __forceinline__ int tile_swz(int row) { return (row >> 1) & 7; }
+
+template <class T, int BM, int BN>
+constexpr int tile_stage_bytes() {
+    return (T::A::kPlanes * BM + T::W::kPlanes * BN) * kTileRow;
+}
+
+// Block: WM x WN waves (256 threads), each a (BM / WM) x (BN / WN) tile of 32 x
+// 32 MFMA tiles.  K runs in stages of 8 chunks (64 bf16 or 128 byte codes) through
+// two LDS buffers; while the MFMAs of stage s run, the registers holding stage
+// s + 1 are converted and written to the other buffer and refilled from global
+// memory with stage s + 2, a share per MFMA step, so that conversion and loads
+// hide under the matrix cores.  One barrier per stage.
+template <class T, int BM, int BN, int WM, int WN, int kOcc>
+__global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
+    using SA = typename T::A;
+    using SW = typename T::W;
+    static_assert(WM * WN == 4, "4 waves");
+    constexpr int TM = BM / WM / 32, TN = BN / WN / 32, PA = SA::kPlanes;
+    constexpr int kAItems = BM * 8 / 256, kWItems = BN * 8 / 256;
+    constexpr int kSteps = 4 / T::kFragChunks;
+    constexpr int kStage = tile_stage_bytes<T, BM, BN>();
+    constexpr int BK = 8 * SA::kElems;
+    static_assert(SA::kElems == SW::kElems && SW::kPlanes == 1, "operands advance together");
+    static_assert(kAItems >= 1 && kWItems >= 1 && TM >= 1 && TN >= 1, "tile too small");
+    __shared__ __attribute__((aligned(1024))) int8_t lds[2 * kStage];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave % WM, wn = wave / WM, l32 = lane & 31, lh = lane >> 5;
+    // consecutive blocks go to different XCDs: give each XCD a contiguous run of
+    // tiles (row tiles fastest) so that blocks sharing weight rows share an L2
+    const int total = p.tiles_m * p.tiles_n * p.split;
+    const int q8 = total >> 3, r8 = total & 7, xcd = blockIdx.x & 7;
+    const int L = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3);
+    const int tm = L % p.tiles_m, tn = (L / p.tiles_m) % p.tiles_n, ks = L / (p.tiles_m * p.tiles_n);
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int rows_a = T::kDigits ? 4 * p.m : p.m;
+    const int stages = (p.k + BK - 1) / BK;
+    const int s_begin = static_cast<int>(static_cast<int64_t>(ks) * stages / p.split);
+    const int s_end = static_cast<int>(static_cast<int64_t>(ks + 1) * stages / p.split);
+
+    // item i: row (tid + 256 i) / 8, chunk tid % 8
+    const int chunk = tid & 7;
+    const typename SA::elem_t* asrc[kAItems];
+    const typename SW::elem_t* wsrc[kWItems];
+    uint32_t adst[kAItems], wdst[kWItems];
+#pragma unroll
+    for (int i = 0; i < kAItems; ++i) {
+        const int r = (tid >> 3) + 32 * i;
+        asrc[i] = static_cast<const typename SA::elem_t*>(p.a) + static_cast<int64_t>(min(m0 + r, rows_a - 1)) * p.lda;
+        adst[i] = r * kTileRow + ((chunk ^ tile_swz(r)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < kWItems; ++i) {
+        const int r = (tid >> 3) + 32 * i;
+        wsrc[i] = static_cast<const typename SW::elem_t*>(p.w) + static_cast<int64_t>(min(n0 + r, p.n - 1)) * p.k;
+        wdst[i] = PA * BM * kTileRow + r * kTileRow + ((chunk ^ tile_swz(r)) << 4);
+    }
+    // two register sets: stage s of a split goes through set (s - s_begin) & 1
+    struct Regs {
+        typename SA::Raw a[kAItems];
+        typename SW::Raw w[kWItems];
+    } rg[2];
+    auto store_a = [&](const Regs& r, int i, int8_t* st) {
+        u32x4 c[PA];
+        SA::planes(r.a[i], c);
+#pragma unroll
+        for (int pl = 0; pl < PA; ++pl) *reinterpret_cast<u32x4*>(st + pl * BM * kTileRow + adst[i]) = c[pl];
+    };
+    auto store_w = [&](const Regs& r, int i, int8_t* st) {
+        u32x4 c[1];
+        SW::planes(r.w[i], c);
+        *reinterpret_cast<u32x4*>(st + wdst[i]) = c[0];
+    };
+    auto load_a = [&](Regs& r, int i, int s) { r.a[i] = SA::load(asrc[i] + s * BK + chunk * SA::kElems); };
+    auto load_w = [&](Regs& r, int i, int s) { r.w[i] = SW::load(wsrc[i] + s * BK + chunk * SW::kElems); };
+    // fragment of row r (of a plane at `base`) for step `step`
+    auto frag = [&](const int8_t* base, int r, int step) -> typename T::Frag {
+        u32x4 c[T::kFragChunks];
+#pragma unroll
+        for (int j = 0; j < T::kFragChunks; ++j) {
+            const int ch = (2 * step + lh) * T::kFragChunks + j;
+            c[j] = *reinterpret_cast<const u32x4*>(base + r * kTileRow + ((ch ^ tile_swz(r)) << 4));
+        }
+        return T::frag(c);
+    };
+
+    // a plane set's leading plane sums apart from the rest, whose terms are 2^-8 of
+    // its own: the leading sums' additions are then a third as many (and mostly
+    // exact), the others' rounding negligible
+    constexpr int kSets = PA > 1 ? 2 : 1;
+    typename T::Acc acc[kSets][TM][TN];
+#pragma unroll
+    for (int h = 0; h < kSets; ++h)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[h][i][j] = typename T::Acc{};
+
+    // the MFMAs of step `step` of the stage in `st`
+    auto step_mfma = [&](const int8_t* st, int step) {
+        typename T::Frag fa[TM][PA], fw[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int pl = 0; pl < PA; ++pl)
+                fa[i][pl] = frag(st + pl * BM * kTileRow, (wm * TM + i) * 32 + l32, step);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fw[j] = frag(st + PA * BM * kTileRow, (wn * TN + j) * 32 + l32, step);
+#pragma unroll
+        for (int pl = 0; pl < PA; ++pl)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    typename T::Acc& c = acc[pl > 0 ? kSets - 1 : 0][i][j];
+                    c = T::mfma(fa[i][pl], fw[j], c);
+                }
+    };
+    // one stage: its MFMAs, the next stage's registers `r` into the other buffer,
+    // and the stage after next's successor into those registers
+    auto stage = [&](const int8_t* st, int8_t* nst, Regs& r, int s_load) {
+#pragma unroll
+        for (int step = 0; step < kSteps; ++step) {
+            step_mfma(st, step);
+#pragma unroll
+            for (int i = 0; i < kAItems; ++i)
+                if (i * kSteps / kAItems == step) {
+                    store_a(r, i, nst);
+                    load_a(r, i, s_load);
+                }
+#pragma unroll
+            for (int i = 0; i < kWItems; ++i)
+                if (i * kSteps / kWItems == step) {
+                    store_w(r, i, nst);
+                    load_w(r, i, s_load);
+                }
+        }
+        // the LDS writes have landed and every wave is past its reads of `st`; global
+        // loads stay in flight across the barrier
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    // whole stages [s_begin, s_full): loads past the last re-read it (never used)
+    const int s_full = min(s_end, p.k / BK), s_last = s_full - 1;
+    typename T::part_t tot[T::kFlush ? TM : 1][T::kFlush ? TN : 1][16];
+    auto flush = [&]() {
+        if constexpr (T::kFlush) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if constexpr (kSets == 2) acc[0][i][j] += acc[1][i][j];
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) tot[i][j][e] += acc[0][i][j][e];
+#pragma unroll
+                    for (int h = 0; h < kSets; ++h) acc[h][i][j] = typename T::Acc{};
+                }
+        }
+    };
+    if constexpr (T::kFlush) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) tot[i][j][e] = 0;
+    }
+    if (s_begin < s_full) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < kAItems; ++i) load_a(rg[h], i, min(s_begin + h, s_last));
+#pragma unroll
+            for (int i = 0; i < kWItems; ++i) load_w(rg[h], i, min(s_begin + h, s_last));
+        }
+#pragma unroll
+        for (int i = 0; i < kAItems; ++i) {
+            store_a(rg[0], i, lds);
+            load_a(rg[0], i, min(s_begin + 2, s_last));
+        }
+#pragma unroll
+        for (int i = 0; i < kWItems; ++i) {
+            store_w(rg[0], i, lds);
+            load_w(rg[0], i, min(s_begin + 2, s_last));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        int s = s_begin;
+        for (; s + 1 < s_full; s += 2) {
+            stage(lds, lds + kStage, rg[1], min(s + 3, s_last));
+            stage(lds + kStage, lds, rg[0], min(s + 4, s_last));
+            if constexpr (T::kFlush)
+                if (((s + 2 - s_begin) & (T::kFlushStages - 1)) == 0) flush();
+        }
+        if (s < s_full) stage(lds, lds + kStage, rg[1], s_last);
+    }
+    if (s_full < s_end) {  // the partial last stage, element by element (zeros past K)
+        const int k0 = s_full * BK + chunk * SA::kElems;
+#pragma unroll
+        for (int i = 0; i < kAItems; ++i) {
+            rg[0].a[i] = SA::load_part(asrc[i] + k0, p.k - k0);
+            store_a(rg[0], i, lds);
+        }
+#pragma unroll
+        for (int i = 0; i < kWItems; ++i) {
+            rg[0].w[i] = SW::load_part(wsrc[i] + k0, p.k - k0);
+            store_w(rg[0], i, lds);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int step = 0; step < kSteps; ++step) step_mfma(lds, step);
+    }
+    flush();
+
+    auto sum = [&](int i, int j, int e) {
+        if constexpr (T::kFlush)
+            return tot[i][j][e];
+        else
+            return acc[0][i][j][e];
+    };
+    // lane holds D[m = 8 (e/4) + 4 lh + e % 4][n = l32] of each 32 x 32 tile: a
+    // store covers 32 consecutive n of two rows; with digit rows, e % 4 is the
+    // digit and a lane holds whole sums of 4 rows
+    constexpr int kPer = T::kDigits ? 4 : 1;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int nn = n0 + (wn * TN + j) * 32 + l32;
+        const bool nval = nn < p.n;
+        const float sw = p.split == 1 && nval ? p.sw[nn] : 0.0f;
+        const float bv = p.split == 1 && nval && p.bias ? p.bias[nn] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; e += kPer) {
+                const int mm = (m0 + (wm * TM + i) * 32 + 8 * (e >> 2) + 4 * lh + (e & 3)) / kPer;
+                if (!nval || mm >= p.m) continue;
+                typename T::part_t v;
+                if constexpr (T::kDigits)
+                    v = join_digits(sum(i, j, e), sum(i, j, e + 1), sum(i, j, e + 2), sum(i, j, e + 3));
+                else
+                    v = sum(i, j, e);
+                if (p.split == 1)
+                    tile_store<T>(p, v, mm, nn, sw, bv);
+                else
+                    static_cast<typename T::part_t*>(
+                        p.part)[(static_cast<int64_t>(ks) * p.m + mm) * p.n + nn] = v;
+            }
+    }
+}
+
+// Adds the partial sums of a split launch in a fixed order and finishes the outputs.
+template <class T>
+__global__ __launch_bounds__(256) void k_gemm_tile_finish(TileArgs p) {
+    const int64_t mn = static_cast<int64_t>(p.m) * p.n;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= mn) return;
+    const typename T::part_t* part = static_cast<const typename T::part_t*>(p.part) + i;
+    typename T::part_t v = part[0];
+    for (int s = 1; s < p.split; ++s) v += part[s * mn];
+    const int mm = static_cast<int>(i / p.n), nn = static_cast<int>(i - static_cast<int64_t>(mm) * p.n);
+    tile_store<T>(p, v, mm, nn, p.sw[nn], p.bias ? p.bias[nn] : 0.0f);
+}
+
+// x [rows, k] f32 -> digit rows [4 rows, lda] (zeros past k) and the row exponents:
+// one block per row; v = x * 2^(29 - e) rounded to an integer (|v| <= 2^30), whose
+// balanced base-256 digits are the bytes of (v + 0x808080) ^ 0x808080 (the top one
+// signed).  The row stays in registers between its maximum and its digits (up to
+// kItems x 1024 values; longer rows are read again).
+template <int kItems>
+__global__ __launch_bounds__(256) void k_split_rows(const float* __restrict__ x, int k, int lda,
+                                                    int8_t* __restrict__ d, int* __restrict__ ea) {
+    __shared__ uint32_t red[4];
+    const int row = blockIdx.x, tid = threadIdx.x;
+    const float* src = x + static_cast<int64_t>(row) * k;
+    auto load = [&](int j) -> f32x4 {  // values 4 j .. 4 j + 3, zeros past k
+        if (4 * j + 4 <= k) return *reinterpret_cast<const f32x4_a4*>(src + 4 * j);
+        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (4 * j < k) v.x = src[4 * j];
+        if (4 * j + 1 < k) v.y = src[4 * j + 1];
+        if (4 * j + 2 < k) v.z = src[4 * j + 2];
+        return v;
+    };
+    // the largest |x| as bits: above every finite value for an infinity or a NaN
+    auto fold = [](uint32_t mx, f32x4 v) {
+        const uint32_t a = max(f32_bits(v.x) & 0x7FFFFFFFu, f32_bits(v.y) & 0x7FFFFFFFu);
+        const uint32_t b = max(f32_bits(v.z) & 0x7FFFFFFFu, f32_bits(v.w) & 0x7FFFFFFFu);
+        return max(mx, max(a, b));
+    };
+    const int items = lda / 4;
+    f32x4 v[kItems];
+    uint32_t mx = 0;
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) v[i] = load(tid + 256 * i);
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) mx = fold(mx, v[i]);
+    for (int j = tid + 256 * kItems; j < items; j += 256) mx = fold(mx, load(j));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = max(mx, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mx), o, kWave)));
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    __syncthreads();
+    mx = max(max(red[0], red[1]), max(red[2], red[3]));
+    const bool finite = mx < 0x7F800000u;
+    const int e = max(static_cast<int>(mx >> 23), 1) - 127;
+    if (tid == 0) ea[row] = finite ? e : kNotFinite;
+    int8_t* dst = d + static_cast<int64_t>(row) * 4 * lda;
+    auto digits = [&](float f) -> uint32_t {
+        const int i = static_cast<int>(rintf(ldexpf(f, 29 - e)));
+        return (static_cast<uint32_t>(i) + 0x00808080u) ^ 0x00808080u;
+    };
+    auto store = [&](int j, f32x4 f) {
+        uint32_t a = 0, b = 0, c = 0, g = 0;
+        if (finite) {
+            a = digits(f.x);
+            b = digits(f.y);
+            c = digits(f.z);
+            g = digits(f.w);
+        }
+        // 4 x 4 byte transpose: word r = digit r of the four values
+        const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u), ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u);
+        const uint32_t cg0 = __builtin_amdgcn_perm(g, c, 0x05010400u), cg1 = __builtin_amdgcn_perm(g, c, 0x07030602u);
+        uint32_t* o = reinterpret_cast<uint32_t*>(dst) + j;
+        const int step = lda / 4;
+        o[0] = __builtin_amdgcn_perm(cg0, ab0, 0x05040100u);
+        o[step] = __builtin_amdgcn_perm(cg0, ab0, 0x07060302u);
+        o[2 * step] = __builtin_amdgcn_perm(cg1, ab1, 0x05040100u);
+        o[3 * step] = __builtin_amdgcn_perm(cg1, ab1, 0x07060302u);
+    };
+#pragma unroll
+    for (int i = 0; i < kItems; ++i)
+        if (tid + 256 * i < items) store(tid + 256 * i, v[i]);
+    for (int j = tid + 256 * kItems; j < items; j += 256) store(j, load(j));
+}
+
+// ------------------------------------------------------------------ host side
+// Tile sizes and the time of one stage of one block in ns: with at most one block
+// on a CU (t1) and per block when several share it (t2), measured on M = 16 to
+// 2048 at N = K = 4096, N = 14336 and K = 14336.
+struct TileShape {
+    int bm, bn, t1, t2;
+};
+constexpr int kTileShapes = 4;
+enum { kTile128x128, kTile64x64, kTile32x128, kTile64x128 };
+template <class T>
+struct TileCosts;
+template <>
+struct TileCosts<GemmI8> {
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 700, 800}, {64, 64, 270, 310}, {32, 128, 285, 325}, {64, 128, 500, 510}};
+};
+template <>
+struct TileCosts<GemmW8> : TileCosts<GemmI8> {};
+template <>
+struct TileCosts<GemmF8> {
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 700, 760}, {64, 64, 270, 300}, {32, 128, 270, 295}, {64, 128, 430, 450}};
+};
+template <>
+struct TileCosts<GemmF8b> {
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 850, 1060}, {64, 64, 420, 270}, {32, 128, 540, 300}, {64, 128, 600, 500}};
+};
+template <>
+struct TileCosts<GemmF8W> {
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 2100, 2400}, {64, 64, 840, 690}, {32, 128, 780, 600}, {64, 128, 1150, 960}};
+};
+
+constexpr int kTileDma = -1;  // the LDS-DMA kernels' 128 x 256 tiles
+
+struct TilePlan {
+    int shape, split, tiles_m, tiles_n;
+    int64_t part_bytes;
+};
+
+// The shape and K split with the smallest estimate: rounds of blocks over the CUs
+// times the stages of a block times the stage's time; a split adds the finishing
+// launch (3 us) and its partial sums' traffic (4 TB/s) and is worth it where the
+// tiles alone leave CUs idle.  `dma_stage` > 0: the LDS-DMA kernel serves these
+// operands at that time per 128-byte stage.
+template <class T>
+TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int dma_stage, bool may_split) {
+    const int64_t cus = device_cu_count(), rows = T::kDigits ? 4 * m : m;
+    const int64_t stages = (k + 8 * T::A::kElems - 1) / (8 * T::A::kElems);
+    TilePlan best{kTile64x64, 1, 0, 0, 0};
+    int64_t best_ns = INT64_MAX;
+    if (dma_stage > 0) {
+        const int64_t blocks = ((rows + 127) / 128) * ((n + 255) / 256);
+        best.shape = kTileDma;
+        best_ns = (blocks + cus - 1) / cus * (k / 128) * dma_stage + 4000;
+    }
+    for (int c = 0; c < kTileShapes; ++c) {
+        const TileShape& t = TileCosts<T>::shape[c];
+        const int64_t tm = (rows + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
+        for (int split : {1, 2, 3, 4, 6, 8, 12, 16}) {
+            if (split > 1 && (!may_split || stages < 4 * split || tm * tn * split > 4 * cus)) break;
+            const int64_t rounds = (tm * tn * split + cus - 1) / cus, per = (stages + split - 1) / split;
+            int64_t ns = rounds == 1 ? t.t1 * per : std::max<int64_t>(t.t1, rounds * t.t2) * per;
+            ns += 3000;
+            const int64_t part = split * m * n * static_cast<int64_t>(sizeof(typename T::part_t));
+            if (split > 1) ns += 3000 + 2 * part / 4000;
+            if (ns < best_ns) {
+                best_ns = ns;
+                best = TilePlan{c, split, 0, 0, split > 1 ? part : 0};
+            }
+        }
+    }
+    if (best.shape != kTileDma) {
+        const TileShape& t = TileCosts<T>::shape[best.shape];
+        best.tiles_m = static_cast<int>((rows + t.bm - 1) / t.bm);
+        best.tiles_n = static_cast<int>((n + t.bn - 1) / t.bn);
+    }
+    return best;
+}
+
+// m, n and k (and 4 m with digit rows) fit the kernels' 32-bit indexes
+inline bool tile_fits(int64_t rows, int64_t n, int64_t k) {
+    return rows < (int64_t(1) << 31) - 128 && n < (int64_t(1) << 31) - 128 && k < (int64_t(1) << 31) - 1024 &&
+           ((rows + 31) / 32) * ((n + 63) / 64) < (int64_t(1) << 31);
+}
+
+// Launches the plan's tiles (not kTileDma) and, for a split, the finishing kernel.
+template <class T>
+int launch_tile(const TilePlan& plan, TileArgs p, hipStream_t st, const char* what) {
+    p.tiles_m = plan.tiles_m;
+    p.tiles_n = plan.tiles_n;
+    p.split = plan.split;
+    const unsigned grid = static_cast<unsigned>(static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.split);
+    switch (plan.shape) {
+    case kTile128x128: k_gemm_tile<T, 128, 128, 2, 2, 1><<<grid, 256, 0, st>>>(p); break;
+    case kTile64x64: k_gemm_tile<T, 64, 64, 2, 2, 2><<<grid, 256, 0, st>>>(p); break;
+    case kTile32x128: k_gemm_tile<T, 32, 128, 1, 4, 2><<<grid, 256, 0, st>>>(p); break;
+    default: k_gemm_tile<T, 64, 128, 2, 2, 2><<<grid, 256, 0, st>>>(p); break;
+    }
+    if (p.split > 1) {
+        const int rc = check_launch(what);
+        if (rc != TQ_OK) return rc;
+        const int64_t blocks = (static_cast<int64_t>(p.m) * p.n + 255) / 256;
+        k_gemm_tile_finish<T><<<static_cast<unsigned>(blocks), 256, 0, st>>>(p);
+    }
+    return check_launch(what);
+}
+
+}  // namespace
+}  // namespace tq

@@ -562,7 +562,10 @@ Result<QuantizedLinear> QuantizedLinear::from_tensors(const Tensor& weight, cons
 }
 
 size_t QuantizedLinear::workspace_bytes(int64_t m) const {
+    const int64_t n = static_cast<int64_t>(out_), k = static_cast<int64_t>(in_);
     if (mode_ == Mode::FP8 && m <= kFusedA8MaxM) return static_cast<size_t>(m) * in_ * sizeof(float);
+    if (mode_ == Mode::FP8) return static_cast<size_t>(tq_gemm_fp8_workspace_bytes(m, n, k));
+    if (mode_ == Mode::W8A8) return static_cast<size_t>(tq_gemm_w8a8_workspace_bytes(m, n, k));
     if (mode_ != Mode::W4 || m <= 16 || (w4_.tile_rows > 0 && m <= kTiledPassesMaxM)) return 0;
     return static_cast<size_t>(tq_gemm_w4g128_bf16_workspace_bytes(m, static_cast<int64_t>(in_)));
 }
@@ -572,6 +575,8 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
     const auto ts = reinterpret_cast<tq_stream_t>(stream);
     const float* b = bias_ ? bias_->data() : nullptr;
     const int64_t n = static_cast<int64_t>(out_), k = static_cast<int64_t>(in_);
+    // the workspace forms split K over blocks; a smaller workspace is not used
+    const bool has_ws = workspace && workspace_bytes >= this->workspace_bytes(m);
     int st = TQ_OK;
     switch (mode_) {
         case Mode::W4: {
@@ -612,8 +617,10 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
                 return TheanoError::invalid_argument("QuantizedLinear::forward_device: w8a8 needs activation scratch");
             st = tq_quantize_i8_rowwise(static_cast<const float*>(x), m, k, act_codes, act_scales, ts);
             if (st == TQ_OK)
-                st = tq_gemm_w8a8(act_codes, act_scales, w8_.codes.data(), w8_.scales.data(), b, m, n, k, nullptr, y,
-                                  ts);
+                st = has_ws ? tq_gemm_w8a8_ws(act_codes, act_scales, w8_.codes.data(), w8_.scales.data(), b, m, n, k,
+                                                 nullptr, workspace, static_cast<int64_t>(workspace_bytes), y, ts)
+                               : tq_gemm_w8a8(act_codes, act_scales, w8_.codes.data(), w8_.scales.data(), b, m, n, k,
+                                              nullptr, y, ts);
             break;
         }
         case Mode::FP8: {  // as W8A8 (FP8 at 4096 x 4096: 10.0 against 12.9 us at m = 3)
@@ -628,7 +635,10 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
             if (m > kFusedA8MaxM) {
                 st = tq_quantize_fp8_rowwise(static_cast<const float*>(x), m, k, qa, act_scales, ts);
                 if (st == TQ_OK)
-                    st = tq_gemm_fp8(qa, act_scales, fp8_.codes.data(), fp8_.scales.data(), b, m, n, k, y, ts);
+                    st = has_ws ? tq_gemm_fp8_ws(qa, act_scales, fp8_.codes.data(), fp8_.scales.data(), b, m, n, k,
+                                                    workspace, static_cast<int64_t>(workspace_bytes), y, ts)
+                                   : tq_gemm_fp8(qa, act_scales, fp8_.codes.data(), fp8_.scales.data(), b, m, n, k, y,
+                                                 ts);
                 break;
             }
             // decode: the GEMV over x_hat = e4m3(qa) * sa, the GEMM's activation values

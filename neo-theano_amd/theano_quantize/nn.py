@@ -140,6 +140,11 @@ class QuantizedLinear(Module):
     def _act_dtype(self):
         return torch.bfloat16 if self.mode == "w4" else torch.float32
 
+    def _workspace(self, entry, m, device):
+        """(device scratch or None, its bytes) for m tokens, as `entry` sizes it."""
+        nb = int(getattr(_abi.lib(), entry)(m, self.out_features, self.in_features))
+        return (torch.empty(nb, dtype=torch.uint8, device=device) if nb else None), nb
+
     def forward(self, x):
         x = on_device(x, self._act_dtype(), "QuantizedLinear.forward")
         squeeze = x.dim() == 1
@@ -181,8 +186,9 @@ class QuantizedLinear(Module):
             qa = torch.empty((m, k), dtype=torch.uint8, device=x.device)
             sa = torch.empty(m, dtype=torch.float32, device=x.device)
             _abi.call("tq_quantize_fp8_rowwise", ptr(x), m, k, ptr(qa), ptr(sa), stream())
-            _abi.call("tq_gemm_fp8", ptr(qa), ptr(sa), ptr(self.qweight), ptr(self.scales),
-                      ptr(self.bias), m, n, k, ptr(y), stream())
+            ws, nb = self._workspace("tq_gemm_fp8_workspace_bytes", m, x.device)
+            _abi.call("tq_gemm_fp8_ws", ptr(qa), ptr(sa), ptr(self.qweight), ptr(self.scales),
+                      ptr(self.bias), m, n, k, ptr(ws), nb, ptr(y), stream())
         elif self.mode in ("fp8", "fp8_weight"):
             if self.mode == "fp8":  # x -> e4m3(qa) * sa, the GEMM's activation values
                 qa = torch.empty((m, k), dtype=torch.uint8, device=x.device)
@@ -198,8 +204,9 @@ class QuantizedLinear(Module):
             qa = torch.empty((m, k), dtype=torch.int8, device=x.device)
             sa = torch.empty(m, dtype=torch.float32, device=x.device)
             _abi.call("tq_quantize_i8_rowwise", ptr(x), m, k, ptr(qa), ptr(sa), stream())
-            _abi.call("tq_gemm_w8a8", ptr(qa), ptr(sa), ptr(self.qweight), ptr(self.scales),
-                      ptr(self.bias), m, n, k, None, ptr(y), stream())
+            ws, nb = self._workspace("tq_gemm_w8a8_workspace_bytes", m, x.device)
+            _abi.call("tq_gemm_w8a8_ws", ptr(qa), ptr(sa), ptr(self.qweight), ptr(self.scales),
+                      ptr(self.bias), m, n, k, None, ptr(ws), nb, ptr(y), stream())
         return y.squeeze(0) if squeeze else y
 
 

@@ -1,0 +1,119 @@
+"""The register-staged tile GEMM behind the 8-bit Linears (tq_gemm_tile.h): odd and
+tile-edge sizes, codes at odd addresses, K split over blocks, against the same
+product in float64 (exact for INT8 codes: every partial sum is an integer below
+2^53)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (m, n, k): below, at and past the 32/64/128 tile edges; K below one 64- or 128-byte
+# stage, at and past stage edges, odd; few tiles of long K (split over blocks)
+SHAPES = [(1, 1, 1), (3, 5, 17), (17, 64, 63), (31, 33, 64), (33, 65, 129), (64, 128, 255), (65, 129, 1000),
+          (77, 1003, 1000), (128, 131, 128), (200, 257, 384), (40, 70, 8193), (16, 100, 14336), (129, 48, 4099)]
+
+
+def _codes(torch, shape, seed, fp8):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    if fp8:
+        x = (torch.randn(shape, generator=g, device="cuda") * 60).clamp(-448, 448)
+        return x.to(torch.float8_e4m3fn)
+    return torch.randint(-128, 128, shape, generator=g, device="cuda", dtype=torch.int8)
+
+
+def _at_offset(torch, t, off):
+    """`t`'s bytes at an address `off` past a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 64, dtype=torch.uint8, device="cuda")
+    v = buf[off:off + t.numel()]
+    v.copy_(t.view(torch.uint8).reshape(-1))
+    return buf, v
+
+
+def _run(torch, fp8, qa, qw, m, n, k, bias, off, with_ws):
+    from theano_quantize import _abi
+    from theano_quantize._tensor import ptr, stream
+
+    g = torch.Generator(device="cuda").manual_seed(m * 31 + n)
+    sa = torch.rand(m, generator=g, device="cuda") + 0.5
+    sw = torch.rand(n, generator=g, device="cuda") + 0.5
+    b = torch.randn(n, generator=g, device="cuda") if bias else None
+    ka, va = _at_offset(torch, qa, off)
+    kw, vw = _at_offset(torch, qw, off)
+    y = torch.full((m, n), float("nan"), device="cuda")
+    acc = torch.full((m, n), -7, dtype=torch.int32, device="cuda")
+    name = "tq_gemm_fp8" if fp8 else "tq_gemm_w8a8"
+    nb = int(getattr(_abi.lib(), name + "_workspace_bytes")(m, n, k))
+    ws = torch.empty(max(nb, 8), dtype=torch.uint8, device="cuda").fill_(0xA5)
+    args = [ptr(va), ptr(sa), ptr(vw), ptr(sw), ptr(b), m, n, k] + ([] if fp8 else [ptr(acc)])
+    if with_ws:
+        _abi.call(name + "_ws", *args, ptr(ws), nb, ptr(y), stream())
+    else:
+        _abi.call(name, *args, ptr(y), stream())
+    torch.cuda.synchronize()
+    prod = qa.double() @ qw.double().t().contiguous()
+    ref = prod * sa.double()[:, None] * sw.double()
+    if b is not None:
+        ref = ref + b.double()
+    return y.double(), acc, prod, ref
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("with_ws", [False, True])
+def test_w8a8_any_shape_exact(tq, m, n, k, with_ws):
+    import torch
+
+    for off in (0, 3):
+        y, acc, prod, ref = _run(torch, False, _codes(torch, (m, k), 1, False), _codes(torch, (n, k), 2, False), m, n, k,
+                                 off == 0, off, with_ws)
+        assert torch.equal(acc.double(), prod)
+        # f32 of the sum, the product with sa and the fma: three roundings of 2^-24 each
+        bound = 4 * 2.0 ** -24 * (ref.abs() + 1.0)
+        assert bool(((y - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("with_ws", [False, True])
+def test_fp8_any_shape(tq, m, n, k, with_ws):
+    import torch
+
+    qa, qw = _codes(torch, (m, k), 3, True), _codes(torch, (n, k), 4, True)
+    y, _, _, ref = _run(torch, True, qa, qw, m, n, k, True, 5, with_ws)
+    # exact bf16 products; every f32 addition of a run of 256 rounds by at most 2^-23 (twice
+    # half an ulp, for an adder that truncates) of the largest partial sum, bounded by the
+    # sum of magnitudes; measured errors are a hundred times smaller
+    mag = (qa.double().abs() @ qw.double().abs().t().contiguous()) * 1.5 * 1.5
+    bound = 2.0 ** -23 * min(k, 256) ** 0.5 * mag + 4 * 2.0 ** -24 * (ref.abs() + 4.0)
+    assert bool(((y - ref).abs() <= bound).all())
+    rel = ((y - ref).norm() / ref.norm()).item()
+    assert rel < 1e-6, rel  # the fp8 matrix instructions' own sums would be 1.5e-5 off
+
+
+def test_fp8_nan_code_stays_in_its_row_and_column(tq):
+    import torch
+
+    m, n, k = 35, 67, 200
+    qa, qw = _codes(torch, (m, k), 5, True), _codes(torch, (n, k), 6, True)
+    qa.view(torch.uint8)[4, k - 1] = 0x7F
+    qw.view(torch.uint8)[9, 0] = 0xFF
+    y, _, _, _ = _run(torch, True, qa, qw, m, n, k, False, 1, False)
+    nan = torch.zeros(m, n, dtype=torch.bool, device="cuda")
+    nan[4] = True
+    nan[:, 9] = True
+    assert torch.equal(y.isnan(), nan)
+
+
+def test_workspace_too_small_is_refused(tq):
+    import torch
+
+    from theano_quantize import _abi
+    from theano_quantize._tensor import ptr, stream
+
+    m, n, k = 64, 100, 14336
+    nb = int(_abi.lib().tq_gemm_w8a8_workspace_bytes(m, n, k))
+    assert nb > 0  # two 64 x 64 tiles: K is split
+    t = torch.zeros(m * k, dtype=torch.int8, device="cuda")
+    f = torch.zeros(m * n, device="cuda")
+    with pytest.raises(tq.InvalidArgument):
+        _abi.call("tq_gemm_w8a8_ws", ptr(t), ptr(f), ptr(torch.zeros(n * k, dtype=torch.int8, device="cuda")), ptr(f),
+                  None, m, n, k, None, ptr(f), nb - 1, ptr(f), stream())
+    assert np.isfinite(f.cpu().numpy()).all()
