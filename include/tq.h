@@ -214,6 +214,22 @@ int tq_gemv_w8(const float* x, int64_t m, const int8_t* q, const float* s,
 int tq_gemv_fp8(const float* x, int64_t m, const uint8_t* q, const float* s,
                 const float* bias, int64_t n, int64_t k, float* y, tq_stream_t stream);
 
+/* The two weight-only Linears above at any M: the GEMV for M <= 8, the matrix cores
+ * beyond.  INT8: each row of x becomes a 31-bit fixed-point number in four int8 digit
+ * rows and the sums are exact integers (closer to the exact y than f32 sums; a row
+ * holding an infinity or a NaN is summed in f32).  FP8: x split exactly into three
+ * bf16 planes, f32 sums.  Any N, K; f32 pointers 4-byte aligned.  `workspace`: device
+ * memory of at least the ..._workspace_bytes(M, N, K) bytes (0 for M <= 8), 256-byte
+ * aligned, contents need not be initialised. */
+int64_t tq_gemm_w8_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tq_gemm_w8(const float* x, int64_t m, const int8_t* q, const float* s, const float* bias,
+               int64_t n, int64_t k, void* workspace, int64_t workspace_bytes, float* y,
+               tq_stream_t stream);
+int64_t tq_gemm_fp8_weight_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tq_gemm_fp8_weight(const float* x, int64_t m, const uint8_t* q, const float* s, const float* bias,
+                       int64_t n, int64_t k, void* workspace, int64_t workspace_bytes, float* y,
+                       tq_stream_t stream);
+
 /* Decode-shaped W8A8 with the activation quantization fused in: x f32 [M, K],
  * M <= 16, is quantized per row inside the kernel exactly as
  * tq_quantize_i8_rowwise does, then y = fma(f32(sum_p qa*qw) * sa, sw, bias)

@@ -32,7 +32,7 @@
 
 #include <algorithm>
 
-#include "tq_internal.h"
+#include "tq_digits.h"
 
 namespace tq {
 namespace {
@@ -41,7 +41,6 @@ typedef __bf16 tile_bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // Vectors at the alignment of their elements.
-typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
 typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
 typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
 
@@ -49,14 +48,14 @@ typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
 __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
     return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
-__device__ __forceinline__ uint32_t f32_bits(float v) { return __builtin_bit_cast(uint32_t, v); }
 
 // ---- sources: global elements -> registers (Raw) -> 16-byte LDS chunks ----
 // kElems elements make one chunk of each of kPlanes planes.
 
 // f32 -> three bf16 planes.  hi = x truncated to 8 significand bits, then the
 // (exact) residual twice more: hi + mid + lo == x.  An infinity is its own hi;
-// its residual must be 0, not inf - inf; a NaN stays NaN in mid and lo.
+// its residual must be 0, not inf - inf; a NaN stays NaN in mid and lo.  (Bits
+// below 2^-133, bf16's last place, are dropped: only values under 2^-109 have any.)
 struct SrcF32 {
     typedef float elem_t;
     static constexpr int kElems = 8, kPlanes = 3;
@@ -209,11 +208,6 @@ struct GemmF8 {
     }
 };
 
-// Fixed point of a row (kDigits): value = digits * 2^(e - 29) with 2^e <= the
-// row's largest magnitude < 2^(e + 1); a row holding an infinity or a NaN has no
-// such e and its outputs are summed directly in f32.
-constexpr int kNotFinite = INT32_MAX;
-
 struct TileArgs {
     const void* a;      // A [m, lda] (kDigits: [4 m, lda] digit rows)
     const void* w;      // W [n, k]
@@ -229,26 +223,13 @@ struct TileArgs {
     void* part;    // split > 1: partial sums [split][m][n]
 };
 
-__device__ __forceinline__ int64_t join_digits(int d0, int d1, int d2, int d3) {
-    return ((static_cast<int64_t>(d3) * 256 + d2) * 256 + d1) * 256 + d0;
-}
-
 // y[mm, nn] from its sum
 template <class T>
 __device__ __forceinline__ void tile_store(const TileArgs& p, typename T::part_t v, int mm, int nn, float sw, float b) {
     const int64_t o = static_cast<int64_t>(mm) * p.n + nn;
     if constexpr (T::kDigits) {
-        const int e = p.ea[mm];
-        if (e != kNotFinite) {
-            p.y[o] = static_cast<float>(fma(static_cast<double>(v), ldexp(static_cast<double>(sw), e - 29),
-                                            static_cast<double>(b)));
-        } else {
-            const float* x = p.x + static_cast<int64_t>(mm) * p.k;
-            const int8_t* w = static_cast<const int8_t*>(p.w) + static_cast<int64_t>(nn) * p.k;
-            float sum = 0.0f;
-            for (int k = 0; k < p.k; ++k) sum = fmaf(x[k], static_cast<float>(w[k]), sum);
-            p.y[o] = fmaf(sw, sum, b);
-        }
+        p.y[o] = digit_out(v, p.ea[mm], sw, b, p.x + static_cast<int64_t>(mm) * p.k,
+                           static_cast<const int8_t*>(p.w) + static_cast<int64_t>(nn) * p.k, p.k);
     } else if constexpr (T::kRowScale) {
         if constexpr (__is_same(typename T::part_t, int32_t))
             if (p.acc) p.acc[o] = v;
@@ -520,76 +501,6 @@ __global__ __launch_bounds__(256) void k_gemm_tile_finish(TileArgs p) {
     for (int s = 1; s < p.split; ++s) v += part[s * mn];
     const int mm = static_cast<int>(i / p.n), nn = static_cast<int>(i - static_cast<int64_t>(mm) * p.n);
     tile_store<T>(p, v, mm, nn, p.sw[nn], p.bias ? p.bias[nn] : 0.0f);
-}
-
-// x [rows, k] f32 -> digit rows [4 rows, lda] (zeros past k) and the row exponents:
-// one block per row; v = x * 2^(29 - e) rounded to an integer (|v| <= 2^30), whose
-// balanced base-256 digits are the bytes of (v + 0x808080) ^ 0x808080 (the top one
-// signed).  The row stays in registers between its maximum and its digits (up to
-// kItems x 1024 values; longer rows are read again).
-template <int kItems>
-__global__ __launch_bounds__(256) void k_split_rows(const float* __restrict__ x, int k, int lda,
-                                                    int8_t* __restrict__ d, int* __restrict__ ea) {
-    __shared__ uint32_t red[4];
-    const int row = blockIdx.x, tid = threadIdx.x;
-    const float* src = x + static_cast<int64_t>(row) * k;
-    auto load = [&](int j) -> f32x4 {  // values 4 j .. 4 j + 3, zeros past k
-        if (4 * j + 4 <= k) return *reinterpret_cast<const f32x4_a4*>(src + 4 * j);
-        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (4 * j < k) v.x = src[4 * j];
-        if (4 * j + 1 < k) v.y = src[4 * j + 1];
-        if (4 * j + 2 < k) v.z = src[4 * j + 2];
-        return v;
-    };
-    // the largest |x| as bits: above every finite value for an infinity or a NaN
-    auto fold = [](uint32_t mx, f32x4 v) {
-        const uint32_t a = max(f32_bits(v.x) & 0x7FFFFFFFu, f32_bits(v.y) & 0x7FFFFFFFu);
-        const uint32_t b = max(f32_bits(v.z) & 0x7FFFFFFFu, f32_bits(v.w) & 0x7FFFFFFFu);
-        return max(mx, max(a, b));
-    };
-    const int items = lda / 4;
-    f32x4 v[kItems];
-    uint32_t mx = 0;
-#pragma unroll
-    for (int i = 0; i < kItems; ++i) v[i] = load(tid + 256 * i);
-#pragma unroll
-    for (int i = 0; i < kItems; ++i) mx = fold(mx, v[i]);
-    for (int j = tid + 256 * kItems; j < items; j += 256) mx = fold(mx, load(j));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = max(mx, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mx), o, kWave)));
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    mx = max(max(red[0], red[1]), max(red[2], red[3]));
-    const bool finite = mx < 0x7F800000u;
-    const int e = max(static_cast<int>(mx >> 23), 1) - 127;
-    if (tid == 0) ea[row] = finite ? e : kNotFinite;
-    int8_t* dst = d + static_cast<int64_t>(row) * 4 * lda;
-    auto digits = [&](float f) -> uint32_t {
-        const int i = static_cast<int>(rintf(ldexpf(f, 29 - e)));
-        return (static_cast<uint32_t>(i) + 0x00808080u) ^ 0x00808080u;
-    };
-    auto store = [&](int j, f32x4 f) {
-        uint32_t a = 0, b = 0, c = 0, g = 0;
-        if (finite) {
-            a = digits(f.x);
-            b = digits(f.y);
-            c = digits(f.z);
-            g = digits(f.w);
-        }
-        // 4 x 4 byte transpose: word r = digit r of the four values
-        const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u), ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u);
-        const uint32_t cg0 = __builtin_amdgcn_perm(g, c, 0x05010400u), cg1 = __builtin_amdgcn_perm(g, c, 0x07030602u);
-        uint32_t* o = reinterpret_cast<uint32_t*>(dst) + j;
-        const int step = lda / 4;
-        o[0] = __builtin_amdgcn_perm(cg0, ab0, 0x05040100u);
-        o[step] = __builtin_amdgcn_perm(cg0, ab0, 0x07060302u);
-        o[2 * step] = __builtin_amdgcn_perm(cg1, ab1, 0x05040100u);
-        o[3 * step] = __builtin_amdgcn_perm(cg1, ab1, 0x07060302u);
-    };
-#pragma unroll
-    for (int i = 0; i < kItems; ++i)
-        if (tid + 256 * i < items) store(tid + 256 * i, v[i]);
-    for (int j = tid + 256 * kItems; j < items; j += 256) store(j, load(j));
 }
 
 // ------------------------------------------------------------------ host side

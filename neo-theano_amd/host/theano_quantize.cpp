@@ -564,6 +564,8 @@ Result<QuantizedLinear> QuantizedLinear::from_tensors(const Tensor& weight, cons
 size_t QuantizedLinear::workspace_bytes(int64_t m) const {
     const int64_t n = static_cast<int64_t>(out_), k = static_cast<int64_t>(in_);
     if (mode_ == Mode::FP8 && m <= kFusedA8MaxM) return static_cast<size_t>(m) * in_ * sizeof(float);
+    if (mode_ == Mode::W8) return static_cast<size_t>(tq_gemm_w8_workspace_bytes(m, n, k));
+    if (mode_ == Mode::FP8Weight) return static_cast<size_t>(tq_gemm_fp8_weight_workspace_bytes(m, n, k));
     if (mode_ == Mode::FP8) return static_cast<size_t>(tq_gemm_fp8_workspace_bytes(m, n, k));
     if (mode_ == Mode::W8A8) return static_cast<size_t>(tq_gemm_w8a8_workspace_bytes(m, n, k));
     if (mode_ != Mode::W4 || m <= 16 || (w4_.tile_rows > 0 && m <= kTiledPassesMaxM)) return 0;
@@ -575,8 +577,9 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
     const auto ts = reinterpret_cast<tq_stream_t>(stream);
     const float* b = bias_ ? bias_->data() : nullptr;
     const int64_t n = static_cast<int64_t>(out_), k = static_cast<int64_t>(in_);
-    // the workspace forms split K over blocks; a smaller workspace is not used
-    const bool has_ws = workspace && workspace_bytes >= this->workspace_bytes(m);
+    // the workspace forms: a smaller or misaligned workspace is not used
+    const bool has_ws = workspace && workspace_bytes >= this->workspace_bytes(m) &&
+                        reinterpret_cast<uintptr_t>(workspace) % 256 == 0;
     int st = TQ_OK;
     switch (mode_) {
         case Mode::W4: {
@@ -598,6 +601,11 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
         }
         case Mode::W8: {
             const auto* xf = static_cast<const float*>(x);
+            if (has_ws) {
+                st = tq_gemm_w8(xf, m, w8_.codes.data(), w8_.scales.data(), b, n, k, workspace,
+                                static_cast<int64_t>(workspace_bytes), y, ts);
+                break;
+            }
             for (int64_t m0 = 0; m0 < m && st == TQ_OK; m0 += 16) {
                 const int64_t mm = std::min<int64_t>(16, m - m0);
                 st = tq_gemv_w8(xf + m0 * k, mm, w8_.codes.data(), w8_.scales.data(), b, n, k, y + m0 * n, ts);
@@ -652,6 +660,11 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
         }
         case Mode::FP8Weight: {
             const auto* xf = static_cast<const float*>(x);
+            if (has_ws) {
+                st = tq_gemm_fp8_weight(xf, m, fp8_.codes.data(), fp8_.scales.data(), b, n, k, workspace,
+                                        static_cast<int64_t>(workspace_bytes), y, ts);
+                break;
+            }
             for (int64_t m0 = 0; m0 < m && st == TQ_OK; m0 += 16) {
                 const int64_t mm = std::min<int64_t>(16, m - m0);
                 st = tq_gemv_fp8(xf + m0 * k, mm, fp8_.codes.data(), fp8_.scales.data(), b, n, k, y + m0 * n, ts);
@@ -691,7 +704,11 @@ Result<Tensor> QuantizedLinear::try_forward(const Tensor& input) const {
                                    wsb ? ws.data() : nullptr, wsb);
                 if (r.is_ok()) check_hip(hipStreamSynchronize(stream_), "QuantizedLinear::forward");
             } else {
-                r = forward_device(xd.data(), static_cast<int64_t>(m), y.data(), stream_);
+                const size_t wsb = workspace_bytes(static_cast<int64_t>(m));
+                DeviceBuffer<uint8_t> ws(std::max<size_t>(wsb, 1));
+                r = forward_device(xd.data(), static_cast<int64_t>(m), y.data(), stream_, nullptr, nullptr,
+                                   wsb ? ws.data() : nullptr, wsb);
+                if (r.is_ok()) check_hip(hipStreamSynchronize(stream_), "QuantizedLinear::forward");
             }
         }
         if (r.is_err()) return r.unwrap_err();

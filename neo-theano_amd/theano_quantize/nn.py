@@ -17,12 +17,13 @@ Modes (chosen from the QConfig):
            activations (QConfig with weight_dtype and activation_dtype FP8);
   * "fp8_weight"  FP8 e4m3 weight-only, f32 activations (weight_dtype FP8,
            activations not FP8).
-Decode shapes (M <= 16 tokens) run the dequant-GEMV kernels; in "w8a8" and
-"fp8" modes the GEMV quantizes the activation rows itself (the same codes and
-product as quantize + GEMM, one launch).  "w4" runs the tiled GEMV in passes of
-16 tokens up to M = 32, where it is faster than the prefill GEMM, whose 64-row
-M tiles are mostly empty there.  Prefill shapes run the i8-MFMA W8A8 GEMM, the
-fp8-MFMA GEMM or the bf16-MFMA W4A16 GEMM.
+Decode shapes (a few tokens) run the dequant-GEMV kernels; in "w8a8" and "fp8"
+modes the GEMV quantizes the activation rows itself (the same codes and product
+as quantize + GEMM, one launch).  "w4" runs the tiled GEMV in passes of 16 tokens
+up to M = 32, where it is faster than the prefill GEMM, whose 64-row M tiles are
+mostly empty there.  Prefill shapes run the matrix cores: i8 for W8A8 and for the
+INT8 weight-only mode (f32 activations as exact integer digits), fp8, and bf16 for
+the FP8 weight-only and W4A16 modes.
 """
 from __future__ import annotations
 
@@ -174,10 +175,9 @@ class QuantizedLinear(Module):
                 _abi.call("tq_gemm_w4g128_bf16_ws", ptr(x), m, ptr(self.qweight), ptr(self.scales), ptr(self.bias),
                           n, k, ptr(ws), nb, ptr(y), stream())
         elif self.mode == "w8":
-            for m0 in range(0, m, DECODE_MAX_M):
-                mm = min(DECODE_MAX_M, m - m0)
-                _abi.call("tq_gemv_w8", ptr(x[m0:m0 + mm]), mm, ptr(self.qweight), ptr(self.scales),
-                          ptr(self.bias), n, k, ptr(y[m0:m0 + mm]), stream())
+            ws, nb = self._workspace("tq_gemm_w8_workspace_bytes", m, x.device)
+            _abi.call("tq_gemm_w8", ptr(x), m, ptr(self.qweight), ptr(self.scales), ptr(self.bias), n, k, ptr(ws), nb,
+                      ptr(y), stream())
         elif self.mode in ("w8a8", "fp8") and m <= FUSED_A8_MAX_M and _fused_a8_ok(x, self.qweight, k):
             # activation quantization fused into the decode GEMV (one launch)
             _abi.call("tq_gemv_w8a8" if self.mode == "w8a8" else "tq_gemv_fp8a8", ptr(x), m, ptr(self.qweight),
@@ -196,10 +196,9 @@ class QuantizedLinear(Module):
                 xq = torch.empty_like(x)
                 _abi.call("tq_fake_quantize_fp8_rowwise", ptr(x), m, k, ptr(qa), ptr(sa), ptr(xq), stream())
                 x = xq
-            for m0 in range(0, m, DECODE_MAX_M):
-                mm = min(DECODE_MAX_M, m - m0)
-                _abi.call("tq_gemv_fp8", ptr(x[m0:m0 + mm]), mm, ptr(self.qweight), ptr(self.scales),
-                          ptr(self.bias), n, k, ptr(y[m0:m0 + mm]), stream())
+            ws, nb = self._workspace("tq_gemm_fp8_weight_workspace_bytes", m, x.device)
+            _abi.call("tq_gemm_fp8_weight", ptr(x), m, ptr(self.qweight), ptr(self.scales), ptr(self.bias), n, k,
+                      ptr(ws), nb, ptr(y), stream())
         else:
             qa = torch.empty((m, k), dtype=torch.int8, device=x.device)
             sa = torch.empty(m, dtype=torch.float32, device=x.device)

@@ -102,6 +102,87 @@ def test_fp8_nan_code_stays_in_its_row_and_column(tq):
     assert torch.equal(y.isnan(), nan)
 
 
+def _weight_only(torch, fp8, x, qw, m, n, k, bias, off):
+    from theano_quantize import _abi
+    from theano_quantize._tensor import ptr, stream
+
+    g = torch.Generator(device="cuda").manual_seed(m + 7 * n)
+    sw = torch.rand(n, generator=g, device="cuda") + 0.5
+    b = torch.randn(n, generator=g, device="cuda") if bias else None
+    kw, vw = _at_offset(torch, qw, off)
+    name = "tq_gemm_fp8_weight" if fp8 else "tq_gemm_w8"
+    nb = int(getattr(_abi.lib(), name + "_workspace_bytes")(m, n, k))
+    ws = torch.empty(max(nb, 8), dtype=torch.uint8, device="cuda").fill_(0xA5)
+    y = torch.full((m, n), float("nan"), device="cuda")
+    _abi.call(name, ptr(x), m, ptr(vw), ptr(sw), ptr(b), n, k, ptr(ws), nb, ptr(y), stream())
+    torch.cuda.synchronize()
+    return y, sw, b
+
+
+@pytest.mark.parametrize("m,n,k", [s for s in SHAPES if s[0] > 8] + [(9, 4096, 4096), (512, 512, 1024), (300, 4096, 256)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_weight_only_any_shape(tq, m, n, k, fp8):
+    """f32 activations with rows of very different magnitudes (and zero, subnormal and
+    huge ones) times 8-bit codes against float64."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(m, k, generator=g, device="cuda")
+    x *= (10.0 ** torch.linspace(-8, 8, m, device="cuda"))[:, None]
+    x[1] = 0
+    x[2] *= 1e-36
+    x[3, k // 2] *= 1e4  # one value far above its row
+    qw = _codes(torch, (n, k), 8, fp8)
+    for off in (0, 1):
+        y, sw, b = _weight_only(torch, fp8, x, qw, m, n, k, off == 1, off)
+        ref = x.double() @ qw.double().t().contiguous() * sw.double()
+        scale = (x.double().abs() @ qw.double().abs().t().contiguous()) * sw.double()
+        if b is not None:
+            ref = ref + b.double()
+        # INT8: 2^(e - 30) per value, e the exponent of the row's largest, and the final
+        # rounding (below 2^-126 at its least); FP8: as the sums of test_fp8_any_shape, and
+        # bits of x below 2^-133 have no place in a bf16 plane
+        tiny = 2.0 ** -126
+        wsum = qw.double().abs().sum(1) * sw.double()
+        if fp8:
+            bound = 2.0 ** -23 * min(k, 512) ** 0.5 * scale + 2.0 ** -23 * ref.abs() + 2.0 ** -133 * wsum + tiny
+        else:
+            bound = 2.0 ** -30 * x.double().abs().amax(1)[:, None] * wsum + 2.0 ** -24 * ref.abs() + tiny
+        err = (y.double() - ref).abs()
+        assert bool((err <= bound).all()), (err / bound).max().item()
+        rows = torch.arange(m, device="cuda") > 2
+        rel = (err[rows].norm(dim=1) / ref[rows].norm(dim=1)).max().item()
+        assert rel < (4e-7 if fp8 else 1e-7) * (1 + 64 / (n * k) ** 0.5), rel
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("n,k", [(48, 384), (33, 130), (512, 2048)])
+def test_weight_only_rows_that_are_not_finite(tq, fp8, n, k):
+    import torch
+
+    m = 40
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(m, k, generator=g, device="cuda")
+    x[5, 3] = float("inf")
+    x[6, k - 1] = float("-inf")
+    x[7, 0] = float("nan")
+    x.view(torch.int32)[8, 1] = 0x7F800001  # a NaN whose high half is an infinity's
+    x[9, 2], x[9, 4] = float("inf"), float("-inf")
+    x[10, 1] = 3.0e38
+    qw = _codes(torch, (n, k), 9, fp8)
+    y, sw, _ = _weight_only(torch, fp8, x, qw, m, n, k, False, 0)
+    ref = x.double() @ qw.double().t().contiguous() * sw.double()
+    # every class as the exact sum has it, in every row (3e38 times a code past 1 overflows f32)
+    f32 = ref.float()
+    assert torch.equal(y.isnan(), f32.isnan())
+    rows = [i for i in range(m) if i != 10]
+    assert torch.equal(y[rows].isinf(), f32[rows].isinf())
+    inf = f32[rows].isinf()
+    assert torch.equal(y[rows][inf], f32[rows][inf])
+    fin = torch.tensor([i for i in range(m) if i not in (5, 6, 7, 8, 9, 10)], device="cuda")
+    assert ((y[fin].double() - ref[fin]).norm() / ref[fin].norm()).item() < 4e-7
+
+
 def test_workspace_too_small_is_refused(tq):
     import torch
 
