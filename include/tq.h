@@ -203,8 +203,9 @@ int tq_dequantize_i4_g128(const uint8_t* packed, const uint16_t* s_f16, int64_t 
 
 /* Decode-shaped GEMV, INT8 per-row weights, f32 activations x [M, K], M <= 16
  * (longer inputs run in chunks of 16 rows).  Any N, K; f32 pointers 4-byte
- * aligned.  The tuned kernel serves K % 16 == 0, K <= 8192 with x and q 16-byte
- * aligned; other shapes take a shape-general kernel. */
+ * aligned.  One kernel serves K % 16 == 0, K <= 8192 with x and q 16-byte aligned,
+ * another K up to 16384 at any alignment; very short or longer rows take a
+ * shape-general kernel. */
 int tq_gemv_w8(const float* x, int64_t m, const int8_t* q, const float* s,
                const float* bias, int64_t n, int64_t k, float* y, tq_stream_t stream);
 
@@ -214,12 +215,12 @@ int tq_gemv_w8(const float* x, int64_t m, const int8_t* q, const float* s,
 int tq_gemv_fp8(const float* x, int64_t m, const uint8_t* q, const float* s,
                 const float* bias, int64_t n, int64_t k, float* y, tq_stream_t stream);
 
-/* The two weight-only Linears above at any M: the GEMV for M <= 8, the matrix cores
- * beyond.  INT8: each row of x becomes a 31-bit fixed-point number in four int8 digit
+/* The two weight-only Linears above at any M: the GEMV for a few tokens (up to 4
+ * to 8), the matrix cores beyond.  INT8: each row of x becomes a 31-bit fixed-point number in four int8 digit
  * rows and the sums are exact integers (closer to the exact y than f32 sums; a row
  * holding an infinity or a NaN is summed in f32).  FP8: x split exactly into three
  * bf16 planes, f32 sums.  Any N, K; f32 pointers 4-byte aligned.  `workspace`: device
- * memory of at least the ..._workspace_bytes(M, N, K) bytes (0 for M <= 8), 256-byte
+ * memory of at least the ..._workspace_bytes(M, N, K) bytes (0 where the GEMV runs), 256-byte
  * aligned, contents need not be initialised. */
 int64_t tq_gemm_w8_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int tq_gemm_w8(const float* x, int64_t m, const int8_t* q, const float* s, const float* bias,

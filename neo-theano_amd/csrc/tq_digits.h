@@ -40,12 +40,12 @@ __device__ __forceinline__ float digit_out(int64_t v, int e, float sw, float b, 
 // x [rows, k] f32 -> digit rows [4 rows, lda] (zeros past k) and the row exponents:
 // one block per row; v = x * 2^(29 - e) rounded to an integer (|v| <= 2^30), whose
 // balanced base-256 digits are the bytes of (v + 0x808080) ^ 0x808080 (the top one
-// signed).  The row stays in registers between its maximum and its digits (up to
-// kItems x 1024 values; longer rows are read again).
-template <int kItems>
-__global__ __launch_bounds__(256) void k_split_rows(const float* __restrict__ x, int k, int lda,
+// signed).  The row stays in registers between its maximum and its digits (up to 4
+// kItems kThreads values; longer rows are read again).
+template <int kItems, int kThreads>
+__global__ __launch_bounds__(kThreads) void k_split_rows(const float* __restrict__ x, int k, int lda,
                                                     int8_t* __restrict__ d, int* __restrict__ ea) {
-    __shared__ uint32_t red[4];
+    __shared__ uint32_t red[kThreads / kWave];
     const int row = blockIdx.x, tid = threadIdx.x;
     const float* src = x + static_cast<int64_t>(row) * k;
     auto load = [&](int j) -> f32x4 {  // values 4 j .. 4 j + 3, zeros past k
@@ -66,15 +66,16 @@ __global__ __launch_bounds__(256) void k_split_rows(const float* __restrict__ x,
     f32x4 v[kItems];
     uint32_t mx = 0;
 #pragma unroll
-    for (int i = 0; i < kItems; ++i) v[i] = load(tid + 256 * i);
+    for (int i = 0; i < kItems; ++i) v[i] = load(tid + kThreads * i);
 #pragma unroll
     for (int i = 0; i < kItems; ++i) mx = fold(mx, v[i]);
-    for (int j = tid + 256 * kItems; j < items; j += 256) mx = fold(mx, load(j));
+    for (int j = tid + kThreads * kItems; j < items; j += kThreads) mx = fold(mx, load(j));
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = max(mx, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mx), o, kWave)));
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
-    mx = max(max(red[0], red[1]), max(red[2], red[3]));
+#pragma unroll
+    for (int i = 0; i < kThreads / kWave; ++i) mx = max(mx, red[i]);
     const bool finite = mx < 0x7F800000u;
     const int e = max(static_cast<int>(mx >> 23), 1) - 127;
     if (tid == 0) ea[row] = finite ? e : kNotFinite;
@@ -103,8 +104,21 @@ __global__ __launch_bounds__(256) void k_split_rows(const float* __restrict__ x,
     };
 #pragma unroll
     for (int i = 0; i < kItems; ++i)
-        if (tid + 256 * i < items) store(tid + 256 * i, v[i]);
-    for (int j = tid + 256 * kItems; j < items; j += 256) store(j, load(j));
+        if (tid + kThreads * i < items) store(tid + kThreads * i, v[i]);
+    for (int j = tid + kThreads * kItems; j < items; j += kThreads) store(j, load(j));
+}
+
+// Few rows: 1024 threads a row, for the latency of one pass over it; many: 256.
+inline int launch_split_rows(const float* x, int m, int k, int lda, int8_t* d, int* ea, hipStream_t st,
+                             const char* what) {
+    const unsigned rows = static_cast<unsigned>(m);
+    if (m <= 2 * device_cu_count())
+        k_split_rows<4, 1024><<<rows, 1024, 0, st>>>(x, k, lda, d, ea);
+    else if (lda <= 4096)
+        k_split_rows<4, 256><<<rows, 256, 0, st>>>(x, k, lda, d, ea);
+    else
+        k_split_rows<16, 256><<<rows, 256, 0, st>>>(x, k, lda, d, ea);
+    return check_launch(what);
 }
 
 }  // namespace

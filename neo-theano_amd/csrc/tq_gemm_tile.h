@@ -26,7 +26,7 @@
 // Any M, N, K and any alignment of A, W and their rows (element-aligned
 // pointers): global loads are 8 to 32 bytes per lane at byte (codes) or 4-byte
 // (f32) alignment, which global memory instructions take on this target; the
-// last, partial K stage loads element by element; rows past M or N re-read the
+// last, partial K stage is loaded apart, with zeros past K; rows past M or N re-read the
 // last row and are not stored.
 #pragma once
 
@@ -65,10 +65,12 @@ struct SrcF32 {
     __device__ static Raw load(const elem_t* p) {
         return Raw{*reinterpret_cast<const f32x4_a4*>(p), *reinterpret_cast<const f32x4_a4*>(p + 4)};
     }
-    __device__ static Raw load_part(const elem_t* p, int n) {
+    __device__ static Raw load_tail(const elem_t* p, int n, int) {
         float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = i < n ? p[i] : 0.0f;
+        for (int i = 0; i < 8; ++i) v[i] = p[min(i, n - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = i < n ? v[i] : 0.0f;
         return Raw{f32x4{v[0], v[1], v[2], v[3]}, f32x4{v[4], v[5], v[6], v[7]}};
     }
     __device__ static void planes(const Raw& r, u32x4 (&out)[kPlanes]) {
@@ -87,6 +89,43 @@ struct SrcF32 {
         out[2] = u32x4{pack_hi(l[0], l[1]), pack_hi(l[2], l[3]), pack_hi(l[4], l[5]), pack_hi(l[6], l[7])};
     }
 };
+
+// The first `take` (<= 16) bytes from p, zeros after them, where `n` bytes of a row of
+// `k` are left from p on (none: n <= 0).  Rows of 16 bytes and more: one load of 16
+// bytes that ends where the row does at the latest, shifted into place; shorter rows
+// byte by byte.
+__device__ __forceinline__ u32x4 bytes_tail(const uint8_t* p, int take, int n, int k) {
+    uint64_t lo = 0, hi = 0;
+    if (k >= 16) {  // uniform
+        const int back = n >= 16 ? 0 : 16 - n;  // bytes before p that the load takes in
+        const u32x4 v = *reinterpret_cast<const u32x4_a1*>(p - back);
+        lo = v.x | static_cast<uint64_t>(v.y) << 32;
+        hi = v.z | static_cast<uint64_t>(v.w) << 32;
+        if (back >= 8) {
+            lo = hi;
+            hi = 0;
+        }
+        const int s = 8 * (back & 7);
+        if (s) {
+            lo = (lo >> s) | (hi << (64 - s));
+            hi >>= s;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const uint64_t b = p[min(i, n - 1)];
+            if (i < 8)
+                lo |= b << (8 * i);
+            else
+                hi |= b << (8 * (i - 8));
+        }
+    }
+    // zero what `take` leaves out
+    lo = take >= 8 ? lo : take <= 0 ? 0 : lo & (~uint64_t{0} >> (64 - 8 * take));
+    hi = take >= 16 ? hi : take <= 8 ? 0 : hi & (~uint64_t{0} >> (128 - 8 * take));
+    return u32x4{static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi),
+                 static_cast<uint32_t>(hi >> 32)};
+}
 
 // 8 byte codes per chunk: the value of each as bf16 (exact).
 struct ValI8 {
@@ -109,12 +148,9 @@ struct SrcBf16 {
         u32x2 v;
     };
     __device__ static Raw load(const elem_t* p) { return Raw{*reinterpret_cast<const u32x2_a1*>(p)}; }
-    __device__ static Raw load_part(const elem_t* p, int n) {
-        uint32_t w[2] = {0u, 0u};
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (i < n) w[i >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(p[i])) << (8 * (i & 3));
-        return Raw{u32x2{w[0], w[1]}};
+    __device__ static Raw load_tail(const elem_t* p, int n, int k) {
+        const u32x4 v = bytes_tail(reinterpret_cast<const uint8_t*>(p), min(n, 8), n, k);
+        return Raw{u32x2{v.x, v.y}};
     }
     __device__ static void planes(const Raw& r, u32x4 (&out)[1]) {
         uint32_t f[8];
@@ -133,12 +169,8 @@ struct SrcBytes {
         u32x4 v;
     };
     __device__ static Raw load(const elem_t* p) { return Raw{*reinterpret_cast<const u32x4_a1*>(p)}; }
-    __device__ static Raw load_part(const elem_t* p, int n) {
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (i < n) w[i >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(p[i])) << (8 * (i & 3));
-        return Raw{u32x4{w[0], w[1], w[2], w[3]}};
+    __device__ static Raw load_tail(const elem_t* p, int n, int k) {
+        return Raw{bytes_tail(reinterpret_cast<const uint8_t*>(p), min(n, 16), n, k)};
     }
     __device__ static void planes(const Raw& r, u32x4 (&out)[1]) { out[0] = r.v; }
 };
@@ -436,16 +468,16 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
         }
         if (s < s_full) stage(lds, lds + kStage, rg[1], s_last);
     }
-    if (s_full < s_end) {  // the partial last stage, element by element (zeros past K)
+    if (s_full < s_end) {  // the partial last stage (zeros past K)
         const int k0 = s_full * BK + chunk * SA::kElems;
 #pragma unroll
         for (int i = 0; i < kAItems; ++i) {
-            rg[0].a[i] = SA::load_part(asrc[i] + k0, p.k - k0);
+            rg[0].a[i] = SA::load_tail(asrc[i] + k0, p.k - k0, p.k);
             store_a(rg[0], i, lds);
         }
 #pragma unroll
         for (int i = 0; i < kWItems; ++i) {
-            rg[0].w[i] = SW::load_part(wsrc[i] + k0, p.k - k0);
+            rg[0].w[i] = SW::load_tail(wsrc[i] + k0, p.k - k0, p.k);
             store_w(rg[0], i, lds);
         }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");

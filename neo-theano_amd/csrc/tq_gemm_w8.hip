@@ -5,7 +5,8 @@
 //
 // the reference's Linear::forward (crates/theano-nn/src/linear.rs:111-121) over
 // the dequantized weight.  The GEMV (tq_gemv.hip) reads the weights once per 4
-// tokens; here they are read once per 16 to 32 (digit rows) or 64 tokens.
+// tokens; here they are read once per 16 to 32 (digit rows) or 64 tokens.  Which one
+// runs: gemv_runs below.
 //
 // INT8: the activations become digit rows (tq_digits.h, one small launch) and the
 // product is the W8A8 GEMM's with four digit rows per token: the LDS-DMA kernel's
@@ -20,9 +21,22 @@
 namespace tq {
 namespace {
 
-// At most this many tokens run the GEMV in passes of 4 (N = K = 4096: 7.2 us a
-// pass against 17 us for split, GEMM and finish at 9 to 16 tokens).
-constexpr int64_t kGemvMaxM = 8;
+// Which calls run the GEMV (passes over the weights of 4 tokens, of 2 past K = 4096)
+// and which the matrix cores, whose split and finish launches cost ~6 us: up to 4
+// tokens the GEMV (N = K = 4096: 6.9 us at 4; N = 4096, K = 8192: 16 us on both); past
+// 8 the matrix cores (13 against 18 us at 9); between, the GEMV while a pass over the
+// weights is short (N = K = 4096: 11.5-13.5 us against 13; N = 14336, K = 4096: 29-34
+// against 20; N = 4096, K = 4097, 24-33 against 15).  The FP8 form's matrix kernel
+// takes longer: the GEMV's aligned form keeps all of its 5 to 8 tokens.
+bool gemv_runs(int64_t m, int64_t n, int64_t k, bool fp8) {
+    if (m <= 4 || m > 8) return m <= 4;
+    const bool vec16 = k % 16 == 0 && k <= 8192;
+    return vec16 ? fp8 || n * k <= 4096 * 4096 : n * k <= 2 << 20;
+}
+// So little work that one launch of a wave per output is ahead (N = 1000, K = 100: 3.9
+// against 7.1 us at 16 tokens).
+bool tiny(int64_t m, int64_t n, int64_t k) { return k < 16 || (m * n <= 1 << 22 && m * n * k <= 4 << 20); }
+
 constexpr int kDmaStageW8 = 1000;  // ns per stage of the DMA kernel's tiles
 
 int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
@@ -60,7 +74,7 @@ using namespace tq;
 extern "C" {
 
 int64_t tq_gemm_w8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
-    if (m <= kGemvMaxM || n <= 0 || k <= 0 || !w8_fits(m, n, k)) return 0;
+    if (n <= 0 || k <= 0 || gemv_runs(m, n, k, false) || tiny(m, n, k) || !w8_fits(m, n, k)) return 0;
     return w8_workspace(m, k).part + tile_plan<GemmW8>(m, n, k, 0, true).part_bytes;
 }
 
@@ -68,9 +82,9 @@ int tq_gemm_w8(const float* x, int64_t m, const int8_t* q, const float* s, const
                void* workspace, int64_t workspace_bytes, float* y, tq_stream_t stream) {
     const int rc = check_args(x, m, q, s, bias, n, k, y, "tq_gemm_w8");
     if (rc != TQ_OK || m == 0 || n == 0) return rc;
-    if (m <= kGemvMaxM) return tq_gemv_w8(x, m, q, s, bias, n, k, y, stream);
+    if (gemv_runs(m, n, k, false)) return tq_gemv_w8(x, m, q, s, bias, n, k, y, stream);
     const hipStream_t st = as_hip(stream);
-    if (k == 0 || !w8_fits(m, n, k)) return launch_linear_8bit_generic(x, m, q, s, bias, n, k, y, st);
+    if (tiny(m, n, k) || !w8_fits(m, n, k)) return launch_linear_8bit_generic(x, m, q, s, bias, n, k, y, st);
     const int64_t need = tq_gemm_w8_workspace_bytes(m, n, k);
     TQ_REQUIRE(workspace && aligned(workspace, 256) && workspace_bytes >= need,
                "tq_gemm_w8: workspace of %lld bytes (256-byte aligned), %lld needed", (long long)workspace_bytes,
@@ -78,13 +92,8 @@ int tq_gemm_w8(const float* x, int64_t m, const int8_t* q, const float* s, const
     const W8Workspace w = w8_workspace(m, k);
     int8_t* digits = static_cast<int8_t*>(workspace);
     int* ea = reinterpret_cast<int*>(digits + w.ea);
-    const unsigned rows = static_cast<unsigned>(m);
     const int ki = static_cast<int>(k), lda = static_cast<int>(w.lda);
-    if (lda <= 4096)
-        k_split_rows<4><<<rows, 256, 0, st>>>(x, ki, lda, digits, ea);
-    else
-        k_split_rows<16><<<rows, 256, 0, st>>>(x, ki, lda, digits, ea);
-    const int rs = check_launch("tq_gemm_w8 (split)");
+    const int rs = launch_split_rows(x, static_cast<int>(m), ki, lda, digits, ea, st, "tq_gemm_w8 (split)");
     if (rs != TQ_OK) return rs;
     const bool vec = n % 16 == 0 && k % kDmaBK == 0 && aligned(q, 16) && aligned(s, 16) && aligned(y, 16) &&
                      (!bias || aligned(bias, 16));
@@ -113,7 +122,7 @@ int tq_gemm_w8(const float* x, int64_t m, const int8_t* q, const float* s, const
 }
 
 int64_t tq_gemm_fp8_weight_workspace_bytes(int64_t m, int64_t n, int64_t k) {
-    if (m <= kGemvMaxM || n <= 0 || k <= 0 || !f8w_fits(m, n, k)) return 0;
+    if (n <= 0 || k <= 0 || gemv_runs(m, n, k, true) || tiny(m, n, k) || !f8w_fits(m, n, k)) return 0;
     return tile_plan<GemmF8W>(m, n, k, 0, true).part_bytes;
 }
 
@@ -121,9 +130,9 @@ int tq_gemm_fp8_weight(const float* x, int64_t m, const uint8_t* q, const float*
                        int64_t k, void* workspace, int64_t workspace_bytes, float* y, tq_stream_t stream) {
     const int rc = check_args(x, m, q, s, bias, n, k, y, "tq_gemm_fp8_weight");
     if (rc != TQ_OK || m == 0 || n == 0) return rc;
-    if (m <= kGemvMaxM) return tq_gemv_fp8(x, m, q, s, bias, n, k, y, stream);
+    if (gemv_runs(m, n, k, true)) return tq_gemv_fp8(x, m, q, s, bias, n, k, y, stream);
     const hipStream_t st = as_hip(stream);
-    if (k == 0 || !f8w_fits(m, n, k)) return launch_linear_8bit_generic(x, m, q, s, bias, n, k, y, st);
+    if (tiny(m, n, k) || !f8w_fits(m, n, k)) return launch_linear_8bit_generic(x, m, q, s, bias, n, k, y, st);
     const TilePlan plan = tile_plan<GemmF8W>(m, n, k, 0, true);
     TQ_REQUIRE(plan.part_bytes == 0 || (workspace && aligned(workspace, 8) && workspace_bytes >= plan.part_bytes),
                "tq_gemm_fp8_weight: workspace of %lld bytes, %lld needed", (long long)workspace_bytes,

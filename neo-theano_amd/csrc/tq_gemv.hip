@@ -11,6 +11,8 @@
 // non-temporal).  Lane l owns 16-byte slices of a row at byte 16*l of every
 // 1 KB chunk, so each wave-wide load is 1 KB contiguous; a row's partial dot
 // products meet in one wave64 butterfly.  Up to 4 tokens per pass.
+#include <algorithm>
+
 #include "tq_internal.h"
 #include "tq_rowfmt.h"
 
@@ -219,6 +221,123 @@ __global__ __launch_bounds__(64 * kWB, 8 / kWB) void k_gemv_w8(const float* __re
                 const float v = part[wv][ri][m] + part[wv + 1][ri][m];
                 y[m * y_stride + row] = s[row] * v + (bias ? bias[row] : 0.0f);
             }
+        }
+    }
+}
+
+// ------------------------------------------------------- any K from 16 to 16384
+// The same GEMV for long rows (K > 8192) and for K or addresses that are no multiple
+// of 16.  Every wave of a block takes its own kC chunks of 1024 k and holds that slice
+// of x in registers (read once per block, straight from global memory), kKS waves
+// sharing a run of rows; their partial sums of a row meet in LDS.  The weights come as
+// 16-byte loads at byte alignment.  Lane l of a chunk owns k0 = 1024 c + 16 l .. k0 +
+// 15; the lane K ends in reads the row's last 16 codes instead, with zeros for the x
+// values that its neighbour owns, and lanes past K the same with all zeros (a NaN code
+// there is one of the row's own, and makes its row NaN either way).  At N = 4096, K =
+// 14336: 13.0 us at one token, 25 at four, against 92 and 159 us for a wave per
+// output (tq_generic.hip); at K = 4097 7.9 against 28.5 us.
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+typedef i32x4 i32x4_a1 __attribute__((aligned(1)));
+constexpr int kLongWaves = 8;
+constexpr int kLongRun = 64;  // rows per run that the LDS partial sums hold
+
+template <class Code, int kM, int kC, int kKS>
+__global__ __launch_bounds__(64 * kLongWaves, 2) void k_gemv_long(const float* __restrict__ x, int64_t x_stride,
+                                                                  const typename Code::code_t* __restrict__ q,
+                                                                  const float* __restrict__ s,
+                                                                  const float* __restrict__ bias, int64_t n, int k,
+                                                                  float* __restrict__ y, int64_t y_stride,
+                                                                  int64_t run_rows, int tokens) {
+    constexpr int kRows = kC == 1 ? 4 : 2;  // rows per load group
+    __shared__ float part[kLongWaves][kLongRun][kM];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int slice = wv % kKS;
+    const int64_t run = static_cast<int64_t>(blockIdx.x) * (kLongWaves / kKS) + wv / kKS;
+    const int64_t row_begin = run * run_rows, row_end = min(n, row_begin + run_rows);
+    const int64_t row_clamp = min(max(row_begin, row_end - 1), n - 1);
+    int k0[kC], kb[kC];
+    float xr[kM][kC][16];
+#pragma unroll
+    for (int c = 0; c < kC; ++c) {
+        k0[c] = 1024 * (slice * kC + c) + 16 * lane;
+        kb[c] = min(k0[c], k - 16);
+#pragma unroll
+        for (int m = 0; m < kM; ++m)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int mi = kM > 4 ? min(m, tokens - 1) : m;  // only the 8-token form takes fewer
+                const f32x4 v = *reinterpret_cast<const f32x4_a4*>(x + mi * x_stride + kb[c] + 4 * j);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) xr[m][c][4 * j + b] = kb[c] + 4 * j + b >= k0[c] ? v[b] : 0.0f;
+            }
+    }
+    auto load_rows = [&](int64_t row0, i32x4 (&wq)[kRows][kC]) {
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            const typename Code::code_t* src = q + min(row0 + r, row_clamp) * k;
+#pragma unroll
+            for (int c = 0; c < kC; ++c)
+                wq[r][c] = __builtin_nontemporal_load(reinterpret_cast<const i32x4_a1*>(src + kb[c]));
+        }
+    };
+    auto group = [&](int64_t row0, const i32x4 (&cur)[kRows][kC]) {
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+            float acc[kM];
+#pragma unroll
+            for (int m = 0; m < kM; ++m) acc[m] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < kC; ++c)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float w4[4];
+                    Code::decode4(cur[r][c][j], w4);
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+#pragma unroll
+                        for (int m = 0; m < kM; ++m) acc[m] = fmaf(w4[b], xr[m][c][4 * j + b], acc[m]);
+                }
+            const int64_t row = row0 + r;
+#pragma unroll
+            for (int m = 0; m < kM; ++m) {
+                const float v = wave_sum(acc[m]);
+                if (lane == 0 && row < row_end) part[wv][row - row_begin][m] = v;
+            }
+        }
+    };
+    // two register buffers in turn, as in k_gemv_w8 (runs are whole groups)
+    i32x4 wa[kRows][kC], wb[kRows][kC];
+    if (row_begin < row_end) {
+        load_rows(row_begin, wa);
+        for (int64_t row0 = row_begin;;) {
+            if (row0 + kRows >= row_end) {
+                group(row0, wa);
+                break;
+            }
+            load_rows(row0 + kRows, wb);
+            group(row0, wa);
+            row0 += kRows;
+            if (row0 + kRows >= row_end) {
+                group(row0, wb);
+                break;
+            }
+            load_rows(row0 + kRows, wa);
+            group(row0, wb);
+            row0 += kRows;
+        }
+    }
+    __syncthreads();
+    // the first wave of a run adds its slices in order
+    if (slice == 0) {
+        for (int i = lane; i < (row_end - row_begin) * kM; i += kWave) {
+            const int ri = i / kM, m = i - ri * kM;
+            const int64_t row = row_begin + ri;
+            if (kM > 4 && m >= tokens) continue;
+            float v = part[wv][ri][m];
+#pragma unroll
+            for (int t = 1; t < kKS; ++t) v += part[wv + t][ri][m];
+            y[m * y_stride + row] = s[row] * v + (bias ? bias[row] : 0.0f);
         }
     }
 }
@@ -529,6 +648,32 @@ int gemv_a8(const float* x, int64_t m, const typename Fmt::code_t* q, const floa
     return TQ_OK;
 }
 
+template <class Code, int kM, int kC, int kKS>
+void launch_long(const float* x, int64_t xs, const typename Code::code_t* q, const float* s, const float* b, int64_t n,
+                 int64_t k, float* y, int64_t ys, int tokens, hipStream_t st) {
+    constexpr int kRows = kC == 1 ? 4 : 2, kRuns = kLongWaves / kKS;
+    // about two blocks per CU, runs of whole load groups
+    const int64_t slots = static_cast<int64_t>(device_cu_count()) * 2 * kRuns;
+    int64_t rows = (n + slots - 1) / slots;
+    rows = std::min<int64_t>((rows + kRows - 1) / kRows * kRows, kLongRun);
+    const int64_t runs = (n + rows - 1) / rows;
+    k_gemv_long<Code, kM, kC, kKS><<<static_cast<unsigned>((runs + kRuns - 1) / kRuns), 64 * kLongWaves, 0, st>>>(
+        x, xs, q, s, b, n, static_cast<int>(k), y, ys, rows, tokens);
+}
+
+// kM = the pass's tokens, or 8 >= them (the rest repeat the last and are not stored)
+template <class Code, int kM>
+void dispatch_long(const float* x, const typename Code::code_t* q, const float* s, const float* b, int64_t n,
+                   int64_t k, float* y, int tokens, hipStream_t st) {
+    if constexpr (kM <= 4) {
+        if (k > 8192) return launch_long<Code, kM, 2, 8>(x, k, q, s, b, n, k, y, n, tokens, st);
+        if (k > 4096) return launch_long<Code, kM, 1, 8>(x, k, q, s, b, n, k, y, n, tokens, st);
+        if (k > 2048) return launch_long<Code, kM, 1, 4>(x, k, q, s, b, n, k, y, n, tokens, st);
+    }
+    if (k > 1024) return launch_long<Code, kM, 1, 2>(x, k, q, s, b, n, k, y, n, tokens, st);
+    launch_long<Code, kM, 1, 1>(x, k, q, s, b, n, k, y, n, tokens, st);
+}
+
 template <class Code>
 int gemv_8bit(const float* x, int64_t m, const typename Code::code_t* q, const float* s, const float* bias,
               int64_t n, int64_t k, float* y, hipStream_t st, const char* what) {
@@ -540,9 +685,31 @@ int gemv_8bit(const float* x, int64_t m, const typename Code::code_t* q, const f
     TQ_REQUIRE(s, "%s: null scales", what);
     TQ_REQUIRE(aligned(x, 4) && aligned(s, 4) && (!bias || aligned(bias, 4)) && aligned(y, 4),
                "%s: misaligned f32 pointer", what);
-    // the tuned kernel streams 16-byte vectors of K-contiguous rows held in registers
-    if (k == 0 || k % 16 != 0 || k > 8 * 1024 || !aligned(x, 16) || !aligned(q, 16))
+    // the first kernel streams 16-byte vectors of K-contiguous rows held in registers;
+    // k_gemv_long takes longer rows and any alignment, four tokens per pass (eight of
+    // short rows: the tokens' x still fits the registers).  A wave per output stays
+    // ahead where a row is too short for a wave's 1024 k (N = 1000, K = 100: 2.1 to 2.8
+    // us at 1 to 8 tokens against 3.1 to 8.1; N = 1003, K = 1000: 4.7 to 6.6 against 3.2
+    // to 5.7 at 1 to 4 tokens, 7.3 against 9.2 at 8; N = 300, K = 5000: 22 against 11 at 8).
+    const bool vec16 = k % 16 == 0 && k <= 8 * 1024 && aligned(x, 16) && aligned(q, 16);
+    if (k < 16 || k > 16 * 1024 || (!vec16 && (k <= 512 || (m > 4 && m <= 8 && k <= 2048 && n * k <= 2 << 20))))
         return launch_linear_8bit_generic(x, m, q, s, bias, n, k, y, st);
+    if (!vec16) {
+        const int64_t per = k <= 2048 ? 8 : 4;
+        for (int64_t m0 = 0; m0 < m; m0 += per) {
+            const int mm = static_cast<int>(std::min<int64_t>(per, m - m0));
+            const float* xp = x + m0 * k;
+            float* yp = y + m0 * n;
+            if (mm == 1) dispatch_long<Code, 1>(xp, q, s, bias, n, k, yp, mm, st);
+            else if (mm == 2) dispatch_long<Code, 2>(xp, q, s, bias, n, k, yp, mm, st);
+            else if (mm == 3) dispatch_long<Code, 3>(xp, q, s, bias, n, k, yp, mm, st);
+            else if (mm == 4) dispatch_long<Code, 4>(xp, q, s, bias, n, k, yp, mm, st);
+            else dispatch_long<Code, 8>(xp, q, s, bias, n, k, yp, mm, st);
+            const int rc = check_launch(what);
+            if (rc != TQ_OK) return rc;
+        }
+        return TQ_OK;
+    }
     const int chunks = static_cast<int>((k + 1023) / 1024);
     const int64_t per_pass = chunks <= 4 ? 4 : 2;
     for (int64_t m0 = 0; m0 < m; m0 += per_pass) {
