@@ -312,6 +312,18 @@ int tq_gemm_fp8_ws(const uint8_t* qa, const float* sa, const uint8_t* qw, const 
                    const float* bias, int64_t m, int64_t n, int64_t k, void* workspace,
                    int64_t workspace_bytes, float* y, tq_stream_t stream);
 
+/* tq_quantize_{i8,fp8}_rowwise on x and tq_gemm_{w8a8,fp8}_ws in one call: the codes,
+ * their scales and the partial sums live in `workspace` (at least the
+ * ..._workspace_bytes(M, N, K) bytes, 256-byte aligned). */
+int64_t tq_linear_w8a8_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tq_linear_w8a8(const float* x, int64_t m, const int8_t* qw, const float* sw, const float* bias,
+                   int64_t n, int64_t k, void* workspace, int64_t workspace_bytes, float* y,
+                   tq_stream_t stream);
+int64_t tq_linear_fp8_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tq_linear_fp8(const float* x, int64_t m, const uint8_t* qw, const float* sw, const float* bias,
+                  int64_t n, int64_t k, void* workspace, int64_t workspace_bytes, float* y,
+                  tq_stream_t stream);
+
 /* Prefill-shaped W4A16: x bf16 [M, K], INT4 g128 weights, f32 accumulation with
  * the group scale applied to each 128-long partial sum; y f32 [M, N].
  * K % 128 == 0 (the format), any M, N.  The MFMA kernel serves N % 16 == 0 with

@@ -333,6 +333,16 @@ int64_t a8_part_bytes(int64_t m, int64_t n, int64_t k) {
     return tile_plan<T>(m, n, k, 0, true).part_bytes;
 }
 
+// workspace of tq_linear_{w8a8,fp8}: codes [m, k], then scales [m], then partial sums
+struct LinearA8 {
+    int64_t sa, part;
+};
+LinearA8 linear_a8_layout(int64_t m, int64_t k) {
+    if (m <= 0 || k < 0) return LinearA8{0, 0};
+    const int64_t sa = (m * k + 255) / 256 * 256;
+    return LinearA8{sa, sa + (4 * m + 255) / 256 * 256};
+}
+
 int gemm_w8a8(const int8_t* qa, const float* sa, const int8_t* qw, const float* sw, const float* bias, int64_t m,
               int64_t n, int64_t k, int32_t* acc, void* ws, int64_t ws_bytes, float* y, hipStream_t st,
               const char* what) {
@@ -447,6 +457,52 @@ int tq_gemm_fp8_ws(const uint8_t* qa, const float* sa, const uint8_t* qw, const 
                    int64_t m, int64_t n, int64_t k, void* workspace, int64_t workspace_bytes, float* y,
                    tq_stream_t stream) {
     return gemm_fp8(qa, sa, qw, sw, bias, m, n, k, workspace, workspace_bytes, y, as_hip(stream), "tq_gemm_fp8_ws");
+}
+
+// Quantize and GEMM of one call: the workspace holds the codes, their scales and the
+// GEMM's partial sums.
+int64_t tq_linear_w8a8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    return linear_a8_layout(m, k).part + tq_gemm_w8a8_workspace_bytes(m, n, k);
+}
+
+int tq_linear_w8a8(const float* x, int64_t m, const int8_t* qw, const float* sw, const float* bias, int64_t n,
+                   int64_t k, void* workspace, int64_t workspace_bytes, float* y, tq_stream_t stream) {
+    TQ_REQUIRE(m >= 0 && n >= 0 && k >= 0, "tq_linear_w8a8: negative shape");
+    if (m == 0 || n == 0) return TQ_OK;
+    const int64_t need = tq_linear_w8a8_workspace_bytes(m, n, k);
+    TQ_REQUIRE(workspace && aligned(workspace, 256) && workspace_bytes >= need,
+               "tq_linear_w8a8: workspace of %lld bytes (256-byte aligned), %lld needed", (long long)workspace_bytes,
+               (long long)need);
+    const LinearA8 w = linear_a8_layout(m, k);
+    int8_t* qa = static_cast<int8_t*>(workspace);
+    float* sa = reinterpret_cast<float*>(qa + w.sa);
+    const int64_t part = need - w.part;
+    const int rc = tq_quantize_i8_rowwise(x, m, k, qa, sa, stream);
+    if (rc != TQ_OK) return rc;
+    return gemm_w8a8(qa, sa, qw, sw, bias, m, n, k, nullptr, part ? qa + w.part : nullptr, part, y, as_hip(stream),
+                     "tq_linear_w8a8");
+}
+
+int64_t tq_linear_fp8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    return linear_a8_layout(m, k).part + tq_gemm_fp8_workspace_bytes(m, n, k);
+}
+
+int tq_linear_fp8(const float* x, int64_t m, const uint8_t* qw, const float* sw, const float* bias, int64_t n,
+                  int64_t k, void* workspace, int64_t workspace_bytes, float* y, tq_stream_t stream) {
+    TQ_REQUIRE(m >= 0 && n >= 0 && k >= 0, "tq_linear_fp8: negative shape");
+    if (m == 0 || n == 0) return TQ_OK;
+    const int64_t need = tq_linear_fp8_workspace_bytes(m, n, k);
+    TQ_REQUIRE(workspace && aligned(workspace, 256) && workspace_bytes >= need,
+               "tq_linear_fp8: workspace of %lld bytes (256-byte aligned), %lld needed", (long long)workspace_bytes,
+               (long long)need);
+    const LinearA8 w = linear_a8_layout(m, k);
+    uint8_t* qa = static_cast<uint8_t*>(workspace);
+    float* sa = reinterpret_cast<float*>(qa + w.sa);
+    const int64_t part = need - w.part;
+    const int rc = tq_quantize_fp8_rowwise(x, m, k, qa, sa, stream);
+    if (rc != TQ_OK) return rc;
+    return gemm_fp8(qa, sa, qw, sw, bias, m, n, k, part ? qa + w.part : nullptr, part, y, as_hip(stream),
+                    "tq_linear_fp8");
 }
 
 }  // extern "C"

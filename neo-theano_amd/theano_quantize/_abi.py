@@ -67,6 +67,10 @@ SIGNATURES = {
     "tq_gemm_w8a8_ws": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p, _i64, _p, _p],
     "tq_gemm_fp8_workspace_bytes": [_i64, _i64, _i64],
     "tq_gemm_fp8_ws": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _i64, _p, _p],
+    "tq_linear_w8a8_workspace_bytes": [_i64, _i64, _i64],
+    "tq_linear_w8a8": [_p, _i64, _p, _p, _p, _i64, _i64, _p, _i64, _p, _p],
+    "tq_linear_fp8_workspace_bytes": [_i64, _i64, _i64],
+    "tq_linear_fp8": [_p, _i64, _p, _p, _p, _i64, _i64, _p, _i64, _p, _p],
     "tq_dtype_size": [_int],
     "tq_convert": [_p, _int, _p, _int, _i64, _p],
     "tq_attention_f32": [_p, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _i64, _i64, _i64, _p, _i64, _p],
@@ -84,10 +88,12 @@ _RESTYPE = {"tq_status_string": ctypes.c_char_p, "tq_last_error": ctypes.c_char_
             "tq_w4g128_tile_rows": ctypes.c_int64, "tq_mlp_w4g128_workspace_bytes": ctypes.c_int64,
             "tq_mlp_w4g128_decode_workspace_bytes": ctypes.c_int64,
             "tq_gemm_w8_workspace_bytes": ctypes.c_int64, "tq_gemm_fp8_weight_workspace_bytes": ctypes.c_int64,
+            "tq_linear_w8a8_workspace_bytes": ctypes.c_int64, "tq_linear_fp8_workspace_bytes": ctypes.c_int64,
             "tq_gemm_w8a8_workspace_bytes": ctypes.c_int64, "tq_gemm_fp8_workspace_bytes": ctypes.c_int64,
             "tq_gemm_w4g128_bf16_workspace_bytes": ctypes.c_int64, "tq_dtype_size": ctypes.c_int64}
 
 _lib = None
+_entries = {}  # name -> ctypes function, filled when the library is loaded
 
 
 def lib():
@@ -102,15 +108,24 @@ def lib():
             fn = getattr(L, name)
             fn.argtypes = args
             fn.restype = _RESTYPE.get(name, _int)
+            _entries[name] = fn
         _lib = L
     return _lib
 
 
+def entry(name):
+    """The ctypes function of an entry point (addresses are passed as plain ints)."""
+    fn = _entries.get(name)
+    if fn is None:
+        lib()
+        fn = _entries[name]
+    return fn
+
+
 def call(name, *args):
     """Calls a status-returning entry point and raises the mapped exception."""
-    L = lib()
-    st = getattr(L, name)(*args)
+    st = (_entries.get(name) or entry(name))(*args)
     if st != 0:
-        msg = L.tq_last_error().decode(errors="replace")
+        msg = lib().tq_last_error().decode(errors="replace")
         raise_for_status(st, f"{name}: {msg}")
     return st

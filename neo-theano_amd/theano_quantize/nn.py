@@ -141,71 +141,62 @@ class QuantizedLinear(Module):
     def _act_dtype(self):
         return torch.bfloat16 if self.mode == "w4" else torch.float32
 
-    def _workspace(self, entry, m, device):
-        """(device scratch or None, its bytes) for m tokens, as `entry` sizes it."""
-        nb = int(getattr(_abi.lib(), entry)(m, self.out_features, self.in_features))
-        return (torch.empty(nb, dtype=torch.uint8, device=device) if nb else None), nb
+    def _run(self, name, x, m, y, st):
+        """`name` with the workspace that `name`_workspace_bytes asks for, allocated here."""
+        n, k, bias = self.out_features, self.in_features, self.bias
+        nb = _abi.entry(name + "_workspace_bytes")(m, n, k)
+        ws = x.new_empty(nb, dtype=torch.uint8) if nb else None
+        _abi.call(name, x.data_ptr(), m, self.qweight.data_ptr(), self.scales.data_ptr(), ptr(bias), n, k, ptr(ws), nb,
+                  y.data_ptr(), st)
 
     def forward(self, x):
         x = on_device(x, self._act_dtype(), "QuantizedLinear.forward")
         squeeze = x.dim() == 1
         if squeeze:
             x = x.unsqueeze(0)
-        if x.dim() != 2 or x.shape[1] != self.in_features:
+        n, k = self.out_features, self.in_features
+        if x.dim() != 2 or x.shape[1] != k:
             raise InvalidArgument(
                 f"QuantizedLinear.forward: shape mismatch, expected [*, {self.in_features}], "
                 f"got {tuple(x.shape)}")
         m = x.shape[0]
-        y = torch.empty((m, self.out_features), dtype=torch.float32, device=x.device)
-        n, k = self.out_features, self.in_features
-        if self.mode == "w4":
+        y = x.new_empty((m, n), dtype=torch.float32)
+        mode, st = self.mode, stream()
+        if mode == "w4":
+            bias = ptr(self.bias)
             if m <= TILED_PASSES_MAX_M and self.tiled is not None:
-                pt, st, t = self.tiled
-                for m0 in range(0, m, TILED_MAX_M):
-                    mm = min(TILED_MAX_M, m - m0)
-                    _abi.call("tq_gemv_w4g128_tiled", ptr(x[m0:m0 + mm]), mm, ptr(pt), ptr(st), ptr(self.bias), n,
-                              k, t, ptr(y[m0:m0 + mm]), stream())
+                pt, ts, t = self.tiled
+                xp, yp, pt, ts = x.data_ptr(), y.data_ptr(), pt.data_ptr(), ts.data_ptr()
+                for m0 in range(0, m, TILED_MAX_M):  # x rows are 2 K bytes, y rows 4 N
+                    _abi.call("tq_gemv_w4g128_tiled", xp + 2 * k * m0, min(TILED_MAX_M, m - m0), pt, ts, bias, n, k, t,
+                              yp + 4 * n * m0, st)
             elif m <= DECODE_MAX_M:
-                _abi.call("tq_gemv_w4g128", ptr(x), m, ptr(self.qweight), ptr(self.scales), ptr(self.bias), n, k,
-                          ptr(y), stream())
+                _abi.call("tq_gemv_w4g128", x.data_ptr(), m, self.qweight.data_ptr(), self.scales.data_ptr(), bias, n, k,
+                          y.data_ptr(), st)
             else:
                 # prefill: pipelined kernels with x's k-order and group sums in a workspace
-                nb = int(_abi.lib().tq_gemm_w4g128_bf16_workspace_bytes(m, k))
-                ws = torch.empty((max(nb, 1),), dtype=torch.uint8, device=x.device)
-                _abi.call("tq_gemm_w4g128_bf16_ws", ptr(x), m, ptr(self.qweight), ptr(self.scales), ptr(self.bias),
-                          n, k, ptr(ws), nb, ptr(y), stream())
-        elif self.mode == "w8":
-            ws, nb = self._workspace("tq_gemm_w8_workspace_bytes", m, x.device)
-            _abi.call("tq_gemm_w8", ptr(x), m, ptr(self.qweight), ptr(self.scales), ptr(self.bias), n, k, ptr(ws), nb,
-                      ptr(y), stream())
-        elif self.mode in ("w8a8", "fp8") and m <= FUSED_A8_MAX_M and _fused_a8_ok(x, self.qweight, k):
+                nb = _abi.entry("tq_gemm_w4g128_bf16_workspace_bytes")(m, k)
+                ws = x.new_empty(max(nb, 1), dtype=torch.uint8)
+                _abi.call("tq_gemm_w4g128_bf16_ws", x.data_ptr(), m, self.qweight.data_ptr(), self.scales.data_ptr(),
+                          bias, n, k, ws.data_ptr(), nb, y.data_ptr(), st)
+        elif mode == "w8":
+            self._run("tq_gemm_w8", x, m, y, st)
+        elif mode in ("w8a8", "fp8") and m <= FUSED_A8_MAX_M and _fused_a8_ok(x, self.qweight, k):
             # activation quantization fused into the decode GEMV (one launch)
-            _abi.call("tq_gemv_w8a8" if self.mode == "w8a8" else "tq_gemv_fp8a8", ptr(x), m, ptr(self.qweight),
-                      ptr(self.scales), ptr(self.bias), n, k, ptr(y), stream())
-        elif self.mode == "fp8" and m > FUSED_A8_MAX_M:
-            qa = torch.empty((m, k), dtype=torch.uint8, device=x.device)
-            sa = torch.empty(m, dtype=torch.float32, device=x.device)
-            _abi.call("tq_quantize_fp8_rowwise", ptr(x), m, k, ptr(qa), ptr(sa), stream())
-            ws, nb = self._workspace("tq_gemm_fp8_workspace_bytes", m, x.device)
-            _abi.call("tq_gemm_fp8_ws", ptr(qa), ptr(sa), ptr(self.qweight), ptr(self.scales),
-                      ptr(self.bias), m, n, k, ptr(ws), nb, ptr(y), stream())
-        elif self.mode in ("fp8", "fp8_weight"):
-            if self.mode == "fp8":  # x -> e4m3(qa) * sa, the GEMM's activation values
+            _abi.call("tq_gemv_w8a8" if mode == "w8a8" else "tq_gemv_fp8a8", x.data_ptr(), m, self.qweight.data_ptr(),
+                      self.scales.data_ptr(), ptr(self.bias), n, k, y.data_ptr(), st)
+        elif mode == "w8a8":
+            self._run("tq_linear_w8a8", x, m, y, st)
+        elif mode == "fp8" and m > FUSED_A8_MAX_M:
+            self._run("tq_linear_fp8", x, m, y, st)
+        else:
+            if mode == "fp8":  # x -> e4m3(qa) * sa, the GEMM's activation values
                 qa = torch.empty((m, k), dtype=torch.uint8, device=x.device)
                 sa = torch.empty(m, dtype=torch.float32, device=x.device)
                 xq = torch.empty_like(x)
-                _abi.call("tq_fake_quantize_fp8_rowwise", ptr(x), m, k, ptr(qa), ptr(sa), ptr(xq), stream())
+                _abi.call("tq_fake_quantize_fp8_rowwise", ptr(x), m, k, ptr(qa), ptr(sa), ptr(xq), st)
                 x = xq
-            ws, nb = self._workspace("tq_gemm_fp8_weight_workspace_bytes", m, x.device)
-            _abi.call("tq_gemm_fp8_weight", ptr(x), m, ptr(self.qweight), ptr(self.scales), ptr(self.bias), n, k,
-                      ptr(ws), nb, ptr(y), stream())
-        else:
-            qa = torch.empty((m, k), dtype=torch.int8, device=x.device)
-            sa = torch.empty(m, dtype=torch.float32, device=x.device)
-            _abi.call("tq_quantize_i8_rowwise", ptr(x), m, k, ptr(qa), ptr(sa), stream())
-            ws, nb = self._workspace("tq_gemm_w8a8_workspace_bytes", m, x.device)
-            _abi.call("tq_gemm_w8a8_ws", ptr(qa), ptr(sa), ptr(self.qweight), ptr(self.scales),
-                      ptr(self.bias), m, n, k, None, ptr(ws), nb, ptr(y), stream())
+            self._run("tq_gemm_fp8_weight", x, m, y, st)
         return y.squeeze(0) if squeeze else y
 
 
@@ -255,8 +246,8 @@ class QuantizedMLP(Module):
         """Device bytes of intermediates forward() needs for m tokens."""
         if self._decode_path(m):
             mm = min(m, DECODE_MLP_PASS_M)  # one pass at a time
-            return int(_abi.lib().tq_mlp_w4g128_decode_workspace_bytes(mm, self.d, self.f))
-        return int(_abi.lib().tq_mlp_w4g128_workspace_bytes(m, self.d, self.f))
+            return _abi.entry("tq_mlp_w4g128_decode_workspace_bytes")(mm, self.d, self.f)
+        return _abi.entry("tq_mlp_w4g128_workspace_bytes")(m, self.d, self.f)
 
     def forward(self, x, workspace=None):
         """y = (SiLU(x Wg^T) * (x Wu^T)) Wd^T for x bf16 [M, D]; `workspace` is an
@@ -264,22 +255,21 @@ class QuantizedMLP(Module):
         x = on_device(x, torch.bfloat16, "QuantizedMLP.forward")
         if x.dim() != 2 or x.shape[1] != self.d:
             raise InvalidArgument(f"QuantizedMLP.forward: expected [M, {self.d}], got {tuple(x.shape)}")
-        m = x.shape[0]
-        need = self.workspace_bytes(m)
+        m, d, f, st = x.shape[0], self.d, self.f, stream()
         if workspace is None:
-            workspace = torch.empty((max(need, 1),), dtype=torch.uint8, device=x.device)
-        y = torch.empty((m, self.d), dtype=torch.float32, device=x.device)
-        wsb = workspace.numel() * workspace.element_size()
+            workspace = x.new_empty(max(self.workspace_bytes(m), 1), dtype=torch.uint8)
+        y = x.new_empty((m, d), dtype=torch.float32)
+        ws, wsb = workspace.data_ptr(), workspace.numel() * workspace.element_size()
         if self._decode_path(m):
             gu_t, gu_st, dn_t, dn_st, dn_rows = self.decode
+            gu_t, gu_st, dn_t, dn_st = gu_t.data_ptr(), gu_st.data_ptr(), dn_t.data_ptr(), dn_st.data_ptr()
+            xp, yp = x.data_ptr(), y.data_ptr()  # x rows are 2 D bytes, y rows 4 D
             for m0 in range(0, m, DECODE_MLP_PASS_M):  # passes ordered on the stream share the workspace
-                mm = min(DECODE_MLP_PASS_M, m - m0)
-                _abi.call("tq_mlp_w4g128_decode", ptr(x[m0:m0 + mm]), mm, self.d, self.f, ptr(gu_t), ptr(gu_st),
-                          ptr(dn_t), ptr(dn_st), dn_rows, ptr(workspace), wsb, ptr(y[m0:m0 + mm]), stream())
+                _abi.call("tq_mlp_w4g128_decode", xp + 2 * d * m0, min(DECODE_MLP_PASS_M, m - m0), d, f, gu_t, gu_st,
+                          dn_t, dn_st, dn_rows, ws, wsb, yp + 4 * d * m0, st)
             return y
-        _abi.call("tq_mlp_w4g128", ptr(x), m, self.d, self.f, ptr(self.gate[0]), ptr(self.gate[1]),
-                  ptr(self.up[0]), ptr(self.up[1]), ptr(self.down[0]), ptr(self.down[1]),
-                  ptr(workspace), wsb, ptr(y), stream())
+        _abi.call("tq_mlp_w4g128", x.data_ptr(), m, d, f, ptr(self.gate[0]), ptr(self.gate[1]), ptr(self.up[0]),
+                  ptr(self.up[1]), ptr(self.down[0]), ptr(self.down[1]), ws, wsb, y.data_ptr(), st)
         return y
 
 
