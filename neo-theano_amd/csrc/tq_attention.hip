@@ -57,26 +57,23 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) {
                                                    0, 0, 0);
 }
 
-__device__ __forceinline__ uint16_t bf16_bits(float v) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
-__device__ __forceinline__ float bf16_value(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// v = hi + lo (+ < 2^-18 |v|): hi = bf16(v), lo = bf16(v - hi)
-__device__ __forceinline__ void split(float v, uint16_t& hi, uint16_t& lo) {
-    hi = bf16_bits(v);
-    lo = bf16_bits(v - bf16_value(hi));
+// a, b -> packed bf16 pairs (a low): v = hi + lo (+ < 2^-18 |v|), hi = bf16(v),
+// lo = bf16(v - hi).  Both conversions round two values in one instruction, whose
+// result is already the packed pair: 3 VALU operations per value.
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+    const float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xFFFF0000u);
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
 }
 
 // 8 f32 -> packed bf16 hi and lo
 __device__ __forceinline__ void split8(const float* v, u32x4& hi, u32x4& lo) {
     uint32_t h[4], l[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        uint16_t h0, l0, h1, l1;
-        split(v[2 * i], h0, l0);
-        split(v[2 * i + 1], h1, l1);
-        h[i] = h0 | static_cast<uint32_t>(h1) << 16;
-        l[i] = l0 | static_cast<uint32_t>(l1) << 16;
-    }
+    for (int i = 0; i < 4; ++i) split2(v[2 * i], v[2 * i + 1], h[i], l[i]);
     hi = u32x4{h[0], h[1], h[2], h[3]};
     lo = u32x4{l[0], l[1], l[2], l[3]};
 }
@@ -97,6 +94,7 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
     constexpr int kVRow = kKT + 8;     // transposed V plane row (bf16), padded
     constexpr int kBlocks = kDP / 32;  // 32-wide d blocks of O^T
     constexpr int kElems = kKT * kDP / (kW * kWave);  // tile elements per thread (K and V each)
+    constexpr bool kMaskEarly = kElems * kDP < 16 * 128;  // not the narrow form at 128
     static_assert(!kVec || kElems % 4 == 0, "whole quads per thread");
     __shared__ __attribute__((aligned(16))) uint16_t ksh[2][kKT * kKRow], ksl[2][kKT * kKRow];
     __shared__ __attribute__((aligned(16))) uint16_t vsh[2][kDP * kVRow], vsl[2][kDP * kVRow];
@@ -126,6 +124,7 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
     const float* mrow =
         mask ? mask + ((mask_batch == 1 ? 0 : static_cast<int64_t>(b)) * S + min(qrow, S - 1)) * static_cast<int64_t>(S)
              : nullptr;
+    const bool mask_quads = (S & 3) == 0 && (reinterpret_cast<uintptr_t>(mask) & 15) == 0;
 
     // tile loads.  Scalar: element e = tid + 256 i -> key e / kDP, d e % kDP
     // (coalesced along d).  kVec: K item e -> key e / (kDP / 4), the quad of d
@@ -144,6 +143,8 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
     const uint32_t koff = static_cast<uint32_t>((tid / (kDP / 4)) * ldk + col + min(dq, D - 4));
     const uint32_t voff = static_cast<uint32_t>(4 * (tid / kDP) * ldv + col + min(dv, D - 1));
     const bool kin = dq < D, vin = dv < D;
+    // The loads leave their registers untouched until the tile is stored: zeroing them
+    // here made every tile wait for its successor's loads before its own MFMAs.
     auto load_tile = [&](int j0) {
         if constexpr (kVec) {
             if (j0 + kKT <= S) {  // a whole tile (uniform): no row clamps
@@ -151,81 +152,72 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
                 for (int i = 0; i < kQuads; ++i) {
                     const float* kb = k + (base + j0 + i * kKeyStepK) * ldk;
                     const float4 kv = *reinterpret_cast<const float4*>(kb + koff);
-                    kreg[4 * i] = kin ? kv.x : 0.f;
-                    kreg[4 * i + 1] = kin ? kv.y : 0.f;
-                    kreg[4 * i + 2] = kin ? kv.z : 0.f;
-                    kreg[4 * i + 3] = kin ? kv.w : 0.f;
+                    kreg[4 * i] = kv.x;
+                    kreg[4 * i + 1] = kv.y;
+                    kreg[4 * i + 2] = kv.z;
+                    kreg[4 * i + 3] = kv.w;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float x = (v + (base + j0 + i * kKeyStepV + r) * ldv)[voff];
-                        vreg[4 * i + r] = vin ? x : 0.f;
-                    }
+                    for (int r = 0; r < 4; ++r) vreg[4 * i + r] = (v + (base + j0 + i * kKeyStepV + r) * ldv)[voff];
                 }
                 return;
             }
 #pragma unroll
             for (int i = 0; i < kQuads; ++i) {
                 const int e = tid + i * kW * kWave;
-                const int key = e / (kDP / 4), d = 4 * (e % (kDP / 4));
-                const bool ok = j0 + key < S && d < D;
+                const int key = e / (kDP / 4), k4 = 4 * (e / kDP);
                 const int64_t row = base + min(j0 + key, S - 1);
-                const float4 kv = *reinterpret_cast<const float4*>(k + row * ldk + col + min(d, D - 4));
-                kreg[4 * i] = ok ? kv.x : 0.f;
-                kreg[4 * i + 1] = ok ? kv.y : 0.f;
-                kreg[4 * i + 2] = ok ? kv.z : 0.f;
-                kreg[4 * i + 3] = ok ? kv.w : 0.f;
-                const int dv = e % kDP, k4 = 4 * (e / kDP);
+                const float4 kv = *reinterpret_cast<const float4*>(k + row * ldk + col + min(dq, D - 4));
+                kreg[4 * i] = kv.x;
+                kreg[4 * i + 1] = kv.y;
+                kreg[4 * i + 2] = kv.z;
+                kreg[4 * i + 3] = kv.w;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const bool okv = j0 + k4 + r < S && dv < D;
-                    const float x = v[(base + min(j0 + k4 + r, S - 1)) * ldv + col + min(dv, D - 1)];
-                    vreg[4 * i + r] = okv ? x : 0.f;
-                }
+                for (int r = 0; r < 4; ++r)
+                    vreg[4 * i + r] = v[(base + min(j0 + k4 + r, S - 1)) * ldv + col + min(dv, D - 1)];
             }
         } else {
 #pragma unroll
             for (int i = 0; i < kElems; ++i) {
                 const int e = tid + i * kW * kWave, key = e / kDP, d = e % kDP;
-                const bool ok = j0 + key < S && d < D;
-                const int64_t row = base + (ok ? j0 + key : 0);
-                kreg[i] = ok ? k[row * ldk + col + d] : 0.f;
-                vreg[i] = ok ? v[row * ldv + col + d] : 0.f;
+                const int64_t row = base + min(j0 + key, S - 1);
+                kreg[i] = k[row * ldk + col + min(d, D - 1)];
+                vreg[i] = v[row * ldv + col + min(d, D - 1)];
             }
         }
     };
-    auto store_tile = [&](int buf) {
+    // the tile of keys j0 .. j0 + 31 into buffer `buf`, zeros past S and past D
+    auto store_tile = [&](int buf, int j0) {
         if constexpr (kVec) {
 #pragma unroll
             for (int i = 0; i < kQuads; ++i) {
                 const int e = tid + i * kW * kWave;
-                const int key = e / (kDP / 4), d = 4 * (e % (kDP / 4));
-                uint16_t h4[4], l4[4];
+                const int key = e / (kDP / 4), k4 = 4 * (e / kDP);
+                const bool ok = kin && j0 + key < S;
+                uint32_t h[2], l[2];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) split(kreg[4 * i + r], h4[r], l4[r]);
-                *reinterpret_cast<uint2*>(&ksh[buf][key * kKRow + d]) =
-                    make_uint2(h4[0] | static_cast<uint32_t>(h4[1]) << 16, h4[2] | static_cast<uint32_t>(h4[3]) << 16);
-                *reinterpret_cast<uint2*>(&ksl[buf][key * kKRow + d]) =
-                    make_uint2(l4[0] | static_cast<uint32_t>(l4[1]) << 16, l4[2] | static_cast<uint32_t>(l4[3]) << 16);
-                const int dv = e % kDP, k4 = 4 * (e / kDP);
+                for (int r = 0; r < 2; ++r)
+                    split2(ok ? kreg[4 * i + 2 * r] : 0.f, ok ? kreg[4 * i + 2 * r + 1] : 0.f, h[r], l[r]);
+                *reinterpret_cast<uint2*>(&ksh[buf][key * kKRow + dq]) = make_uint2(h[0], h[1]);
+                *reinterpret_cast<uint2*>(&ksl[buf][key * kKRow + dq]) = make_uint2(l[0], l[1]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) split(vreg[4 * i + r], h4[r], l4[r]);
+                for (int r = 0; r < 2; ++r)
+                    split2(vin && j0 + k4 + 2 * r < S ? vreg[4 * i + 2 * r] : 0.f,
+                           vin && j0 + k4 + 2 * r + 1 < S ? vreg[4 * i + 2 * r + 1] : 0.f, h[r], l[r]);
                 // keys 4a .. 4a + 3 sit at 4 consecutive columns of the transposed tile
-                *reinterpret_cast<uint2*>(&vsh[buf][dv * kVRow + vcol(k4)]) =
-                    make_uint2(h4[0] | static_cast<uint32_t>(h4[1]) << 16, h4[2] | static_cast<uint32_t>(h4[3]) << 16);
-                *reinterpret_cast<uint2*>(&vsl[buf][dv * kVRow + vcol(k4)]) =
-                    make_uint2(l4[0] | static_cast<uint32_t>(l4[1]) << 16, l4[2] | static_cast<uint32_t>(l4[3]) << 16);
+                *reinterpret_cast<uint2*>(&vsh[buf][dv * kVRow + vcol(k4)]) = make_uint2(h[0], h[1]);
+                *reinterpret_cast<uint2*>(&vsl[buf][dv * kVRow + vcol(k4)]) = make_uint2(l[0], l[1]);
             }
         } else {
 #pragma unroll
             for (int i = 0; i < kElems; ++i) {
                 const int e = tid + i * kW * kWave, key = e / kDP, d = e % kDP;
-                uint16_t hi, lo;
-                split(kreg[i], hi, lo);
-                ksh[buf][key * kKRow + d] = hi;
-                ksl[buf][key * kKRow + d] = lo;
-                split(vreg[i], hi, lo);
-                vsh[buf][d * kVRow + vcol(key)] = hi;
-                vsl[buf][d * kVRow + vcol(key)] = lo;
+                const bool ok = j0 + key < S && d < D;
+                uint32_t hi, lo;
+                split2(ok ? kreg[i] : 0.f, ok ? vreg[i] : 0.f, hi, lo);
+                ksh[buf][key * kKRow + d] = static_cast<uint16_t>(hi);
+                ksl[buf][key * kKRow + d] = static_cast<uint16_t>(lo);
+                vsh[buf][d * kVRow + vcol(key)] = static_cast<uint16_t>(hi >> 16);
+                vsl[buf][d * kVRow + vcol(key)] = static_cast<uint16_t>(lo >> 16);
             }
         }
     };
@@ -236,13 +228,31 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
     float m = -INFINITY, l = 0.f;
 
     load_tile(0);
-    store_tile(0);
+    store_tile(0, 0);
     __syncthreads();
     int buf = 0;
     for (int j0 = 0; j0 < S; j0 += kKT) {
         const bool more = j0 + kKT < S;
         if (more) load_tile(j0 + kKT);  // in flight during this tile
 
+        // the mask's 16 values of this lane: keys 8 a + 4 g .. + 3, as quads where the rows
+        // are 16-byte aligned.  In flight during the first product where the registers
+        // hold them (kMaskEarly).
+        f32x4 mk[4];
+        auto load_mask = [&]() {
+            if (mask_quads && j0 + kKT <= S) {
+                asm volatile("");
+#pragma unroll
+                for (int a = 0; a < 4; ++a) mk[a] = *reinterpret_cast<const f32x4*>(mrow + j0 + 8 * a + 4 * g);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mk[r >> 2][r & 3] = mrow[min(j0 + 8 * (r >> 2) + 4 * g + (r & 3), S - 1)];
+            }
+        };
+        if (kMaskEarly && mask) {
+            asm volatile("");
+            load_mask();
+        }
         // S^T[key][q] = sum_d K[key][d] Q[q][d]: lane holds keys 8(r/4) + 4g + r%4 of query lr
         f32x16 st = f32x16{};
         {
@@ -258,26 +268,38 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
             }
         }
         // scores in log2 units: s * scale * log2(e) (+ mask * log2(e)), so that the
-        // probabilities are one v_exp_f32 (2^x) each
+        // probabilities are one v_exp_f32 (2^x) each.  Without a mask the scale goes
+        // into the exponent's fma, the maximum being taken of the products.
         float p[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) p[r] = st[r];
+        float unit = scale2;
+        // `mask` (a kernel argument) and the tile are uniform: real branches (the empty
+        // statement keeps the compiler from computing both sides)
+        if (mask) {
+            asm volatile("");
+            unit = 1.0f;
+            if (!kMaskEarly) load_mask();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) p[r] = fmaf(mk[r >> 2][r & 3], kLog2e, p[r] * scale2);
+        }
+        if (j0 + kKT > S) {
+            asm volatile("");
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (j0 + 8 * (r >> 2) + 4 * g + (r & 3) >= S) p[r] = -INFINITY;
+        }
         float mt = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int key = j0 + 8 * (r >> 2) + 4 * g + (r & 3);
-            float sc = st[r] * scale2;
-            // `mask` (a kernel argument) is uniform: no divergent branch; the index is clamped
-            if (mask) sc = fmaf(mrow[min(key, S - 1)], kLog2e, sc);
-            sc = key < S ? sc : -INFINITY;
-            p[r] = sc;
-            mt = fmaxf(mt, sc);
-        }
+        for (int r = 0; r < 16; ++r) mt = fmaxf(mt, p[r]);
+        mt *= unit;
         mt = fmaxf(mt, __shfl_xor(mt, 32, kWave));  // the partner lane holds the other 16 keys
         const float mn = fmaxf(m, mt);
         const float base_m = mn == -INFINITY ? 0.f : mn;  // all masked so far: nothing to add
         float ls = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            p[r] = __builtin_amdgcn_exp2f(p[r] - base_m);
+            p[r] = __builtin_amdgcn_exp2f(fmaf(p[r], unit, -base_m));
             ls += p[r];
         }
         ls += __shfl_xor(ls, 32, kWave);
@@ -291,10 +313,13 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
         split8(p + 8, ph[1], pl[1]);
         // O^T[d][q] += sum_key V[key][d] P[q][key]
         // alpha is 1 in every lane once the running maxima settle: the rescale is skipped
-        const bool rescale = __ballot(alpha != 1.0f) != 0;
+        if (__ballot(alpha != 1.0f) != 0) {
+            asm volatile("");  // a real branch
+#pragma unroll
+            for (int c = 0; c < kBlocks; ++c) ot[c] *= alpha;
+        }
 #pragma unroll
         for (int c = 0; c < kBlocks; ++c) {
-            if (rescale) ot[c] *= alpha;
             const uint16_t* vh = &vsh[buf][(32 * c + lr) * kVRow + 8 * g];
             const uint16_t* vl = &vsl[buf][(32 * c + lr) * kVRow + 8 * g];
 #pragma unroll
@@ -307,7 +332,7 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
             }
         }
         if (more) {
-            store_tile(buf ^ 1);  // the other buffer: last read before the previous barrier
+            store_tile(buf ^ 1, j0 + kKT);  // the other buffer: last read before the previous barrier
             __syncthreads();
             buf ^= 1;
         }
