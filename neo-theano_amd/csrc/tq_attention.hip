@@ -25,7 +25,7 @@
 // first product: lane half g holds keys 8a + 4g + b (a, b < 4), and the
 // transposed V tile stores key k at column k with bits 2 and 3 swapped, so the
 // 8 keys of a 16-key MFMA step are one contiguous 16-byte read.  The head
-// dimension is padded with zeros to 32, 64 or 128.  A running max of -inf
+// dimension is padded with zeros to 32, 64, 96 or 128.  A running max of -inf
 // (every key so far masked) leaves the row untouched; a row masked everywhere
 // ends as 0/0 = NaN, as the reference's softmax gives.
 //
@@ -46,6 +46,7 @@ namespace tq {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
 
 constexpr int kWaves = 4;           // waves per block (8 in the wide form)
 constexpr int kQW = 32;              // query rows per wave
@@ -76,6 +77,15 @@ __device__ __forceinline__ void split8(const float* v, u32x4& hi, u32x4& lo) {
     for (int i = 0; i < 4; ++i) split2(v[2 * i], v[2 * i + 1], h[i], l[i]);
     hi = u32x4{h[0], h[1], h[2], h[3]};
     lo = u32x4{l[0], l[1], l[2], l[3]};
+}
+
+// A lane's value and its partner's 32 lanes away, combined (v_permlane32_swap_b32, a
+// vector operation; __shfl_xor is a round trip through LDS).
+template <class Op>
+__device__ __forceinline__ float with_partner(float v, Op op) {
+    const uint32_t u = __float_as_uint(v);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
 __device__ __forceinline__ int vcol(int key) { return (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1); }
@@ -113,18 +123,30 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
 #pragma unroll
         for (int st = 0; st < kSteps; ++st) {
             float qv[8];
+            if constexpr (kVec) {  // whole quads (D % 4 == 0), any alignment
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int d = 16 * st + 8 * g + j;
-                qv[j] = d < D ? qr[d] : 0.f;
+                for (int j = 0; j < 8; j += 4) {
+                    const int d = 16 * st + 8 * g + j;
+                    const f32x4 t = *reinterpret_cast<const f32x4_a4*>(qr + min(d, D - 4));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) qv[j + e] = d < D ? t[e] : 0.f;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int d = 16 * st + 8 * g + j;
+                    qv[j] = qr[min(d, D - 1)];
+                    qv[j] = d < D ? qv[j] : 0.f;
+                }
             }
             split8(qv, qh[st], ql[st]);
+            // (the raw values of two steps in registers at a time)
+            if (st % 2 == 1) __builtin_amdgcn_sched_barrier(0);
         }
     }
     const float* mrow =
         mask ? mask + ((mask_batch == 1 ? 0 : static_cast<int64_t>(b)) * S + min(qrow, S - 1)) * static_cast<int64_t>(S)
              : nullptr;
-    const bool mask_quads = (S & 3) == 0 && (reinterpret_cast<uintptr_t>(mask) & 15) == 0;
 
     // tile loads.  Scalar: element e = tid + 256 i -> key e / kDP, d e % kDP
     // (coalesced along d).  kVec: K item e -> key e / (kDP / 4), the quad of d
@@ -142,6 +164,7 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
     const int dq = 4 * (tid % (kDP / 4)), dv = tid % kDP;
     const uint32_t koff = static_cast<uint32_t>((tid / (kDP / 4)) * ldk + col + min(dq, D - 4));
     const uint32_t voff = static_cast<uint32_t>(4 * (tid / kDP) * ldv + col + min(dv, D - 1));
+    static_assert(!kVec || kW * kWave % kDP == 0, "an item's column does not depend on the item");
     const bool kin = dq < D, vin = dv < D;
     // The loads leave their registers untouched until the tile is stored: zeroing them
     // here made every tile wait for its successor's loads before its own MFMAs.
@@ -161,19 +184,24 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
                 }
                 return;
             }
+            // the last, partial tile: rows clamped, as 32-bit offsets from its first
+            const float* kt = k + (base + j0) * ldk;
+            const float* vt = v + (base + j0) * ldv;
+            const uint32_t lk = static_cast<uint32_t>(ldk), lv = static_cast<uint32_t>(ldv);
 #pragma unroll
             for (int i = 0; i < kQuads; ++i) {
                 const int e = tid + i * kW * kWave;
-                const int key = e / (kDP / 4), k4 = 4 * (e / kDP);
-                const int64_t row = base + min(j0 + key, S - 1);
-                const float4 kv = *reinterpret_cast<const float4*>(k + row * ldk + col + min(dq, D - 4));
+                const uint32_t key = min(e / (kDP / 4), S - 1 - j0);
+                const f32x4 kv = *reinterpret_cast<const f32x4*>(kt + (key * lk + col + min(dq, D - 4)));
                 kreg[4 * i] = kv.x;
                 kreg[4 * i + 1] = kv.y;
                 kreg[4 * i + 2] = kv.z;
                 kreg[4 * i + 3] = kv.w;
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    vreg[4 * i + r] = v[(base + min(j0 + k4 + r, S - 1)) * ldv + col + min(dv, D - 1)];
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t kr = min(4 * (e / kDP) + r, S - 1 - j0);
+                    vreg[4 * i + r] = vt[kr * lv + col + min(dv, D - 1)];
+                }
             }
         } else {
 #pragma unroll
@@ -225,7 +253,7 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
     f32x16 ot[kBlocks];
 #pragma unroll
     for (int c = 0; c < kBlocks; ++c) ot[c] = f32x16{};
-    float m = -INFINITY, l = 0.f;
+    float m = -INFINITY, l = 0.f;  // l: this lane's half of the row's sum
 
     load_tile(0);
     store_tile(0, 0);
@@ -235,15 +263,15 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
         const bool more = j0 + kKT < S;
         if (more) load_tile(j0 + kKT);  // in flight during this tile
 
-        // the mask's 16 values of this lane: keys 8 a + 4 g .. + 3, as quads where the rows
-        // are 16-byte aligned.  In flight during the first product where the registers
-        // hold them (kMaskEarly).
+        // the mask's 16 values of this lane: keys 8 a + 4 g .. + 3, as quads (at 4-byte
+        // alignment: a mask row is S values) in whole tiles.  In flight during the first
+        // product where the registers hold them (kMaskEarly).
         f32x4 mk[4];
         auto load_mask = [&]() {
-            if (mask_quads && j0 + kKT <= S) {
+            if (j0 + kKT <= S) {
                 asm volatile("");
 #pragma unroll
-                for (int a = 0; a < 4; ++a) mk[a] = *reinterpret_cast<const f32x4*>(mrow + j0 + 8 * a + 4 * g);
+                for (int a = 0; a < 4; ++a) mk[a] = *reinterpret_cast<const f32x4_a4*>(mrow + j0 + 8 * a + 4 * g);
             } else {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) mk[r >> 2][r & 3] = mrow[min(j0 + 8 * (r >> 2) + 4 * g + (r & 3), S - 1)];
@@ -293,18 +321,17 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
 #pragma unroll
         for (int r = 0; r < 16; ++r) mt = fmaxf(mt, p[r]);
         mt *= unit;
-        mt = fmaxf(mt, __shfl_xor(mt, 32, kWave));  // the partner lane holds the other 16 keys
+        mt = with_partner(mt, OpMax{});  // the partner lane holds the other 16 keys
         const float mn = fmaxf(m, mt);
         const float base_m = mn == -INFINITY ? 0.f : mn;  // all masked so far: nothing to add
-        float ls = 0.f;
+        float ls[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             p[r] = __builtin_amdgcn_exp2f(fmaf(p[r], unit, -base_m));
-            ls += p[r];
+            ls[r & 3] += p[r];
         }
-        ls += __shfl_xor(ls, 32, kWave);
         const float alpha = __builtin_amdgcn_exp2f(m - base_m);
-        l = l * alpha + ls;
+        l = fmaf(l, alpha, (ls[0] + ls[1]) + (ls[2] + ls[3]));
         m = mn;
         // P^T operand: step t of 16 keys takes registers 8t .. 8t+7 (keys 16t + 8h + 4g + b,
         // slot 4h + b), the order of the transposed V tile's columns
@@ -314,9 +341,17 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
         // O^T[d][q] += sum_key V[key][d] P[q][key]
         // alpha is 1 in every lane once the running maxima settle: the rescale is skipped
         if (__ballot(alpha != 1.0f) != 0) {
-            asm volatile("");  // a real branch
+            // in place: multiplies that the compiler may give other destinations made it
+            // hold the running output twice, with as many copies a tile (the products that
+            // wrote it ended a barrier and this tile's scores ago)
 #pragma unroll
-            for (int c = 0; c < kBlocks; ++c) ot[c] *= alpha;
+            for (int c = 0; c < kBlocks; ++c)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    float t = ot[c][e];
+                    asm volatile("v_mul_f32 %0, %1, %0" : "+v"(t) : "v"(alpha));
+                    ot[c][e] = t;
+                }
         }
 #pragma unroll
         for (int c = 0; c < kBlocks; ++c) {
@@ -337,9 +372,14 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
             buf ^= 1;
         }
     }
+    l = with_partner(l, OpAdd{});
     // lane holds O^T[d = 32c + 8(r/4) + 4g + r%4][q = lr]
-    if (qrow < S) {
-        float* orow = o + (base + qrow) * ldo + col;
+    // (the row formed again from the thread's index: it would hold registers through the loop)
+    int t2 = threadIdx.x;
+    asm volatile("" : "+v"(t2));
+    const int row = blockIdx.x * (kW * kQW) + (t2 >> 6) * kQW + (t2 & 31);
+    if (row < S) {
+        float* orow = o + (base + row) * ldo + col;
         const float inv = 1.0f / l;
 #pragma unroll
         for (int c = 0; c < kBlocks; ++c)
@@ -401,10 +441,13 @@ extern "C" int tq_attention_f32(const float* q, int64_t ldq, const float* k, int
     // (and element offsets within a key tile below 2^31)
     const bool vec = head_dim % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 && aligned(k, 16) && aligned(v, 16) &&
                      kKT * std::max(ldk, ldv) + e < (int64_t(1) << 31);
-    // head dim 128: 8-wave blocks where they still give every CU a block (measured
-    // at S = 2048, H = 32: 310-315 against 343 us eager)
-    const int64_t wide_blocks = (seq + 8 * kQW - 1) / (8 * kQW) * heads * batch;
-    const int waves = vec && head_dim > 64 && wide_blocks >= device_cu_count() ? 8 : kWaves;
+    // Waves per block (32 queries each).  Head dims past 64: 8 (6 at up to 96, where a
+    // thread's tile items then share a column), each key tile split once for all of them
+    // (S = 2048, 32 heads of 128: 237 us against 267 with 4), unless half as many already
+    // give at most one block per CU.
+    const int most = head_dim > 96 ? 8 : 6;
+    const int64_t half_blocks = (seq + most / 2 * kQW - 1) / (most / 2 * kQW) * heads * batch;
+    const int waves = !vec || head_dim <= 64 ? kWaves : half_blocks > device_cu_count() ? most : most / 2;
     const dim3 grid(static_cast<unsigned>((seq + waves * kQW - 1) / (waves * kQW)), static_cast<unsigned>(heads),
                     static_cast<unsigned>(batch));
 #define TQ_ATT(KERNEL, ...)                                                                                     \
@@ -414,6 +457,8 @@ extern "C" int tq_attention_f32(const float* q, int64_t ldq, const float* k, int
         if (vec) TQ_ATT(k_attention_vec, 32, kWaves); else TQ_ATT(k_attention, 32);
     } else if (head_dim <= 64) {
         if (vec) TQ_ATT(k_attention_vec, 64, kWaves); else TQ_ATT(k_attention, 64);
+    } else if (vec && head_dim <= 96) {
+        if (waves == 6) TQ_ATT(k_attention_vec, 96, 6); else TQ_ATT(k_attention_vec, 96, 3);
     } else if (vec) {
         if (waves == 8) TQ_ATT(k_attention_vec, 128, 8); else TQ_ATT(k_attention_vec, 128, kWaves);
     } else {

@@ -237,3 +237,33 @@ def test_mha_quantized_activations_stagewise(tq, oracle, mode):
     qo, so = quant(ws[3])
     assert_close(y, lin(qa, sa, qo, so, bs[3]), RTOL, ATOL, "out_proj")
     assert torch.isfinite(torch.from_numpy(y)).all()
+
+
+@pytest.mark.parametrize("B,S,H,D", [(1, 70, 2, 80), (2, 193, 3, 96), (1, 97, 3, 68), (1, 192, 180, 96), (1, 33, 260, 72),
+                                     (1, 257, 129, 100), (2, 31, 5, 124)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_core_block_shapes(tq, B, S, H, D, masked):
+    """Head dims past 64 in 3- and 6-wave (up to 96) and 4- and 8-wave blocks, partial
+    query blocks and key tiles, mask rows that are not 16-byte aligned, a row masked
+    everywhere: against float64."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(S * D)
+    qkv = torch.randn(B * S, 3 * H * D, generator=g, device="cuda")
+    mask = None
+    if masked:
+        mask = torch.randn(1, S, S, generator=g, device="cuda")
+        mask[0, torch.rand(S, S, generator=g, device="cuda") < 0.5] = float("-inf")
+        mask[0, 3] = float("-inf")
+    got = run_core(tq, host(qkv), B, S, H, None if mask is None else host(mask)).reshape(B, S, H, D)
+    q, k, v = (t.reshape(B, S, H, D).double() for t in qkv.split(H * D, 1))
+    for h in range(0, H, max(1, H // 5)):
+        for b in range(B):
+            s = (q[b, :, h].contiguous() @ k[b, :, h].t().contiguous()) / D ** 0.5
+            if mask is not None:
+                s = s + mask[0].double()
+            ref = host(torch.softmax(s, -1) @ v[b, :, h].contiguous())
+            out = got[b, :, h]
+            assert np.array_equal(np.isnan(out), np.isnan(ref))
+            ok = ~np.isnan(ref)
+            assert_close(out[ok], ref[ok], RTOL, ATOL, f"head {h}")
