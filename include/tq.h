@@ -326,8 +326,7 @@ int tq_linear_fp8(const float* x, int64_t m, const uint8_t* qw, const float* sw,
 
 /* Prefill-shaped W4A16: x bf16 [M, K], INT4 g128 weights, f32 accumulation with
  * the group scale applied to each 128-long partial sum; y f32 [M, N].
- * K % 128 == 0 (the format), any M, N.  The MFMA kernel serves N % 16 == 0 with
- * 16-byte aligned x, packed, y and bias; other cases take a shape-general kernel. */
+ * K % 128 == 0 (the format), any M, N, element-aligned pointers. */
 int tq_gemm_w4g128_bf16(const uint16_t* x_bf16, int64_t m, const uint8_t* packed,
                         const uint16_t* s_f16, const float* bias, int64_t n, int64_t k,
                         float* y, tq_stream_t stream);
@@ -347,6 +346,15 @@ int tq_gemm_w4g128_bf16_ws(const uint16_t* x_bf16, int64_t m, const uint8_t* pac
                            void* workspace, int64_t workspace_bytes, float* y,
                            tq_stream_t stream);
 
+/* The Linear on the pipelined kernels or the register-staged tiles (K split over
+ * blocks where they leave compute units idle), whichever suits the sizes.
+ * `workspace`: at least tq_linear_w4g128_workspace_bytes(M, N, K) bytes (may be 0),
+ * 256-byte aligned. */
+int64_t tq_linear_w4g128_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int tq_linear_w4g128(const uint16_t* x_bf16, int64_t m, const uint8_t* packed, const uint16_t* s_f16,
+                     const float* bias, int64_t n, int64_t k, void* workspace, int64_t workspace_bytes,
+                     float* y, tq_stream_t stream);
+
 /* Quantized Llama-style FFN (build-defined composition of Linear, SiLU
  * (crates/theano-nn/src/activation.rs:66-79) and Tensor::mul):
  *   h = SiLU(x Wg^T) * (x Wu^T);   y = h Wd^T   (f32 [M, D]).
@@ -354,9 +362,12 @@ int tq_gemm_w4g128_bf16_ws(const uint16_t* x_bf16, int64_t m, const uint8_t* pac
  * D % 128 == 0, F % 128 == 0.  `workspace` is device memory of at least
  * tq_mlp_w4g128_workspace_bytes(M, D, F) bytes (intermediates: x in the
  * kernels' k-order, h as bf16 hi + lo planes, group sums; or h as f32 [M, F]
- * on the shape-general path), 16-byte aligned; the pipelined kernels run when
+ * on the register-staged tiles), 16-byte aligned; the pipelined kernels run when
  * D % 256 == 0, F % 256 == 0, the workspace is 256-byte aligned and the
- * scales 4-byte aligned.  x, packed weights and y 16-byte aligned. */
+ * scales 4-byte aligned.  With tq_mlp_w4g128_split_workspace_bytes(M, D, F) bytes
+ * (256-byte aligned) the tiles also split K over blocks, and run wherever they are
+ * ahead.  x, packed weights and y 16-byte aligned. */
+int64_t tq_mlp_w4g128_split_workspace_bytes(int64_t m, int64_t d, int64_t f);
 int64_t tq_mlp_w4g128_workspace_bytes(int64_t m, int64_t d, int64_t f);
 int tq_mlp_w4g128(const uint16_t* x_bf16, int64_t m, int64_t d, int64_t f,
                   const uint8_t* gate_packed, const uint16_t* gate_s,

@@ -40,6 +40,8 @@
 // stage, after which the next stage's operands are read while the last MFMAs
 // of the stage run.  MFMA: v_mfma_f32_32x32x16_bf16, A = activations (m), B =
 // unpacked weights (n), so each lane's 16 outputs share one n (one scale).
+#include <algorithm>
+
 #include "tq_internal.h"
 
 namespace tq {
@@ -497,6 +499,69 @@ FfnWorkspace ffn_workspace(int64_t m, int64_t d, int64_t f) {
     return w;
 }
 
+// Wide or narrow tiles per launch, whichever leaves less work on the busiest CU.
+struct FfnTiles {
+    bool gu_narrow, dn_narrow;
+    int64_t gu_cost, dn_cost;  // launch_cost of the chosen ones
+};
+FfnTiles ffn_tiles(int64_t m, int64_t d, int64_t f) {
+    static_assert(GuCfg::BN == GuSCfg::BN && DnCfg::BM == DnSCfg::BM, "the tile sets share these sides");
+    const int64_t gu_tm = (m + GuCfg::BM - 1) / GuCfg::BM, gus_tm = (m + GuSCfg::BM - 1) / GuSCfg::BM;
+    const int64_t gu_tn = f / GuCfg::BN, dn_tm = (m + DnCfg::BM - 1) / DnCfg::BM;
+    const int64_t gn = launch_cost(gus_tm * gu_tn, GuSCfg::BM, GuSCfg::BN, d / 128, kNarrowGuCost);
+    const int64_t gw = launch_cost(gu_tm * gu_tn, GuCfg::BM, GuCfg::BN, d / 128, kWideCost);
+    const int64_t nn = launch_cost(dn_tm * (d / DnSCfg::BN) * kDnSplit, DnSCfg::BM, DnSCfg::BN, f / 256, kNarrowDnCost);
+    const int64_t nw = launch_cost(dn_tm * (d / DnCfg::BN) * kDnSplit, DnCfg::BM, DnCfg::BN, f / 256, kWideCost);
+    return FfnTiles{gn < gw, nn < nw, std::min(gn, gw), std::min(nn, nw)};
+}
+
+// Linear: K halves are added into y when the doubled grid still fits one round on the
+// CUs and each half keeps at least 8 groups (two addends onto zero: the sum does not
+// depend on their order).  Wide or narrow tiles, whichever leaves less work on the
+// busiest CU (wide ones need N % 256).
+struct LinTiles {
+    bool narrow, split;
+    int64_t tiles_m, tiles_n, cost;
+};
+LinTiles lin_tiles(int64_t m, int64_t n, int64_t k) {
+    auto plan = [&](int64_t bm, int64_t bn, int64_t per_unit) {
+        LinTiles t{};
+        t.tiles_m = (m + bm - 1) / bm;
+        t.tiles_n = n / bn;
+        t.split = 2 * t.tiles_m * t.tiles_n <= device_cu_count() && k / 128 >= 16;
+        t.cost = launch_cost(t.tiles_m * t.tiles_n * (t.split ? 2 : 1), bm, bn, k / 128 / (t.split ? 2 : 1), per_unit);
+        return t;
+    };
+    LinTiles narrow = plan(LinSCfg::BM, LinSCfg::BN, kNarrowLinCost);
+    narrow.narrow = true;
+    const LinTiles wide = plan(LinCfg::BM, LinCfg::BN, kWideCost);
+    return n % LinCfg::BN != 0 || narrow.cost < wide.cost ? narrow : wide;
+}
+
+// ns of a wide tile's (16384 outputs') group: gate/up 2.0 us, down 2.1 us, Linear (32768
+// outputs) 2.2 us at M = 512, D = K = 4096, F = N = 14336
+constexpr int64_t kUnit16384 = 16384 * kWideCost;
+constexpr int64_t kGuUnitNs = 2000, kDnUnitNs = 2100, kLinUnitNs = 1100;
+
+// Whether the pipelined kernels run an FFN of these sizes: they take D and F in
+// multiples of 256, and stay ahead of the register-staged tiles where their own tiles
+// fill the chip (M = 435, D = 256, F = 9728, whose down projection is 14 blocks: 60 us
+// on them, 44 on the tiles; M = 64, D = 8192, F = 1024: 84 and 35 us).
+bool ffn_pipelined(int64_t m, int64_t d, int64_t f) {
+    if (d % 256 != 0 || f % 256 != 0) return false;
+    const FfnTiles t = ffn_tiles(m, d, f);
+    const int64_t ns = 12000 + (t.gu_cost / 1000 * kGuUnitNs + t.dn_cost / 1000 * kDnUnitNs) / (kUnit16384 / 1000);
+    return ns <= mlp_tile_cost(m, d, f).ns;
+}
+
+// The same for the Linear (N % 128, K % 256).
+bool lin_pipelined(int64_t m, int64_t n, int64_t k) {
+    if (k == 0 || k % 256 != 0 || n % LinSCfg::BN != 0) return false;
+    const W4TileCost tile = w4_linear_tile_cost(m, n, k);
+    if (tile.ns == 0) return false;
+    return 9000 + lin_tiles(m, n, k).cost / 1000 * kLinUnitNs / (kUnit16384 / 1000) <= tile.ns;
+}
+
 }  // namespace
 }  // namespace tq
 
@@ -506,9 +571,13 @@ extern "C" {
 
 int64_t tq_mlp_w4g128_workspace_bytes(int64_t m, int64_t d, int64_t f) {
     if (m <= 0 || d <= 0 || f <= 0) return 0;
-    // the shape-general path keeps h as f32 [M, F] in the same buffer
-    const int64_t fast = ffn_workspace(m, d, f).bytes, general = m * f * 4;
-    return fast > general ? fast : general;
+    // the unsplit tiles keep h as f32 [M, F] in the same buffer
+    return std::max(ffn_workspace(m, d, f).bytes, m * f * 4);
+}
+
+int64_t tq_mlp_w4g128_split_workspace_bytes(int64_t m, int64_t d, int64_t f) {
+    const int64_t least = tq_mlp_w4g128_workspace_bytes(m, d, f);
+    return least == 0 || ffn_pipelined(m, d, f) ? least : std::max(least, mlp_tile_cost(m, d, f).bytes);
 }
 
 int tq_mlp_w4g128(const uint16_t* x_bf16, int64_t m, int64_t d, int64_t f, const uint8_t* gate_packed,
@@ -534,9 +603,11 @@ int tq_mlp_w4g128(const uint16_t* x_bf16, int64_t m, int64_t d, int64_t f, const
     // 4-byte aligned scales) and tile the output columns by 128 (gate/up) and 256 (down)
     const bool fast = d % 256 == 0 && f % 256 == 0 && aligned(gate_s, 4) && aligned(up_s, 4) && aligned(down_s, 4) &&
                       aligned(workspace, 256);
-    if (!fast)
-        return launch_mlp_w4g128_general(x_bf16, m, d, f, gate_packed, gate_s, up_packed, up_s, down_packed, down_s,
-                                         static_cast<float*>(workspace), y, st);
+    const bool may_split =
+        aligned(workspace, 256) && workspace_bytes >= tq_mlp_w4g128_split_workspace_bytes(m, d, f);
+    if (!fast || (may_split && !ffn_pipelined(m, d, f)))
+        return launch_mlp_tile(x_bf16, m, d, f, gate_packed, gate_s, up_packed, up_s, down_packed, down_s, workspace,
+                               may_split && !ffn_pipelined(m, d, f), y, st);
 
     const FfnWorkspace w = ffn_workspace(m, d, f);
     uint8_t* base = static_cast<uint8_t*>(workspace);
@@ -548,16 +619,11 @@ int tq_mlp_w4g128(const uint16_t* x_bf16, int64_t m, int64_t d, int64_t f, const
 
     const int64_t items = m * (d / 128);
     TQ_REQUIRE((items + 15) / 16 < (int64_t(1) << 31), "tq_mlp_w4g128: problem too large");
-    // wide or narrow tiles per launch, whichever leaves less work on the busiest CU
-    static_assert(GuCfg::BN == GuSCfg::BN && DnCfg::BM == DnSCfg::BM, "the tile sets share these sides");
-    const int64_t gu_tm = (m + GuCfg::BM - 1) / GuCfg::BM, gus_tm = (m + GuSCfg::BM - 1) / GuSCfg::BM;
+    const FfnTiles t = ffn_tiles(m, d, f);
+    const bool gu_narrow = t.gu_narrow, dn_narrow = t.dn_narrow;
     const int64_t gu_tn = f / GuCfg::BN, dn_tm = (m + DnCfg::BM - 1) / DnCfg::BM;
-    const bool gu_narrow = launch_cost(gus_tm * gu_tn, GuSCfg::BM, GuSCfg::BN, d / 128, kNarrowGuCost) <
-                           launch_cost(gu_tm * gu_tn, GuCfg::BM, GuCfg::BN, d / 128, kWideCost);
-    const bool dn_narrow =
-        launch_cost(dn_tm * (d / DnSCfg::BN) * kDnSplit, DnSCfg::BM, DnSCfg::BN, f / 256, kNarrowDnCost) <
-        launch_cost(dn_tm * (d / DnCfg::BN) * kDnSplit, DnCfg::BM, DnCfg::BN, f / 256, kWideCost);
-    const int64_t gu_tiles_m = gu_narrow ? gus_tm : gu_tm, gu_tiles = gu_tiles_m * gu_tn;
+    const int64_t gu_tiles_m = (m + (gu_narrow ? GuSCfg::BM : GuCfg::BM) - 1) / (gu_narrow ? GuSCfg::BM : GuCfg::BM);
+    const int64_t gu_tiles = gu_tiles_m * gu_tn;
     const int64_t dn_tiles_n = d / (dn_narrow ? DnSCfg::BN : DnCfg::BN), dn_tiles = dn_tm * dn_tiles_n * kDnSplit;
     TQ_REQUIRE(gu_tiles < (int64_t(1) << 31) && dn_tiles < (int64_t(1) << 31), "tq_mlp_w4g128: problem too large");
 
@@ -637,26 +703,9 @@ int tq_gemm_w4g128_bf16_ws(const uint16_t* x_bf16, int64_t m, const uint8_t* pac
     const int64_t mpad = (m + 127) / 128 * 128;
     uint16_t* xp = static_cast<uint16_t*>(workspace);
     uint32_t* xs = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(workspace) + align256(m * k * 2));
-    // K halves are added into y when the doubled grid still fits one round on the CUs
-    // and each half keeps at least 8 groups (two addends onto zero: the sum does not
-    // depend on their order).  Wide or narrow tiles, whichever leaves less work on
-    // the busiest CU (wide ones need N % 256).
-    auto plan = [&](int64_t bm, int64_t bn, int64_t per_unit, int64_t* tm, int64_t* tn, bool* split) {
-        *tm = (m + bm - 1) / bm;
-        *tn = n / bn;
-        *split = 2 * *tm * *tn <= device_cu_count() && k / 128 >= 16;
-        return launch_cost(*tm * *tn * (*split ? 2 : 1), bm, bn, k / 128 / (*split ? 2 : 1), per_unit);
-    };
-    int64_t tiles_m, tiles_n, wtm, wtn;
-    bool split, wsplit;
-    const int64_t narrow_cost = plan(LinSCfg::BM, LinSCfg::BN, kNarrowLinCost, &tiles_m, &tiles_n, &split);
-    const bool narrow =
-        n % LinCfg::BN != 0 || narrow_cost < plan(LinCfg::BM, LinCfg::BN, kWideCost, &wtm, &wtn, &wsplit);
-    if (!narrow) {
-        tiles_m = wtm;
-        tiles_n = wtn;
-        split = wsplit;
-    }
+    const LinTiles t = lin_tiles(m, n, k);
+    const bool narrow = t.narrow, split = t.split;
+    const int64_t tiles_m = t.tiles_m, tiles_n = t.tiles_n;
     const int64_t items = m * (k / 128);
     TQ_REQUIRE((items + 15) / 16 < (int64_t(1) << 31) && tiles_m * tiles_n * 2 < (int64_t(1) << 31),
                "tq_gemm_w4g128_bf16_ws: problem too large");
@@ -687,6 +736,31 @@ int tq_gemm_w4g128_bf16_ws(const uint16_t* x_bf16, int64_t m, const uint8_t* pac
     else
         k_ffn<kLnWM, kLnWN, kLnTM, kLnTN, 1, 1, 1><<<blocks, LinCfg::kThreads, 0, st>>>(a);
     return check_launch("tq_gemm_w4g128_bf16_ws");
+}
+
+// The Linear on whichever of the two suits its sizes.
+int64_t tq_linear_w4g128_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    return lin_pipelined(m, n, k) ? tq_gemm_w4g128_bf16_workspace_bytes(m, k) : w4_linear_tile_cost(m, n, k).bytes;
+}
+
+int tq_linear_w4g128(const uint16_t* x_bf16, int64_t m, const uint8_t* packed, const uint16_t* s_f16,
+                     const float* bias, int64_t n, int64_t k, void* workspace, int64_t workspace_bytes, float* y,
+                     tq_stream_t stream) {
+    TQ_REQUIRE(m >= 0 && n >= 0 && k >= 0, "tq_linear_w4g128: negative shape");
+    TQ_REQUIRE(k % 128 == 0, "tq_linear_w4g128: K=%lld is not a multiple of 128", (long long)k);
+    if (m == 0 || n == 0) return TQ_OK;
+    const int64_t need = tq_linear_w4g128_workspace_bytes(m, n, k);
+    TQ_REQUIRE(need == 0 || (workspace && aligned(workspace, 256) && workspace_bytes >= need),
+               "tq_linear_w4g128: workspace of %lld bytes (256-byte aligned), %lld needed", (long long)workspace_bytes,
+               (long long)need);
+    if (lin_pipelined(m, n, k))
+        return tq_gemm_w4g128_bf16_ws(x_bf16, m, packed, s_f16, bias, n, k, workspace, workspace_bytes, y, stream);
+    TQ_REQUIRE(y && (k == 0 || (x_bf16 && packed && s_f16)), "tq_linear_w4g128: null pointer");
+    TQ_REQUIRE(aligned(x_bf16, 2) && aligned(s_f16, 2) && aligned(y, 4) && (!bias || aligned(bias, 4)),
+               "tq_linear_w4g128: misaligned pointer");
+    return launch_w4_linear_tile(x_bf16, m, packed, s_f16, bias, n, k, need ? workspace : nullptr, y, as_hip(stream),
+                                 "tq_linear_w4g128");
 }
 
 }  // extern "C"

@@ -17,7 +17,12 @@
 //    bits, by truncation) and every code is exact in bf16, so each product is
 //    exact and only the f32 sums round.
 //
-// The bf16 forms add their running sums into a second set of accumulators every
+//  * GemmW4, GemmW4GateUp, GemmW4H: INT4 g128 codes widened to bf16 (exact) against bf16
+//    activations (GemmW4H: f32 activations as bf16 hi + lo); every 128-long group's sum
+//    is scaled by its f16 scale as it is added to the total.  GemmW4GateUp runs two
+//    weight matrices side by side and stores h = SiLU(gate) * up.
+//
+// The 8-bit bf16 forms add their running sums into a second set of accumulators every
 // kFlushStages stages (in f64 for GemmF8b), so that a sum's rounding grows with
 // the square root of a run's length and not of K: relative errors at K = 14336 are
 // 1.2e-7 (GemmF8W) and 4.7e-8 (GemmF8b), against 2.8e-7 and 7.2e-8 for a wave's f32
@@ -43,6 +48,15 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // Vectors at the alignment of their elements.
 typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
 typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef uint32_t u32_a1 __attribute__((aligned(1)));
+
+typedef __bf16 tile_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float tile_f32x2 __attribute__((ext_vector_type(2)));
+// a and b rounded to bf16, packed (a low)
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((tile_f32x2{a, b}), tile_bf16x2));
+}
 
 // high halves of a and b as one dword (a low)
 __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
@@ -58,7 +72,7 @@ __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
 // below 2^-133, bf16's last place, are dropped: only values under 2^-109 have any.)
 struct SrcF32 {
     typedef float elem_t;
-    static constexpr int kElems = 8, kPlanes = 3;
+    static constexpr int kElems = 8, kPlanes = 3, kPer = 1;
     struct Raw {
         f32x4 a, b;
     };
@@ -143,7 +157,7 @@ struct ValFp8 {
 template <class Val>
 struct SrcBf16 {
     typedef typename Val::code_t elem_t;
-    static constexpr int kElems = 8, kPlanes = 1;
+    static constexpr int kElems = 8, kPlanes = 1, kPer = 1;
     struct Raw {
         u32x2 v;
     };
@@ -164,7 +178,7 @@ struct SrcBf16 {
 template <class T>
 struct SrcBytes {
     typedef T elem_t;
-    static constexpr int kElems = 16, kPlanes = 1;
+    static constexpr int kElems = 16, kPlanes = 1, kPer = 1;
     struct Raw {
         u32x4 v;
     };
@@ -175,12 +189,65 @@ struct SrcBytes {
     __device__ static void planes(const Raw& r, u32x4 (&out)[1]) { out[0] = r.v; }
 };
 
+// f32 -> bf16 hi and lo (round to nearest: hi + lo keeps 2^-18 of the value); an
+// infinity is its own hi.
+struct SrcF32HiLo {
+    typedef float elem_t;
+    static constexpr int kElems = 8, kPlanes = 2, kPer = 1;
+    typedef SrcF32::Raw Raw;
+    __device__ static Raw load(const elem_t* p) { return SrcF32::load(p); }
+    __device__ static Raw load_tail(const elem_t* p, int n, int k) { return SrcF32::load_tail(p, n, k); }
+    __device__ static void planes(const Raw& r, u32x4 (&out)[2]) {
+        const float v[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float a = v[2 * i], b = v[2 * i + 1];
+            h[i] = bf16_pair(a, b);
+            const float ha = __uint_as_float(h[i] << 16), hb = __uint_as_float(h[i] & 0xFFFF0000u);
+            l[i] = bf16_pair(a == ha ? 0.0f : a - ha, b == hb ? 0.0f : b - hb);
+        }
+        out[0] = u32x4{h[0], h[1], h[2], h[3]};
+        out[1] = u32x4{l[0], l[1], l[2], l[3]};
+    }
+};
+
+// bf16 activations as they are.
+struct SrcBf16Raw {
+    typedef uint16_t elem_t;
+    static constexpr int kElems = 8, kPlanes = 1, kPer = 1;
+    struct Raw {
+        u32x4 v;
+    };
+    __device__ static Raw load(const elem_t* p) { return Raw{*reinterpret_cast<const u32x4_a2*>(p)}; }
+    __device__ static Raw load_tail(const elem_t* p, int, int) { return load(p); }  // K % 128 == 0: no tails
+    __device__ static void planes(const Raw& r, u32x4 (&out)[1]) { out[0] = r.v; }
+};
+
+// 8 nibbles (low first) -> bf16 of code / 16, exact (v_cvt_off_f32_i4; the 16 goes into
+// the group scale).
+struct SrcW4 {
+    typedef uint8_t elem_t;
+    static constexpr int kElems = 8, kPlanes = 1, kPer = 2;
+    struct Raw {
+        uint32_t v;
+    };
+    __device__ static Raw load(const elem_t* p) { return Raw{*reinterpret_cast<const u32_a1*>(p)}; }
+    __device__ static Raw load_tail(const elem_t* p, int, int) { return load(p); }
+    __device__ static void planes(const Raw& r, u32x4 (&out)[1]) {
+        uint32_t f[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = f32_bits(__builtin_amdgcn_cvt_off_f32_i4(static_cast<int>(r.v >> (4 * i))));
+        out[0] = u32x4{pack_hi(f[0], f[1]), pack_hi(f[2], f[3]), pack_hi(f[4], f[5]), pack_hi(f[6], f[7])};
+    }
+};
+
 // ---- operand traits ----
 // kFragChunks 16-byte chunks per lane and MFMA; an MFMA step covers twice that
 // many chunks of a row (one share per lane half).
 struct OpBf16 {
     typedef f32x16 Acc;
-    static constexpr bool kFlush = true, kDigits = false;
+    static constexpr bool kFlush = true, kDigits = false, kGroups = false, kGateUp = false;
     static constexpr int kFragChunks = 1;
     typedef u32x4 Frag;
     __device__ static Frag frag(const u32x4 (&c)[1]) { return c[0]; }
@@ -203,12 +270,25 @@ struct GemmF8b : OpBf16 {
     static constexpr bool kRowScale = true;
     static constexpr int kFlushStages = 4;
 };
+struct GemmW4 : OpBf16 {
+    typedef SrcBf16Raw A;
+    typedef SrcW4 W;
+    typedef float part_t;
+    static constexpr bool kRowScale = false, kGroups = true;
+    static constexpr int kFlushStages = 2;  // one group
+};
+struct GemmW4GateUp : GemmW4 {
+    static constexpr bool kGateUp = true;
+};
+struct GemmW4H : GemmW4 {
+    typedef SrcF32HiLo A;
+};
 struct GemmI8 {
     typedef SrcBytes<int8_t> A;
     typedef SrcBytes<int8_t> W;
     typedef i32x16 Acc;
     typedef int32_t part_t;
-    static constexpr bool kRowScale = true, kFlush = false, kDigits = false;
+    static constexpr bool kRowScale = true, kFlush = false, kDigits = false, kGroups = false, kGateUp = false;
     static constexpr int kFragChunks = 1;
     typedef i32x4 Frag;
     __device__ static Frag frag(const u32x4 (&c)[1]) { return __builtin_bit_cast(i32x4, c[0]); }
@@ -226,7 +306,7 @@ struct GemmF8 {
     typedef SrcBytes<uint8_t> W;
     typedef f32x16 Acc;
     typedef float part_t;
-    static constexpr bool kRowScale = true, kFlush = false, kDigits = false;
+    static constexpr bool kRowScale = true, kFlush = false, kDigits = false, kGroups = false, kGateUp = false;
     static constexpr int kFragChunks = 2;
     typedef i32x8 Frag;
     __device__ static Frag frag(const u32x4 (&c)[2]) {
@@ -248,12 +328,18 @@ struct TileArgs {
     const float* x;     // the f32 activations [m, k] (kDigits, rows that are not finite)
     const float* sw;    // column scales [n]
     const float* bias;  // [n] or null
+    const uint16_t* sg;   // f16 group scales [n, k / 128] (kGroups)
+    const void* w2;       // kGateUp: w and sg are gate's, w2 and sg2 up's, n both rows' count
+    const uint16_t* sg2;  // (n = 2 F: partial sums hold gate's F columns, then up's)
     int m, n, k, lda;   // m counts outputs' rows
     int tiles_m, tiles_n, split;
     int32_t* acc;  // int32 sums [m, n] or null (GemmI8)
     float* y;      // [m, n]
     void* part;    // split > 1: partial sums [split][m][n]
 };
+
+// SiLU(g) * u, as the FFN kernels form it
+__device__ __forceinline__ float silu_mul(float g, float u) { return g * (1.0f / (1.0f + __expf(-g))) * u; }
 
 // y[mm, nn] from its sum
 template <class T>
@@ -262,6 +348,8 @@ __device__ __forceinline__ void tile_store(const TileArgs& p, typename T::part_t
     if constexpr (T::kDigits) {
         p.y[o] = digit_out(v, p.ea[mm], sw, b, p.x + static_cast<int64_t>(mm) * p.k,
                            static_cast<const int8_t*>(p.w) + static_cast<int64_t>(nn) * p.k, p.k);
+    } else if constexpr (T::kGroups) {
+        p.y[o] = v + b;
     } else if constexpr (T::kRowScale) {
         if constexpr (__is_same(typename T::part_t, int32_t))
             if (p.acc) p.acc[o] = v;
@@ -309,10 +397,12 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
     const int L = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3);
     const int tm = L % p.tiles_m, tn = (L / p.tiles_m) % p.tiles_n, ks = L / (p.tiles_m * p.tiles_n);
     const int m0 = tm * BM, n0 = tn * BN;
-    const int rows_a = T::kDigits ? 4 * p.m : p.m;
+    const int rows_a = T::kDigits ? 4 * p.m : p.m, rows_w = T::kGateUp ? p.n / 2 : p.n;
+    static_assert(!T::kGateUp || TN == 2, "a wave holds 32 gate and the same 32 up columns");
     const int stages = (p.k + BK - 1) / BK;
-    const int s_begin = static_cast<int>(static_cast<int64_t>(ks) * stages / p.split);
-    const int s_end = static_cast<int>(static_cast<int64_t>(ks + 1) * stages / p.split);
+    constexpr int kUnit = T::kGroups ? 2 : 1;  // whole groups per split (two stages each)
+    const int s_begin = static_cast<int>(static_cast<int64_t>(ks) * (stages / kUnit) / p.split) * kUnit;
+    const int s_end = static_cast<int>(static_cast<int64_t>(ks + 1) * (stages / kUnit) / p.split) * kUnit;
 
     // item i: row (tid + 256 i) / 8, chunk tid % 8
     const int chunk = tid & 7;
@@ -328,7 +418,15 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
 #pragma unroll
     for (int i = 0; i < kWItems; ++i) {
         const int r = (tid >> 3) + 32 * i;
-        wsrc[i] = static_cast<const typename SW::elem_t*>(p.w) + static_cast<int64_t>(min(n0 + r, p.n - 1)) * p.k;
+        const void* w = p.w;
+        int row = n0 + r;
+        if constexpr (T::kGateUp) {
+            // tile row 64 t + i: gate row i of the block's t-th 32, i < 32, then up's
+            row = n0 / 2 + 32 * (r >> 6) + (r & 31);
+            w = r & 32 ? p.w2 : p.w;
+        }
+        wsrc[i] = static_cast<const typename SW::elem_t*>(w) +
+                  static_cast<int64_t>(min(row, rows_w - 1)) * (p.k / SW::kPer);
         wdst[i] = PA * BM * kTileRow + r * kTileRow + ((chunk ^ tile_swz(r)) << 4);
     }
     // two register sets: stage s of a split goes through set (s - s_begin) & 1
@@ -348,7 +446,18 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
         *reinterpret_cast<u32x4*>(st + wdst[i]) = c[0];
     };
     auto load_a = [&](Regs& r, int i, int s) { r.a[i] = SA::load(asrc[i] + s * BK + chunk * SA::kElems); };
-    auto load_w = [&](Regs& r, int i, int s) { r.w[i] = SW::load(wsrc[i] + s * BK + chunk * SW::kElems); };
+    auto load_w = [&](Regs& r, int i, int s) { r.w[i] = SW::load(wsrc[i] + (s * BK + chunk * SW::kElems) / SW::kPer); };
+    // output column of the lane in its j-th tile (kGateUp: of gate and of up alike)
+    auto column = [&](int j) { return T::kGateUp ? n0 / 2 + wn * 32 + l32 : n0 + (wn * TN + j) * 32 + l32; };
+    // the f16 scales of group g of the lane's columns
+    uint16_t sc[TN];
+    auto load_scales = [&](int g) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const uint16_t* sg = T::kGateUp && j == 1 ? p.sg2 : p.sg;
+            sc[j] = sg[static_cast<int64_t>(min(column(j), rows_w - 1)) * (p.k / 128) + g];
+        }
+    };
     // fragment of row r (of a plane at `base`) for step `step`
     auto frag = [&](const int8_t* base, int r, int step) -> typename T::Frag {
         u32x4 c[T::kFragChunks];
@@ -425,8 +534,14 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     if constexpr (kSets == 2) acc[0][i][j] += acc[1][i][j];
+                    if constexpr (T::kGroups) {
+                        const float sj = 16.0f * __half2float(__ushort_as_half(sc[j]));
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) tot[i][j][e] += acc[0][i][j][e];
+                        for (int e = 0; e < 16; ++e) tot[i][j][e] = fmaf(acc[0][i][j][e], sj, tot[i][j][e]);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) tot[i][j][e] += acc[0][i][j][e];
+                    }
 #pragma unroll
                     for (int h = 0; h < kSets; ++h) acc[h][i][j] = typename T::Acc{};
                 }
@@ -461,6 +576,7 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         int s = s_begin;
         for (; s + 1 < s_full; s += 2) {
+            if constexpr (T::kGroups) load_scales(s / kUnit);
             stage(lds, lds + kStage, rg[1], min(s + 3, s_last));
             stage(lds + kStage, lds, rg[0], min(s + 4, s_last));
             if constexpr (T::kFlush)
@@ -477,14 +593,14 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
         }
 #pragma unroll
         for (int i = 0; i < kWItems; ++i) {
-            rg[0].w[i] = SW::load_tail(wsrc[i] + k0, p.k - k0, p.k);
+            rg[0].w[i] = SW::load_tail(wsrc[i] + k0 / SW::kPer, p.k - k0, p.k);
             store_w(rg[0], i, lds);
         }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
         for (int step = 0; step < kSteps; ++step) step_mfma(lds, step);
     }
-    flush();
+    if constexpr (!T::kGroups) flush();
 
     auto sum = [&](int i, int j, int e) {
         if constexpr (T::kFlush)
@@ -496,11 +612,30 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
     // store covers 32 consecutive n of two rows; with digit rows, e % 4 is the
     // digit and a lane holds whole sums of 4 rows
     constexpr int kPer = T::kDigits ? 4 : 1;
+    if constexpr (T::kGateUp) {
+        const int nn = column(0), f = rows_w;
+        if (nn >= f) return;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int mm = m0 + (wm * TM + i) * 32 + 8 * (e >> 2) + 4 * lh + (e & 3);
+                if (mm >= p.m) continue;
+                if (p.split == 1) {
+                    p.y[static_cast<int64_t>(mm) * f + nn] = silu_mul(sum(i, 0, e), sum(i, TN - 1, e));
+                } else {
+                    float* o = static_cast<float*>(p.part) + (static_cast<int64_t>(ks) * p.m + mm) * p.n + nn;
+                    o[0] = sum(i, 0, e);
+                    o[f] = sum(i, TN - 1, e);
+                }
+            }
+        return;
+    }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-        const int nn = n0 + (wn * TN + j) * 32 + l32;
+        const int nn = column(j);
         const bool nval = nn < p.n;
-        const float sw = p.split == 1 && nval ? p.sw[nn] : 0.0f;
+        const float sw = !T::kGroups && p.split == 1 && nval ? p.sw[nn] : 0.0f;
         const float bv = p.split == 1 && nval && p.bias ? p.bias[nn] : 0.0f;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -527,12 +662,19 @@ template <class T>
 __global__ __launch_bounds__(256) void k_gemm_tile_finish(TileArgs p) {
     const int64_t mn = static_cast<int64_t>(p.m) * p.n;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= mn) return;
-    const typename T::part_t* part = static_cast<const typename T::part_t*>(p.part) + i;
+    const int cols = T::kGateUp ? p.n / 2 : p.n;
+    if (i >= static_cast<int64_t>(p.m) * cols) return;
+    const int mm = static_cast<int>(i / cols), nn = static_cast<int>(i - static_cast<int64_t>(mm) * cols);
+    const typename T::part_t* part = static_cast<const typename T::part_t*>(p.part) + static_cast<int64_t>(mm) * p.n + nn;
     typename T::part_t v = part[0];
     for (int s = 1; s < p.split; ++s) v += part[s * mn];
-    const int mm = static_cast<int>(i / p.n), nn = static_cast<int>(i - static_cast<int64_t>(mm) * p.n);
-    tile_store<T>(p, v, mm, nn, p.sw[nn], p.bias ? p.bias[nn] : 0.0f);
+    if constexpr (T::kGateUp) {
+        float u = part[cols];
+        for (int s = 1; s < p.split; ++s) u += part[s * mn + cols];
+        p.y[i] = silu_mul(v, u);
+    } else {
+        tile_store<T>(p, v, mm, nn, T::kGroups ? 0.0f : p.sw[nn], p.bias ? p.bias[nn] : 0.0f);
+    }
 }
 
 // ------------------------------------------------------------------ host side
@@ -565,11 +707,24 @@ struct TileCosts<GemmF8W> {
     static constexpr TileShape shape[kTileShapes] = {{128, 128, 2100, 2400}, {64, 64, 840, 690}, {32, 128, 780, 600}, {64, 128, 1150, 960}};
 };
 
+template <>
+struct TileCosts<GemmW4> {
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 900, 800}, {64, 64, 400, 300}, {32, 128, 640, 325}, {64, 128, 680, 490}};
+};
+template <>
+struct TileCosts<GemmW4GateUp> {
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 820, 780}, {64, 64, 0, 0}, {32, 128, 0, 0}, {64, 128, 650, 525}};
+};
+template <>
+struct TileCosts<GemmW4H> {
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 1500, 1900}, {64, 64, 720, 570}, {32, 128, 810, 475}, {64, 128, 1000, 815}};
+};
+
 constexpr int kTileDma = -1;  // the LDS-DMA kernels' 128 x 256 tiles
 
 struct TilePlan {
     int shape, split, tiles_m, tiles_n;
-    int64_t part_bytes;
+    int64_t part_bytes, ns;
 };
 
 // The shape and K split with the smallest estimate: rounds of blocks over the CUs
@@ -581,7 +736,7 @@ template <class T>
 TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int dma_stage, bool may_split) {
     const int64_t cus = device_cu_count(), rows = T::kDigits ? 4 * m : m;
     const int64_t stages = (k + 8 * T::A::kElems - 1) / (8 * T::A::kElems);
-    TilePlan best{kTile64x64, 1, 0, 0, 0};
+    TilePlan best{kTile64x128, 1, 0, 0, 0, 0};
     int64_t best_ns = INT64_MAX;
     if (dma_stage > 0) {
         const int64_t blocks = ((rows + 127) / 128) * ((n + 255) / 256);
@@ -589,6 +744,7 @@ TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int dma_stage, bool may_spli
         best_ns = (blocks + cus - 1) / cus * (k / 128) * dma_stage + 4000;
     }
     for (int c = 0; c < kTileShapes; ++c) {
+        if (T::kGateUp && (c == kTile64x64 || c == kTile32x128)) continue;  // two column tiles per wave
         const TileShape& t = TileCosts<T>::shape[c];
         const int64_t tm = (rows + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
         for (int split : {1, 2, 3, 4, 6, 8, 12, 16}) {
@@ -600,7 +756,7 @@ TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int dma_stage, bool may_spli
             if (split > 1) ns += 3000 + 2 * part / 4000;
             if (ns < best_ns) {
                 best_ns = ns;
-                best = TilePlan{c, split, 0, 0, split > 1 ? part : 0};
+                best = TilePlan{c, split, 0, 0, split > 1 ? part : 0, ns};
             }
         }
     }
@@ -627,14 +783,19 @@ int launch_tile(const TilePlan& plan, TileArgs p, hipStream_t st, const char* wh
     const unsigned grid = static_cast<unsigned>(static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.split);
     switch (plan.shape) {
     case kTile128x128: k_gemm_tile<T, 128, 128, 2, 2, 1><<<grid, 256, 0, st>>>(p); break;
-    case kTile64x64: k_gemm_tile<T, 64, 64, 2, 2, 2><<<grid, 256, 0, st>>>(p); break;
-    case kTile32x128: k_gemm_tile<T, 32, 128, 1, 4, 2><<<grid, 256, 0, st>>>(p); break;
-    default: k_gemm_tile<T, 64, 128, 2, 2, 2><<<grid, 256, 0, st>>>(p); break;
+    case kTile64x128: k_gemm_tile<T, 64, 128, 2, 2, 2><<<grid, 256, 0, st>>>(p); break;
+    default:
+        if constexpr (!T::kGateUp) {
+            if (plan.shape == kTile64x64)
+                k_gemm_tile<T, 64, 64, 2, 2, 2><<<grid, 256, 0, st>>>(p);
+            else
+                k_gemm_tile<T, 32, 128, 1, 4, 2><<<grid, 256, 0, st>>>(p);
+        }
     }
     if (p.split > 1) {
         const int rc = check_launch(what);
         if (rc != TQ_OK) return rc;
-        const int64_t blocks = (static_cast<int64_t>(p.m) * p.n + 255) / 256;
+        const int64_t blocks = (static_cast<int64_t>(p.m) * (T::kGateUp ? p.n / 2 : p.n) + 255) / 256;
         k_gemm_tile_finish<T><<<static_cast<unsigned>(blocks), 256, 0, st>>>(p);
     }
     return check_launch(what);

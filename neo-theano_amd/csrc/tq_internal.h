@@ -58,13 +58,21 @@ int launch_gemm_w8a8_generic(const int8_t* qa, const float* sa, const int8_t* qw
 int launch_gemm_fp8_generic(const uint8_t* qa, const float* sa, const uint8_t* qw, const float* sw,
                             const float* bias, int64_t m, int64_t n, int64_t k, float* y, hipStream_t st);
 
-// FFN block for shapes the pipelined kernels of tq_ffn.hip do not take (D or F
-// not a multiple of 256, 2-byte aligned scales): 16x16x32 MFMA kernels of
-// tq_mlp.hip with h kept as f32 [M, F] in `h`.
-int launch_mlp_w4g128_general(const uint16_t* x_bf16, int64_t m, int64_t d, int64_t f, const uint8_t* gate_packed,
-                              const uint16_t* gate_s, const uint8_t* up_packed, const uint16_t* up_s,
-                              const uint8_t* down_packed, const uint16_t* down_s, float* h, float* y,
-                              hipStream_t st);
+// INT4 g128 Linear and FFN on the register-staged tiles (tq_mlp.hip), any M and N,
+// element-aligned pointers: the estimated time (0 for sizes that the shape-general
+// kernel takes) and the workspace with K split over blocks; `part` null or
+// `may_split` false runs unsplit (the FFN then needs only h, 4 M F bytes).
+struct W4TileCost {
+    int64_t ns, bytes;
+};
+W4TileCost w4_linear_tile_cost(int64_t m, int64_t n, int64_t k);
+int launch_w4_linear_tile(const uint16_t* x_bf16, int64_t m, const uint8_t* packed, const uint16_t* s_f16,
+                          const float* bias, int64_t n, int64_t k, void* part, float* y, hipStream_t st,
+                          const char* what);
+W4TileCost mlp_tile_cost(int64_t m, int64_t d, int64_t f);
+int launch_mlp_tile(const uint16_t* x_bf16, int64_t m, int64_t d, int64_t f, const uint8_t* gate_packed,
+                    const uint16_t* gate_s, const uint8_t* up_packed, const uint16_t* up_s, const uint8_t* down_packed,
+                    const uint16_t* down_s, void* workspace, bool may_split, float* y, hipStream_t st);
 
 #define TQ_REQUIRE(cond, ...)                                 \
     do {                                                      \

@@ -67,6 +67,8 @@ SIGNATURES = {
     "tq_gemm_w8a8_ws": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p, _i64, _p, _p],
     "tq_gemm_fp8_workspace_bytes": [_i64, _i64, _i64],
     "tq_gemm_fp8_ws": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _i64, _p, _p],
+    "tq_linear_w4g128_workspace_bytes": [_i64, _i64, _i64],
+    "tq_linear_w4g128": [_p, _i64, _p, _p, _p, _i64, _i64, _p, _i64, _p, _p],
     "tq_linear_w8a8_workspace_bytes": [_i64, _i64, _i64],
     "tq_linear_w8a8": [_p, _i64, _p, _p, _p, _i64, _i64, _p, _i64, _p, _p],
     "tq_linear_fp8_workspace_bytes": [_i64, _i64, _i64],
@@ -78,6 +80,7 @@ SIGNATURES = {
     "tq_gemm_w4g128_bf16_workspace_bytes": [_i64, _i64],
     "tq_gemm_w4g128_bf16_ws": [_p, _i64, _p, _p, _p, _i64, _i64, _p, _i64, _p, _p],
     "tq_mlp_w4g128_workspace_bytes": [_i64, _i64, _i64],
+    "tq_mlp_w4g128_split_workspace_bytes": [_i64, _i64, _i64],
     "tq_mlp_w4g128": [_p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _p],
     "tq_mlp_w4g128_decode_workspace_bytes": [_i64, _i64, _i64],
     "tq_repack_w4g128_gate_up_tiled": [_p, _p, _p, _p, _i64, _i64, _p, _p, _p],
@@ -88,6 +91,8 @@ _RESTYPE = {"tq_status_string": ctypes.c_char_p, "tq_last_error": ctypes.c_char_
             "tq_w4g128_tile_rows": ctypes.c_int64, "tq_mlp_w4g128_workspace_bytes": ctypes.c_int64,
             "tq_mlp_w4g128_decode_workspace_bytes": ctypes.c_int64,
             "tq_gemm_w8_workspace_bytes": ctypes.c_int64, "tq_gemm_fp8_weight_workspace_bytes": ctypes.c_int64,
+            "tq_linear_w4g128_workspace_bytes": ctypes.c_int64,
+            "tq_mlp_w4g128_split_workspace_bytes": ctypes.c_int64,
             "tq_linear_w8a8_workspace_bytes": ctypes.c_int64, "tq_linear_fp8_workspace_bytes": ctypes.c_int64,
             "tq_gemm_w8a8_workspace_bytes": ctypes.c_int64, "tq_gemm_fp8_workspace_bytes": ctypes.c_int64,
             "tq_gemm_w4g128_bf16_workspace_bytes": ctypes.c_int64, "tq_dtype_size": ctypes.c_int64}

@@ -174,11 +174,7 @@ class QuantizedLinear(Module):
                 _abi.call("tq_gemv_w4g128", x.data_ptr(), m, self.qweight.data_ptr(), self.scales.data_ptr(), bias, n, k,
                           y.data_ptr(), st)
             else:
-                # prefill: pipelined kernels with x's k-order and group sums in a workspace
-                nb = _abi.entry("tq_gemm_w4g128_bf16_workspace_bytes")(m, k)
-                ws = x.new_empty(max(nb, 1), dtype=torch.uint8)
-                _abi.call("tq_gemm_w4g128_bf16_ws", x.data_ptr(), m, self.qweight.data_ptr(), self.scales.data_ptr(),
-                          bias, n, k, ws.data_ptr(), nb, y.data_ptr(), st)
+                self._run("tq_linear_w4g128", x, m, y, st)
         elif mode == "w8":
             self._run("tq_gemm_w8", x, m, y, st)
         elif mode in ("w8a8", "fp8") and m <= FUSED_A8_MAX_M and _fused_a8_ok(x, self.qweight, k):
@@ -243,7 +239,8 @@ class QuantizedMLP(Module):
         return m <= 8 or (m <= DECODE_MLP_MAX_M and self.d <= DECODE_MLP_ONE_PASS_D)
 
     def workspace_bytes(self, m: int) -> int:
-        """Device bytes of intermediates forward() needs for m tokens."""
+        """Device bytes of intermediates that forward() needs for m tokens (given a
+        workspace; without one it may allocate more, see tq_mlp_w4g128)."""
         if self._decode_path(m):
             mm = min(m, DECODE_MLP_PASS_M)  # one pass at a time
             return _abi.entry("tq_mlp_w4g128_decode_workspace_bytes")(mm, self.d, self.f)
@@ -257,7 +254,10 @@ class QuantizedMLP(Module):
             raise InvalidArgument(f"QuantizedMLP.forward: expected [M, {self.d}], got {tuple(x.shape)}")
         m, d, f, st = x.shape[0], self.d, self.f, stream()
         if workspace is None:
-            workspace = x.new_empty(max(self.workspace_bytes(m), 1), dtype=torch.uint8)
+            # of its own, prefill takes what its kernels can use for splitting K
+            nb = (self.workspace_bytes(m) if self._decode_path(m)
+                  else _abi.entry("tq_mlp_w4g128_split_workspace_bytes")(m, d, f))
+            workspace = x.new_empty(max(nb, 1), dtype=torch.uint8)
         y = x.new_empty((m, d), dtype=torch.float32)
         ws, wsb = workspace.data_ptr(), workspace.numel() * workspace.element_size()
         if self._decode_path(m):

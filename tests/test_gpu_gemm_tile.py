@@ -23,9 +23,10 @@ def _codes(torch, shape, seed, fp8):
 
 def _at_offset(torch, t, off):
     """`t`'s bytes at an address `off` past a 16-byte boundary."""
-    buf = torch.empty(t.numel() + 64, dtype=torch.uint8, device="cuda")
-    v = buf[off:off + t.numel()]
-    v.copy_(t.view(torch.uint8).reshape(-1))
+    b = t.view(torch.uint8).reshape(-1)
+    buf = torch.empty(b.numel() + 64, dtype=torch.uint8, device="cuda")
+    v = buf[off:off + b.numel()]
+    v.copy_(b)
     return buf, v
 
 
@@ -234,3 +235,63 @@ def test_workspace_too_small_is_refused(tq):
         _abi.call("tq_gemm_w8a8_ws", ptr(t), ptr(f), ptr(torch.zeros(n * k, dtype=torch.int8, device="cuda")), ptr(f),
                   None, m, n, k, None, ptr(f), nb - 1, ptr(f), stream())
     assert np.isfinite(f.cpu().numpy()).all()
+
+
+def _w4(torch, tq, rows, k, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    q, s = tq.quantize_i4_g128(torch.randn(rows, k, generator=g, device="cuda") * 0.02)
+    return q, s, tq.dequantize_i4_g128(q, s).double()
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 1000, 128), (40, 130, 14336), (65, 129, 4096), (100, 515, 384), (389, 5827, 256),
+                                   (64, 4096, 2048), (300, 33, 1024), (129, 128, 8192), (35, 20, 256)])
+def test_w4_linear_tiles(tq, m, n, k):
+    """The INT4 Linear's tiles at edges of M and N, odd and even group counts, K split
+    over blocks; packed bytes, scales and x at their elements' alignment."""
+    import torch
+
+    from theano_quantize import _abi
+    from theano_quantize._tensor import ptr, stream
+
+    q, s, w = _w4(torch, tq, n, k, 21)
+    g = torch.Generator(device="cuda").manual_seed(22)
+    x = torch.empty(m * k + 1, dtype=torch.bfloat16, device="cuda")[1:].view(m, k)
+    x.copy_(torch.randn(m, k, generator=g, device="cuda"))
+    b = torch.randn(n, generator=g, device="cuda")
+    kq, vq = _at_offset(torch, q, 3)
+    ks, vs = _at_offset(torch, s, 2)
+    ref = x.double() @ w.t().contiguous() + b.double()
+    mag = x.double().abs() @ w.abs().t().contiguous() + b.double().abs()
+    nb = int(_abi.lib().tq_linear_w4g128_workspace_bytes(m, n, k))
+    ws = torch.empty(max(nb, 8), dtype=torch.uint8, device="cuda").fill_(0xA5)
+    for name, extra in (("tq_linear_w4g128", [ptr(ws), nb]), ("tq_gemm_w4g128_bf16", [])):
+        y = torch.full((m, n), float("nan"), device="cuda")
+        _abi.call(name, ptr(x), m, ptr(vq), ptr(vs), ptr(b), n, k, *extra, ptr(y), stream())
+        # eight MFMA additions of 16 exact products per group, each within 2^-23 of the largest
+        # partial sum, then one per group; the pipelined kernels' offset form (K % 256, N % 128)
+        # adds 24 times the activations' sum and takes it away again
+        off = 24.0 if nb and k % 256 == 0 and n % 128 == 0 else 1.0
+        bound = 2.0 ** -23 * off * (8 + k / 128) ** 0.5 * mag + 2.0 ** -22 * ref.abs()
+        assert bool(((y.double() - ref).abs() <= bound).all()), name
+
+
+@pytest.mark.parametrize("m,d,f", [(33, 128, 128), (48, 640, 1408), (100, 384, 128), (65, 128, 3200), (200, 1152, 384),
+                                   (300, 256, 2432), (64, 2048, 256), (130, 4096, 384)])
+def test_w4_mlp_tiles(tq, m, d, f):
+    """The FFN's tiles, with their own workspace (K split) and with the least one."""
+    import torch
+
+    (g, gs, gw), (u, us, uw), (dn, ds, dw) = (_w4(torch, tq, r, c, 30 + i)
+                                              for i, (r, c) in enumerate([(f, d), (f, d), (d, f)]))
+    mlp = tq.QuantizedMLP(d, f, (g, gs), (u, us), (dn, ds), tiled=False)
+    gen = torch.Generator(device="cuda").manual_seed(d + f)
+    x = torch.randn(m, d, generator=gen, device="cuda").to(torch.bfloat16)
+    a = x.double() @ gw.t().contiguous()
+    h = a / (1 + torch.exp(-a)) * (x.double() @ uw.t().contiguous())
+    ref = h @ dw.t().contiguous()
+    least = torch.empty(mlp.workspace_bytes(m), dtype=torch.uint8, device="cuda").fill_(0xA5)
+    for ws in (None, least):
+        y = mlp.forward(x, ws).double()
+        rel = ((y - ref).norm() / ref.norm()).item()
+        assert rel < 2e-5, rel  # h is handed over as bf16 hi + lo, 2^-17 of each
+        assert bool(((y - ref).abs() <= 1e-4 + 1e-3 * ref.abs()).all())
