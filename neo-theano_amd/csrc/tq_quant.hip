@@ -160,23 +160,66 @@ __global__ __launch_bounds__(64 * kW) void k_quant_rows_split(const float* __res
     }
 }
 
-// ---- per-row quantize, any K / alignment: two passes over the row ----
-template <class Fmt>
-__global__ __launch_bounds__(kBlock) void k_quant_rows_generic(const float* __restrict__ w, int64_t k,
-                                                               typename Fmt::code_t* __restrict__ q,
-                                                               float* __restrict__ s, float* __restrict__ w_hat) {
-    __shared__ float red[kWavesPerBlock];
-    const int64_t row = blockIdx.x;
+// ---- per-row quantize, any K / alignment ----
+// One block of kThreads per row; thread t holds f32x4 items t + kThreads i of it (loads
+// at 4-byte alignment) and stores their codes as words at byte alignment; the last K % 4
+// values go one by one.  Rows past 4 kItems kThreads values are read a second time for
+// the rest.  256 threads per row, 1024 where a launch has few rows and the latency of a
+// long row is all there is.  719 x 8999 takes 7.7 us, 1153 x 15927 17.3 and 14336 x 4097
+// 64, against 23.2, 47.9 and 114 us for 256 threads that read every value twice, one at
+// a time; 6 x 8235 3.5 (11.5), 35 x 5432 3.5 (8.3), 16 x 20000 4.7 (25.2).
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+typedef uint32_t u32_a1 __attribute__((aligned(1)));
+
+template <class Fmt, int kItems, int kThreads>
+__global__ __launch_bounds__(kThreads) void k_quant_rows_any(const float* __restrict__ w, int64_t k,
+                                                             typename Fmt::code_t* __restrict__ q,
+                                                             float* __restrict__ s, float* __restrict__ w_hat) {
+    __shared__ float red[kThreads / kWave];
+    const int64_t row = blockIdx.x, k4 = k >> 2;
     const float* src = w + row * k;
+    const int tid = threadIdx.x, rest = static_cast<int>(k & 3);
+    auto fold = [](float m, f32x4 v) {
+        return fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    };
+    auto load = [&](int64_t j) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(src + 4 * j)); };
+    f32x4 v[kItems];
     float m = -INFINITY;
-    for (int64_t i = threadIdx.x; i < k; i += kBlock) m = fmaxf(m, fabsf(src[i]));
-    const float sc = row_scale<Fmt>(absmax_finish(block_max(m, red)));
-    if (threadIdx.x == 0) s[row] = sc;
+    // every load is issued: threads past the row re-read its last item, which leaves the
+    // maximum unchanged
+    if (k4 > 0) {
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) v[i] = load(min<int64_t>(tid + kThreads * i, k4 - 1));
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) m = fold(m, v[i]);
+        for (int64_t j = tid + kThreads * kItems; j < k4; j += kThreads) m = fold(m, load(j));
+    }
+    const float last = tid < rest ? src[4 * k4 + tid] : 0.0f;
+    if (tid < rest) m = fmaxf(m, fabsf(last));
+    m = wave_max(m);
+    if ((tid & (kWave - 1)) == 0) red[tid / kWave] = m;
+    __syncthreads();
+    m = red[0];
+#pragma unroll
+    for (int i = 1; i < kThreads / kWave; ++i) m = fmaxf(m, red[i]);
+    const float sc = row_scale<Fmt>(absmax_finish(m));
+    if (tid == 0) s[row] = sc;
     const typename Fmt::Row coder(sc);
-    for (int64_t i = threadIdx.x; i < k; i += kBlock) {
-        const typename Fmt::code_t c = coder.code1(src[i]);
-        if (q) q[row * k + i] = c;
-        if (w_hat) w_hat[row * k + i] = Fmt::value1(c, sc);
+    typename Fmt::code_t* qd = q + row * k;
+    float* wd = w_hat ? w_hat + row * k : nullptr;
+    auto store = [&](int64_t j, f32x4 x) {
+        const uint32_t c = coder.code4(x);
+        __builtin_nontemporal_store(c, reinterpret_cast<u32_a1*>(qd + 4 * j));
+        if (wd) __builtin_nontemporal_store(Fmt::value4(c, sc), reinterpret_cast<f32x4_a4*>(wd + 4 * j));
+    };
+#pragma unroll
+    for (int i = 0; i < kItems; ++i)
+        if (tid + kThreads * i < k4) store(tid + kThreads * i, v[i]);
+    for (int64_t j = tid + kThreads * kItems; j < k4; j += kThreads) store(j, load(j));
+    if (tid < rest) {
+        const typename Fmt::code_t c = coder.code1(last);
+        qd[4 * k4 + tid] = c;
+        if (wd) wd[4 * k4 + tid] = Fmt::value1(c, sc);
     }
 }
 
@@ -532,6 +575,12 @@ int launch_quant_rows(const float* w, int64_t rows, int64_t k, typename Fmt::cod
             k_quant_rows_split<Fmt, 8 / kSplitW, kSplitW><<<grid, 64 * kSplitW, 0, st>>>(w, k, q, s, w_hat);
         else
             k_quant_rows_split<Fmt, 16 / kSplitW, kSplitW><<<grid, 64 * kSplitW, 0, st>>>(w, k, q, s, w_hat);
+    } else if (k > 4096 && rows <= (k <= 8192 ? cus : 2 * cus)) {
+        // few long rows, one block each: 16 waves a row instead of 4 (64 x 14336: 3.8
+        // against 6.1 us, 64 x 8192 3.5 against 4.8, 512 x 14336 6.9 against 10.2;
+        // 300 x 5120 is ahead with 4, 4.4 against 4.6)
+        if (k <= 8192) k_quant_rows_any<Fmt, 2, 1024><<<grid, 1024, 0, st>>>(w, k, q, s, w_hat);
+        else k_quant_rows_any<Fmt, 4, 1024><<<grid, 1024, 0, st>>>(w, k, q, s, w_hat);
     } else if (vec && !w_hat && k > 1024 && k <= 4096 && rows <= 8 * cus) {
         // codes only, other K of 1-4 K elements, at most 8 rows per CU: a wave per
         // row.  Past that the persistent blocks below stay ahead (4096 x 4096: 17.3
@@ -555,7 +604,9 @@ int launch_quant_rows(const float* w, int64_t rows, int64_t k, typename Fmt::cod
         else if (items <= 8) k_quant_rows_vec<Fmt, 8><<<pgrid, block, 0, st>>>(w, rows, k, q, s, w_hat);
         else k_quant_rows_vec<Fmt, 16><<<pgrid, block, 0, st>>>(w, rows, k, q, s, w_hat);
     } else {
-        k_quant_rows_generic<Fmt><<<grid, block, 0, st>>>(w, k, q, s, w_hat);
+        if (k <= 1024) k_quant_rows_any<Fmt, 1, kBlock><<<grid, block, 0, st>>>(w, k, q, s, w_hat);
+        else if (k <= 4096) k_quant_rows_any<Fmt, 4, kBlock><<<grid, block, 0, st>>>(w, k, q, s, w_hat);
+        else k_quant_rows_any<Fmt, 16, kBlock><<<grid, block, 0, st>>>(w, k, q, s, w_hat);
     }
     return check_launch(what);
 }

@@ -114,6 +114,40 @@ def test_quantize_rowwise_codes_only_wave_rows(tq, oracle, rows, k):
     assert ieee_equal(host(s8), rs8) and np.array_equal(host(q8), rq8)
 
 
+@pytest.mark.parametrize("rows,k", [(256, 4100), (257, 4100), (3, 8191), (2, 8193), (512, 8196), (513, 8195),
+                                    (2, 16387), (1100, 1021), (600, 4099), (2, 3), (515, 16389)])
+def test_quantize_rowwise_long_and_odd_rows(tq, oracle, rows, k):
+    """Block widths and row lengths on both sides of every rule of the row kernel:
+    codes, scales and w_hat bit-equal to the oracle, rows with a NaN, an infinity, all
+    zeros and exact ties included; the outputs past the last row stay as they were."""
+    import torch
+
+    from theano_quantize import _abi
+
+    w = weights(23, (rows, k), std=1.0)
+    w[0, k - 1] = np.nan
+    w[rows - 1, k // 2] = np.inf
+    if rows > 2:
+        w[1] = 0.0
+        w[2] = tie_row(k) if k > 254 else w[2]
+    rq, rs = oracle.quantize_i8_rowwise(w)
+    fq, fs = oracle.quantize_fp8_rowwise(w)
+    wd, st = dev_tensor(w), torch.cuda.current_stream().cuda_stream
+    for fmt, cq, cs in (("i8", rq, rs), ("fp8", fq, fs)):
+        q = torch.full((rows * k + 64,), 77, dtype=torch.uint8, device="cuda")
+        s = torch.full((rows + 1,), 5.0, device="cuda")
+        _abi.call(f"tq_quantize_{fmt}_rowwise", wd.data_ptr(), rows, k, q.data_ptr(), s.data_ptr(), st)
+        codes = host(q)
+        assert np.array_equal(codes[: rows * k].view(cq.dtype).reshape(rows, k), cq)
+        assert np.all(codes[rows * k :] == 77) and host(s)[rows] == 5.0
+        assert ieee_equal(host(s)[:rows], cs)
+    out = torch.full((rows * k + 16,), 5.0, device="cuda")
+    _abi.call("tq_fake_quantize_i8_rowwise", wd.data_ptr(), rows, k, q.data_ptr(), s.data_ptr(), out.data_ptr(), st)
+    assert ieee_equal(host(out)[: rows * k].reshape(rows, k), oracle.dequantize_i8_rowwise(rq, rs))
+    assert np.all(host(out)[rows * k :] == 5.0)
+    assert np.array_equal(host(q)[: rows * k].view(np.int8).reshape(rows, k), rq)
+
+
 def test_unaligned_and_offset_views(tq, oracle):
     import torch
 
