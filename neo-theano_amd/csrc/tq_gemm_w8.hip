@@ -28,7 +28,11 @@ namespace {
 // weights is short (N = K = 4096: 11.5-13.5 us against 13; N = 14336, K = 4096: 29-34
 // against 20; N = 4096, K = 4097, 24-33 against 15).  The FP8 form's matrix kernel
 // takes longer: the GEMV's aligned form keeps all of its 5 to 8 tokens.
+// Long rows of many outputs go over from 2 INT8 tokens on, at x's traffic (N = 14336, K =
+// 8960: 36 / 45 / 53 us at 2 / 3 / 4 tokens against 33; N = 4096, K = 16384: 16 / 19 / 21
+// against 24).
 bool gemv_runs(int64_t m, int64_t n, int64_t k, bool fp8) {
+    if (!fp8 && m > 1 && k > 8192 && n * k > 96 << 20) return false;
     if (m <= 4 || m > 8) return m <= 4;
     const bool vec16 = k % 16 == 0 && k <= 8192;
     return vec16 ? fp8 || n * k <= 4096 * 4096 : n * k <= 2 << 20;

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(64 * kWB, 8 / kWB) void k_gemv_w8(const float* __re
 // 15; the lane K ends in reads the row's last 16 codes instead, with zeros for the x
 // values that its neighbour owns, and lanes past K the same with all zeros (a NaN code
 // there is one of the row's own, and makes its row NaN either way).  At N = 4096, K =
-// 14336: 13.0 us at one token, 25 at four, against 92 and 159 us for a wave per
+// 14336: 13.0 us at one token, 20.9 at four, against 92 and 159 us for a wave per
 // output (tq_generic.hip); at K = 4097 7.9 against 28.5 us.
 typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
 typedef i32x4 i32x4_a1 __attribute__((aligned(1)));
@@ -652,8 +652,12 @@ template <class Code, int kM, int kC, int kKS>
 void launch_long(const float* x, int64_t xs, const typename Code::code_t* q, const float* s, const float* b, int64_t n,
                  int64_t k, float* y, int64_t ys, int tokens, hipStream_t st) {
     constexpr int kRows = kC == 1 ? 4 : 2, kRuns = kLongWaves / kKS;
-    // about two blocks per CU, runs of whole load groups
-    const int64_t slots = static_cast<int64_t>(device_cu_count()) * 2 * kRuns;
+    // Runs of whole load groups on about two blocks per CU; rows past 8192 on one: every
+    // block reads all of x from L2, at four tokens of K = 14336 half as much again as a
+    // block's share of the weights (N = 4096, K = 14336: 25.1 -> 20.9 us at 4 tokens, 18.0
+    // -> 14.5 at 2; N = 1024 13.1 -> 9.5; shorter rows stay ahead on two, N = 4096, K =
+    // 5000 12.5 against 13.1 us).
+    const int64_t slots = static_cast<int64_t>(device_cu_count()) * (kC == 1 ? 2 : 1) * kRuns;
     int64_t rows = (n + slots - 1) / slots;
     rows = std::min<int64_t>((rows + kRows - 1) / kRows * kRows, kLongRun);
     const int64_t runs = (n + rows - 1) / rows;

@@ -192,6 +192,23 @@ def test_gemv_any_row_length(tq, m, n, k, fp8):
         assert bool(((out.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 1031, 8195), (4, 513, 14336), (3, 1025, 16384), (2, 11183, 9001),
+                                   (2, 11184, 9001)])
+def test_w8_long_rows(tq, m, n, k):
+    """Runs of several rows per block of the long-row GEMV, and both sides of the product
+    (96 Mi weights) from which the matrix cores take them."""
+    import torch
+
+    x = torch.randn(m, k, generator=torch.Generator(device="cuda").manual_seed(m + k), device="cuda")
+    qw = _codes(torch, (n, k), 12, False)
+    y, sw, b = _weight_only(torch, False, x, qw, m, n, k, True, 1)
+    ref = x.double() @ qw.double().t().contiguous() * sw.double() + b.double()
+    mag = (x.double().abs() @ qw.double().abs().t().contiguous()) * sw.double() + b.double().abs()
+    # as test_gemv_any_row_length; the digits' sums stay far inside it
+    bound = 2.0 ** -24 * (k / 64 + 16) ** 0.5 * mag + 2.0 ** -22 * ref.abs()
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("n,k", [(48, 384), (33, 130), (1033, 130), (512, 2048)])
 def test_weight_only_rows_that_are_not_finite(tq, fp8, n, k):
