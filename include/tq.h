@@ -216,11 +216,10 @@ int tq_gemv_fp8(const float* x, int64_t m, const uint8_t* q, const float* s,
                 const float* bias, int64_t n, int64_t k, float* y, tq_stream_t stream);
 
 /* The two weight-only Linears above at any M: the GEMV for a few tokens (up to 4
- * to 8), the matrix cores beyond.  INT8: each row of x becomes a 31-bit fixed-point number in four int8 digit
- * rows and the sums are exact integers (closer to the exact y than f32 sums; a row
- * holding an infinity or a NaN is summed in f32).  FP8: x split exactly into three
- * bf16 planes, f32 sums.  Any N, K; f32 pointers 4-byte aligned.  `workspace`: device
- * memory of at least the ..._workspace_bytes(M, N, K) bytes (0 where the GEMV runs), 256-byte
+ * to 8), the matrix cores beyond, x split exactly into three bf16 planes (bits below
+ * 2^-133 apart, which only values under 2^-109 have) and summed in f32.  Any N, K;
+ * f32 pointers 4-byte aligned.  `workspace`: device memory of at least the
+ * ..._workspace_bytes(M, N, K) bytes (0 where K is not split over blocks), 256-byte
  * aligned, contents need not be initialised. */
 int64_t tq_gemm_w8_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int tq_gemm_w8(const float* x, int64_t m, const int8_t* q, const float* s, const float* bias,

@@ -318,7 +318,6 @@ TileArgs a8_args(const void* qa, const float* sa, const void* qw, const float* s
     p.m = static_cast<int>(m);
     p.n = static_cast<int>(n);
     p.k = static_cast<int>(k);
-    p.lda = p.k;
     p.acc = acc;
     p.y = y;
     p.part = part;

@@ -5,7 +5,6 @@
 // timestamps (kTimed).  See tq_gemm.hip for the design.
 #pragma once
 
-#include "tq_digits.h"
 #include "tq_internal.h"
 
 namespace tq {
@@ -169,63 +168,11 @@ __device__ __forceinline__ void dma_epilogue(const Acc (&acc)[4][2], const DmaCt
     }
 }
 
-// Digit rows (tq_digits.h): the f32 activations and the exponents of the output
-// rows, which the m = 4 `rows` digit rows of the launch stand for.
-struct DigitArgs {
-    const float* x;
-    const int* ea;
-    int rows;
-};
-
-// The epilogue over digit rows: as above, four LDS rows joining into one row of y.
-__device__ __forceinline__ void dma_epilogue_digits(const i32x16 (&acc)[4][2], const DmaCtx& c, int8_t* lds, int m0,
-                                                    int n0, int n, int k, const int8_t* __restrict__ qw,
-                                                    const float* __restrict__ sw, const float* __restrict__ bias,
-                                                    float* __restrict__ y, const DigitArgs& da) {
-    const int lane = c.lane;
-    int8_t* ep = lds + c.wave * (64 * kDmaEpiRow);
-    const int lr = lane & 31, lh = lane >> 5;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const i32x16& a = acc[i][j];
-                const i32x4 v = i32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
-                *reinterpret_cast<i32x4*>(ep + (j * 32 + lr) * kDmaEpiRow + (i * 32 + 8 * g + 4 * lh) * 4) = v;
-            }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int nb = n0 + c.wn * 128 + 4 * lr;
-    if (nb >= n) return;
-    const f32x4 swv = *reinterpret_cast<const f32x4*>(sw + nb);
-    f32x4 bv = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (bias) bv = *reinterpret_cast<const f32x4*>(bias + nb);
-#pragma unroll 2
-    for (int t = 0; t < 16; t += 2) {
-        const int mm = (m0 + c.wm * 64) / 4 + t + lh;
-        if (mm >= da.rows) break;
-        i32x4 d[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            d[r] = *reinterpret_cast<const i32x4*>(ep + (4 * (t + lh) + r) * kDmaEpiRow + lr * 16);
-        const int e = da.ea[mm];
-        const float* xr = da.x + static_cast<int64_t>(mm) * k;
-        f32x4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            o[j] = digit_out(join_digits(d[0][j], d[1][j], d[2][j], d[3][j]), e, swv[j], bv[j], xr,
-                             qw + static_cast<int64_t>(nb + j) * k, k);
-        __builtin_nontemporal_store(o, reinterpret_cast<f32x4*>(y + static_cast<int64_t>(mm) * n + nb));
-    }
-}
-
 // kTimed (the bench library's instantiation only): lane 0 of every wave writes
 // the real-time clock (100 MHz) at its start, once the first stage has landed,
 // after the K loop and after the epilogue's stores, and the wave's hardware
 // id, to ts[(block * 4 + wave) * 6 ..].
-// kDigits: qa holds the digit rows of f32 activations (sa is unused).
-template <bool kTimed = false, bool kDigits = false>
+template <bool kTimed = false>
 __global__ __launch_bounds__(256, 1) void k_gemm_w8a8_dma(const int8_t* __restrict__ qa,
                                                           const float* __restrict__ sa,
                                                           const int8_t* __restrict__ qw,
@@ -233,8 +180,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_w8a8_dma(const int8_t* __restri
                                                           const float* __restrict__ bias, int m, int n,
                                                           int k, int32_t* __restrict__ acc_out,
                                                           float* __restrict__ y, int tiles_m,
-                                                          int tiles_n, uint64_t* __restrict__ ts = nullptr,
-                                                          DigitArgs da = {}) {
+                                                          int tiles_n, uint64_t* __restrict__ ts = nullptr) {
     uint64_t t[4] = {0, 0, 0, 0};
     if constexpr (kTimed) t[0] = __builtin_amdgcn_s_memrealtime();
     __shared__ __attribute__((aligned(1024))) int8_t lds[3 * kDmaStage];
@@ -292,10 +238,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_w8a8_dma(const int8_t* __restri
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if constexpr (kTimed) t[2] = __builtin_amdgcn_s_memrealtime();
-    if constexpr (kDigits)
-        dma_epilogue_digits(acc, c, lds, m0, n0, n, k, qw, sw, bias, y, da);
-    else
-        dma_epilogue(acc, c, lds, m0, n0, m, n, sa, sw, bias, acc_out, y);
+    dma_epilogue(acc, c, lds, m0, n0, m, n, sa, sw, bias, acc_out, y);
     if constexpr (kTimed) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores have left the wave
         t[3] = __builtin_amdgcn_s_memrealtime();

@@ -4,18 +4,12 @@
 //   y[m, n] = epilogue(sum_k A[m, k] * W[n, k])       A, W K-contiguous ("NT")
 //
 //  * GemmI8: A and W INT8 codes, int32 sums (exact).
-//  * GemmW8: A f32, W INT8 codes, on the i8 matrix cores: every row of A is a
-//    fixed-point number of 31 bits below its own largest magnitude, held as four
-//    balanced base-256 digits in four int8 rows (k_split_rows), so the sums of
-//    digits times codes are exact integers and the only errors are 2^-31 of the
-//    row's largest value per element and the final rounding: closer to the exact
-//    sum than f32 FMAs, at four i8 MFMAs per product (two bf16 ones' time).
 //  * GemmF8: A and W e4m3 codes on the fp8 matrix cores.
 //  * GemmF8b: the same codes widened to bf16 (exact products, f32 sums).
-//  * GemmF8W: A f32, W e4m3 codes, on the bf16 matrix cores.  Every f32
+//  * GemmF32<Val>: A f32, W INT8 or e4m3 codes, on the bf16 matrix cores.  Every f32
 //    activation is split exactly into three bf16 planes (8 + 8 + 8 significand
 //    bits, by truncation) and every code is exact in bf16, so each product is
-//    exact and only the f32 sums round.
+//    exact and only the f32 sums round, whatever the spread of a row's values.
 //
 //  * GemmW4, GemmW4GateUp, GemmW4H: INT4 g128 codes widened to bf16 (exact) against bf16
 //    activations (GemmW4H: f32 activations as bf16 hi + lo); every 128-long group's sum
@@ -25,8 +19,10 @@
 // The 8-bit bf16 forms add their running sums into a second set of accumulators every
 // kFlushStages stages (in f64 for GemmF8b), so that a sum's rounding grows with
 // the square root of a run's length and not of K: relative errors at K = 14336 are
-// 1.2e-7 (GemmF8W) and 4.7e-8 (GemmF8b), against 2.8e-7 and 7.2e-8 for a wave's f32
-// FMAs per output.
+// 1.0e-7 (GemmF32) and 4.7e-8 (GemmF8b), against 2.8e-7 and 7.2e-8 for a wave's f32
+// FMAs per output.  Runs of 256 k: with 512, rows that hold one value far above the
+// rest (1000 times, K = 512 to 4096) end 1.2 to 1.6 times a wave's f32 FMAs' error off,
+// with 256 1.0 to 1.25 times, at 2 % more time.
 //
 // Any M, N, K and any alignment of A, W and their rows (element-aligned
 // pointers): global loads are 8 to 32 bytes per lane at byte (codes) or 4-byte
@@ -37,7 +33,7 @@
 
 #include <algorithm>
 
-#include "tq_digits.h"
+#include "tq_internal.h"
 
 namespace tq {
 namespace {
@@ -46,10 +42,13 @@ typedef __bf16 tile_bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // Vectors at the alignment of their elements.
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
 typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
 typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
 typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 typedef uint32_t u32_a1 __attribute__((aligned(1)));
+
+__device__ __forceinline__ uint32_t f32_bits(float v) { return __builtin_bit_cast(uint32_t, v); }
 
 typedef __bf16 tile_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float tile_f32x2 __attribute__((ext_vector_type(2)));
@@ -247,7 +246,7 @@ struct SrcW4 {
 // many chunks of a row (one share per lane half).
 struct OpBf16 {
     typedef f32x16 Acc;
-    static constexpr bool kFlush = true, kDigits = false, kGroups = false, kGateUp = false;
+    static constexpr bool kFlush = true, kGroups = false, kGateUp = false;
     static constexpr int kFragChunks = 1;
     typedef u32x4 Frag;
     __device__ static Frag frag(const u32x4 (&c)[1]) { return c[0]; }
@@ -256,13 +255,16 @@ struct OpBf16 {
                                                        __builtin_bit_cast(tile_bf16x8, b), c, 0, 0, 0);
     }
 };
-struct GemmF8W : OpBf16 {
+template <class Val>
+struct GemmF32 : OpBf16 {
     typedef SrcF32 A;
-    typedef SrcBf16<ValFp8> W;
+    typedef SrcBf16<Val> W;
     typedef float part_t;
     static constexpr bool kRowScale = false;
-    static constexpr int kFlushStages = 8;
+    static constexpr int kFlushStages = 4;
 };
+typedef GemmF32<ValI8> GemmI8W;
+typedef GemmF32<ValFp8> GemmF8W;
 struct GemmF8b : OpBf16 {
     typedef SrcBf16<ValFp8> A;
     typedef SrcBf16<ValFp8> W;
@@ -288,7 +290,7 @@ struct GemmI8 {
     typedef SrcBytes<int8_t> W;
     typedef i32x16 Acc;
     typedef int32_t part_t;
-    static constexpr bool kRowScale = true, kFlush = false, kDigits = false, kGroups = false, kGateUp = false;
+    static constexpr bool kRowScale = true, kFlush = false, kGroups = false, kGateUp = false;
     static constexpr int kFragChunks = 1;
     typedef i32x4 Frag;
     __device__ static Frag frag(const u32x4 (&c)[1]) { return __builtin_bit_cast(i32x4, c[0]); }
@@ -296,17 +298,12 @@ struct GemmI8 {
         return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
     }
 };
-// Rows 4 m .. 4 m + 3 of A are the digits of row m (lowest first).
-struct GemmW8 : GemmI8 {
-    typedef int64_t part_t;
-    static constexpr bool kRowScale = false, kDigits = true;
-};
 struct GemmF8 {
     typedef SrcBytes<uint8_t> A;
     typedef SrcBytes<uint8_t> W;
     typedef f32x16 Acc;
     typedef float part_t;
-    static constexpr bool kRowScale = true, kFlush = false, kDigits = false, kGroups = false, kGateUp = false;
+    static constexpr bool kRowScale = true, kFlush = false, kGroups = false, kGateUp = false;
     static constexpr int kFragChunks = 2;
     typedef i32x8 Frag;
     __device__ static Frag frag(const u32x4 (&c)[2]) {
@@ -321,17 +318,15 @@ struct GemmF8 {
 };
 
 struct TileArgs {
-    const void* a;      // A [m, lda] (kDigits: [4 m, lda] digit rows)
+    const void* a;      // A [m, k]
     const void* w;      // W [n, k]
     const float* sa;    // row scales [m] (kRowScale)
-    const int* ea;      // row exponents [m] (kDigits)
-    const float* x;     // the f32 activations [m, k] (kDigits, rows that are not finite)
     const float* sw;    // column scales [n]
     const float* bias;  // [n] or null
     const uint16_t* sg;   // f16 group scales [n, k / 128] (kGroups)
     const void* w2;       // kGateUp: w and sg are gate's, w2 and sg2 up's, n both rows' count
     const uint16_t* sg2;  // (n = 2 F: partial sums hold gate's F columns, then up's)
-    int m, n, k, lda;   // m counts outputs' rows
+    int m, n, k;
     int tiles_m, tiles_n, split;
     int32_t* acc;  // int32 sums [m, n] or null (GemmI8)
     float* y;      // [m, n]
@@ -345,10 +340,7 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return g * (1.0f /
 template <class T>
 __device__ __forceinline__ void tile_store(const TileArgs& p, typename T::part_t v, int mm, int nn, float sw, float b) {
     const int64_t o = static_cast<int64_t>(mm) * p.n + nn;
-    if constexpr (T::kDigits) {
-        p.y[o] = digit_out(v, p.ea[mm], sw, b, p.x + static_cast<int64_t>(mm) * p.k,
-                           static_cast<const int8_t*>(p.w) + static_cast<int64_t>(nn) * p.k, p.k);
-    } else if constexpr (T::kGroups) {
+    if constexpr (T::kGroups) {
         p.y[o] = v + b;
     } else if constexpr (T::kRowScale) {
         if constexpr (__is_same(typename T::part_t, int32_t))
@@ -397,7 +389,7 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
     const int L = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3);
     const int tm = L % p.tiles_m, tn = (L / p.tiles_m) % p.tiles_n, ks = L / (p.tiles_m * p.tiles_n);
     const int m0 = tm * BM, n0 = tn * BN;
-    const int rows_a = T::kDigits ? 4 * p.m : p.m, rows_w = T::kGateUp ? p.n / 2 : p.n;
+    const int rows_w = T::kGateUp ? p.n / 2 : p.n;
     static_assert(!T::kGateUp || TN == 2, "a wave holds 32 gate and the same 32 up columns");
     const int stages = (p.k + BK - 1) / BK;
     constexpr int kUnit = T::kGroups ? 2 : 1;  // whole groups per split (two stages each)
@@ -412,7 +404,7 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
 #pragma unroll
     for (int i = 0; i < kAItems; ++i) {
         const int r = (tid >> 3) + 32 * i;
-        asrc[i] = static_cast<const typename SA::elem_t*>(p.a) + static_cast<int64_t>(min(m0 + r, rows_a - 1)) * p.lda;
+        asrc[i] = static_cast<const typename SA::elem_t*>(p.a) + static_cast<int64_t>(min(m0 + r, p.m - 1)) * p.k;
         adst[i] = r * kTileRow + ((chunk ^ tile_swz(r)) << 4);
     }
 #pragma unroll
@@ -609,9 +601,7 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
             return acc[0][i][j][e];
     };
     // lane holds D[m = 8 (e/4) + 4 lh + e % 4][n = l32] of each 32 x 32 tile: a
-    // store covers 32 consecutive n of two rows; with digit rows, e % 4 is the
-    // digit and a lane holds whole sums of 4 rows
-    constexpr int kPer = T::kDigits ? 4 : 1;
+    // store covers 32 consecutive n of two rows
     if constexpr (T::kGateUp) {
         const int nn = column(0), f = rows_w;
         if (nn >= f) return;
@@ -640,14 +630,10 @@ __global__ __launch_bounds__(256, kOcc) void k_gemm_tile(TileArgs p) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; e += kPer) {
-                const int mm = (m0 + (wm * TM + i) * 32 + 8 * (e >> 2) + 4 * lh + (e & 3)) / kPer;
+            for (int e = 0; e < 16; ++e) {
+                const int mm = m0 + (wm * TM + i) * 32 + 8 * (e >> 2) + 4 * lh + (e & 3);
                 if (!nval || mm >= p.m) continue;
-                typename T::part_t v;
-                if constexpr (T::kDigits)
-                    v = join_digits(sum(i, j, e), sum(i, j, e + 1), sum(i, j, e + 2), sum(i, j, e + 3));
-                else
-                    v = sum(i, j, e);
+                const typename T::part_t v = sum(i, j, e);
                 if (p.split == 1)
                     tile_store<T>(p, v, mm, nn, sw, bv);
                 else
@@ -693,8 +679,6 @@ struct TileCosts<GemmI8> {
     static constexpr TileShape shape[kTileShapes] = {{128, 128, 700, 800}, {64, 64, 270, 310}, {32, 128, 285, 325}, {64, 128, 500, 510}};
 };
 template <>
-struct TileCosts<GemmW8> : TileCosts<GemmI8> {};
-template <>
 struct TileCosts<GemmF8> {
     static constexpr TileShape shape[kTileShapes] = {{128, 128, 700, 760}, {64, 64, 270, 300}, {32, 128, 270, 295}, {64, 128, 430, 450}};
 };
@@ -706,6 +690,8 @@ template <>
 struct TileCosts<GemmF8W> {
     static constexpr TileShape shape[kTileShapes] = {{128, 128, 2100, 2400}, {64, 64, 840, 690}, {32, 128, 780, 600}, {64, 128, 1150, 960}};
 };
+template <>
+struct TileCosts<GemmI8W> : TileCosts<GemmF8W> {};
 
 template <>
 struct TileCosts<GemmW4> {
@@ -734,19 +720,19 @@ struct TilePlan {
 // operands at that time per 128-byte stage.
 template <class T>
 TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int dma_stage, bool may_split) {
-    const int64_t cus = device_cu_count(), rows = T::kDigits ? 4 * m : m;
+    const int64_t cus = device_cu_count();
     const int64_t stages = (k + 8 * T::A::kElems - 1) / (8 * T::A::kElems);
     TilePlan best{kTile64x128, 1, 0, 0, 0, 0};
     int64_t best_ns = INT64_MAX;
     if (dma_stage > 0) {
-        const int64_t blocks = ((rows + 127) / 128) * ((n + 255) / 256);
+        const int64_t blocks = ((m + 127) / 128) * ((n + 255) / 256);
         best.shape = kTileDma;
         best_ns = (blocks + cus - 1) / cus * (k / 128) * dma_stage + 4000;
     }
     for (int c = 0; c < kTileShapes; ++c) {
         if (T::kGateUp && (c == kTile64x64 || c == kTile32x128)) continue;  // two column tiles per wave
         const TileShape& t = TileCosts<T>::shape[c];
-        const int64_t tm = (rows + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
+        const int64_t tm = (m + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
         for (int split : {1, 2, 3, 4, 6, 8, 12, 16}) {
             if (split > 1 && (!may_split || stages < 4 * split || tm * tn * split > 4 * cus)) break;
             const int64_t rounds = (tm * tn * split + cus - 1) / cus, per = (stages + split - 1) / split;
@@ -762,16 +748,16 @@ TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int dma_stage, bool may_spli
     }
     if (best.shape != kTileDma) {
         const TileShape& t = TileCosts<T>::shape[best.shape];
-        best.tiles_m = static_cast<int>((rows + t.bm - 1) / t.bm);
+        best.tiles_m = static_cast<int>((m + t.bm - 1) / t.bm);
         best.tiles_n = static_cast<int>((n + t.bn - 1) / t.bn);
     }
     return best;
 }
 
-// m, n and k (and 4 m with digit rows) fit the kernels' 32-bit indexes
-inline bool tile_fits(int64_t rows, int64_t n, int64_t k) {
-    return rows < (int64_t(1) << 31) - 128 && n < (int64_t(1) << 31) - 128 && k < (int64_t(1) << 31) - 1024 &&
-           ((rows + 31) / 32) * ((n + 63) / 64) < (int64_t(1) << 31);
+// m, n and k fit the kernels' 32-bit indexes
+inline bool tile_fits(int64_t m, int64_t n, int64_t k) {
+    return m < (int64_t(1) << 31) - 128 && n < (int64_t(1) << 31) - 128 && k < (int64_t(1) << 31) - 1024 &&
+           ((m + 31) / 32) * ((n + 63) / 64) < (int64_t(1) << 31);
 }
 
 // Launches the plan's tiles (not kTileDma) and, for a split, the finishing kernel.

@@ -29,7 +29,6 @@ TileArgs w4_args(const void* a, const uint8_t* packed, const uint16_t* s, const 
     p.m = static_cast<int>(m);
     p.n = static_cast<int>(n);
     p.k = static_cast<int>(k);
-    p.lda = p.k;
     p.y = y;
     p.part = part;
     return p;

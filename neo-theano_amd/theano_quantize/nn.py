@@ -21,9 +21,9 @@ Decode shapes (a few tokens) run the dequant-GEMV kernels; in "w8a8" and "fp8"
 modes the GEMV quantizes the activation rows itself (the same codes and product
 as quantize + GEMM, one launch).  "w4" runs the tiled GEMV in passes of 16 tokens
 up to M = 32, where it is faster than the prefill GEMM, whose 64-row M tiles are
-mostly empty there.  Prefill shapes run the matrix cores: i8 for W8A8 and for the
-INT8 weight-only mode (f32 activations as exact integer digits), fp8, and bf16 for
-the FP8 weight-only and W4A16 modes.
+mostly empty there.  Prefill shapes run the matrix cores: i8 for W8A8, fp8 for
+"fp8", and bf16 for W4A16 and the two 8-bit weight-only modes (f32 activations as
+three exact bf16 planes).
 """
 from __future__ import annotations
 

@@ -140,28 +140,61 @@ def test_weight_only_any_shape(tq, m, n, k, fp8):
     x[2] *= 1e-36
     x[3, k // 2] *= 1e4  # one value far above its row
     qw = _codes(torch, (n, k), 8, fp8)
-    for off in (0, 1):
-        y, sw, b = _weight_only(torch, fp8, x, qw, m, n, k, off == 1, off)
+    for off, bias in ((0, False), (0, True), (1, True)):
+        y, sw, b = _weight_only(torch, fp8, x, qw, m, n, k, bias, off)
         ref = x.double() @ qw.double().t().contiguous() * sw.double()
         scale = (x.double().abs() @ qw.double().abs().t().contiguous()) * sw.double()
         if b is not None:
             ref = ref + b.double()
-        # INT8: 2^(e - 30) per value, e the exponent of the row's largest, and the final
-        # rounding (below 2^-126 at its least); FP8: as the sums of test_fp8_any_shape, and
-        # bits of x below 2^-133 have no place in a bf16 plane
+        # the matrix cores' sums as in test_fp8_any_shape, over runs of 256; bits of x below
+        # 2^-133 have no place in a bf16 plane; the final rounding below 2^-126 at its least
         tiny = 2.0 ** -126
         wsum = qw.double().abs().sum(1) * sw.double()
-        if fp8:
-            bound = 2.0 ** -23 * min(k, 512) ** 0.5 * scale + 2.0 ** -23 * ref.abs() + 2.0 ** -133 * wsum + tiny
-        elif m * n * k <= 4 << 20:  # f32: K / 64 additions per lane and a tree, over rounded products
+        if m * n * k > 4 << 20:
+            bound = 2.0 ** -23 * min(k, 256) ** 0.5 * scale + 2.0 ** -23 * ref.abs() + 2.0 ** -133 * wsum + tiny
+        else:  # f32: K / 64 additions per lane and a tree, over rounded products
             bound = 2.0 ** -23 * (k / 64 + 16) ** 0.5 * scale + 2.0 ** -23 * ref.abs() + tiny
-        else:
-            bound = 2.0 ** -30 * x.double().abs().amax(1)[:, None] * wsum + 2.0 ** -24 * ref.abs() + tiny
         err = (y.double() - ref).abs()
         assert bool((err <= bound).all()), (err / bound).max().item()
         rows = torch.arange(m, device="cuda") > 2
         rel = (err[rows].norm(dim=1) / ref[rows].norm(dim=1)).max().item()
-        assert rel < (4e-7 if fp8 or m * n * k <= 4 << 20 else 1e-7) * (1 + 64 / (n * k) ** 0.5), rel
+        assert rel < 4e-7 * (1 + 64 / (n * k) ** 0.5), rel
+
+
+@pytest.mark.parametrize("m,k", [(13, 4096), (40, 1000), (6, 14336)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_weight_only_rows_of_wide_range(tq, m, k, fp8):
+    """Rows that hold a few values far above the rest, against outputs whose codes there
+    are zero, small or large, and outputs of one code alone: each output to f32 accuracy
+    of its own sum |x| |w|, whatever the row's largest value is.  (At the least those of
+    one code alone and those whose large values meet zeros were off by up to their whole
+    value in a fixed-point form of x.)"""
+    import torch
+
+    n = 1500
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(m, k, generator=g, device="cuda")
+    qw = _codes(torch, (n, k), 13, fp8)
+    one = torch.tensor(1.0, device="cuda").to(qw.dtype)
+    cols = torch.randperm(k, generator=g, device="cuda")[:100]
+    raw, unit = qw.view(torch.uint8), one.view(torch.uint8)
+    raw[:300, cols] = 0  # outputs that do not see the large values
+    raw[300:500, cols] = unit  # or see them with the smallest whole code
+    raw[500:700] = 0  # one code alone: y is that x, times a whole number
+    raw[torch.arange(500, 700, device="cuda"), torch.arange(200, device="cuda") * (k // 200)] = unit
+    raw[:, cols[0]] = 0  # a column that no output uses
+    large = [(c, r) for r in (1e3, 1e5, 1e9, 1e30) for c in (1, 3, 100)]
+    for i in range(m):
+        c, r = large[i % len(large)]
+        x[i, cols[:c]] *= r
+    y, sw, b = _weight_only(torch, fp8, x, qw, m, n, k, False, 0)
+    ref = x.double() @ qw.double().t().contiguous() * sw.double()
+    mag = (x.double().abs() @ qw.double().abs().t().contiguous()) * sw.double()
+    # up to 64 additions in a run of 256 k and K / 256 runs, each rounding by 2^-24 of its
+    # partial sum at most, uniformly: five standard deviations
+    bound = 5 / 3 ** 0.5 * 2.0 ** -24 * (64 + k / 256) ** 0.5 * mag + 2.0 ** -23 * ref.abs() + 2.0 ** -126
+    err = (y.double() - ref).abs() / bound
+    assert err.max().item() <= 1, (err.max().item(), err.argmax().item())
 
 
 @pytest.mark.parametrize("n,k", [(5, 17), (9, 700), (33, 1023), (40, 1041), (130, 2049), (70, 4097), (35, 8200),
@@ -195,8 +228,7 @@ def test_gemv_any_row_length(tq, m, n, k, fp8):
 @pytest.mark.parametrize("m,n,k", [(1, 1031, 8195), (4, 513, 14336), (3, 1025, 16384), (2, 11183, 9001),
                                    (2, 11184, 9001)])
 def test_w8_long_rows(tq, m, n, k):
-    """Runs of several rows per block of the long-row GEMV, and both sides of the product
-    (96 Mi weights) from which the matrix cores take them."""
+    """Runs of several rows per block of the long-row GEMV, up to 96 Mi weights."""
     import torch
 
     x = torch.randn(m, k, generator=torch.Generator(device="cuda").manual_seed(m + k), device="cuda")
@@ -204,7 +236,7 @@ def test_w8_long_rows(tq, m, n, k):
     y, sw, b = _weight_only(torch, False, x, qw, m, n, k, True, 1)
     ref = x.double() @ qw.double().t().contiguous() * sw.double() + b.double()
     mag = (x.double().abs() @ qw.double().abs().t().contiguous()) * sw.double() + b.double().abs()
-    # as test_gemv_any_row_length; the digits' sums stay far inside it
+    # as test_gemv_any_row_length
     bound = 2.0 ** -24 * (k / 64 + 16) ** 0.5 * mag + 2.0 ** -22 * ref.abs()
     assert bool(((y.double() - ref).abs() <= bound).all())
 
@@ -233,6 +265,13 @@ def test_weight_only_rows_that_are_not_finite(tq, fp8, n, k):
     assert torch.equal(y[rows].isinf(), f32[rows].isinf())
     inf = f32[rows].isinf()
     assert torch.equal(y[rows][inf], f32[rows][inf])
+    # the row of 3e38: infinite where that product overflows f32, else to f32 accuracy of its sum
+    p = x[10, 1].double() * qw[:, 1].double()
+    over = p.abs() * sw.double().clamp(min=1) > torch.finfo(torch.float32).max
+    assert torch.equal(y[10][over], (p[over].sign() * float("inf")).float())
+    mag = x[10].double().abs() @ qw.double().abs().t().contiguous() * sw.double()
+    err = (y[10].double() - ref[10]).abs()
+    assert bool((err <= 2.0 ** -24 * (k / 64 + 16) ** 0.5 * mag + 2.0 ** -23 * ref[10].abs())[~over].all())
     fin = torch.tensor([i for i in range(m) if i not in (5, 6, 7, 8, 9, 10)], device="cuda")
     assert ((y[fin].double() - ref[fin]).norm() / ref[fin].norm()).item() < 4e-7
 
