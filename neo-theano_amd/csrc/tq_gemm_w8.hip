@@ -12,21 +12,28 @@
 namespace tq {
 namespace {
 
-// Which calls run the GEMV (passes over the weights of 4 tokens, of 2 past K = 4096)
-// and which the matrix cores, whose split and finish launches cost ~6 us: up to 4
-// tokens the GEMV (N = K = 4096: 6.9 us at 4; N = 4096, K = 8192: 16 us on both); past
-// 8 the matrix cores (13 against 18 us at 9); between, the GEMV while a pass over the
-// weights is short (N = K = 4096: 11.5-13.5 us against 13; N = 14336, K = 4096: 29-34
-// against 20; N = 4096, K = 4097, 24-33 against 15).  The FP8 form's matrix kernel
-// takes longer: the GEMV's aligned form keeps all of its 5 to 8 tokens.
-// Long rows of many outputs go over from 2 INT8 tokens on, at x's traffic (N = 14336, K =
-// 8960: 36 / 45 / 53 us at 2 / 3 / 4 tokens against 33; N = 4096, K = 16384: 16 / 19 / 21
-// against 24).
-bool gemv_runs(int64_t m, int64_t n, int64_t k, bool fp8) {
-    if (!fp8 && m > 1 && k > 8192 && n * k > 96 << 20) return false;
-    if (m <= 4 || m > 8) return m <= 4;
-    const bool vec16 = k % 16 == 0 && k <= 8192;
-    return vec16 ? fp8 || n * k <= 4096 * 4096 : n * k <= 2 << 20;
+// Which calls run the GEMV and which the matrix cores, by the GEMV's passes over the
+// weights (us at cold weights, both sides; the two code types alike):
+//  * up to 4 tokens the GEMV (N = K = 4096: 7 against 16 at 4; N = 4096, K = 8192, two
+//    passes: 16.5 against 22.4), but for wide outputs of rows of 8 K to 10 K, which leave
+//    half of the GEMV's lanes idle (N = 14336, K = 8960 at 4 tokens: 54 against 48; N =
+//    12288, K = 16384: 51 against 74);
+//  * 5 to 8 tokens of aligned rows up to 4096, two passes, while these are short (N = K =
+//    4096: 12.1-13.5 against 16; N = 12288: 25-28 against 28; N = 14336: 27-31 against
+//    28; N = 16384, K = 256: 14 against 8);
+//  * aligned rows up to 8192, three or four passes: N = 4096, K = 6144 at 6 tokens 19.4
+//    against 19.5, K = 8192 24 against 22; at 8 N = 1024, K = 8192 16.4 against 17.5, N =
+//    2048 22 against 18;
+//  * other rows up to 2048, one pass of 8: N = 8000, K = 1000 10.2 against 12.8; longer,
+//    two of 4: N = 1024, K = 14336 18.4 against 21.9 at 8, N = 4096, K = 4097 21 against
+//    18 at 5;
+//  * past 8 the matrix cores (N = K = 4096 at 12: 20 against 16).
+bool gemv_runs(int64_t m, int64_t n, int64_t k) {
+    if (m > 8) return false;
+    if (k <= 4096 && k % 16 == 0) return m <= 4 || (n <= 12288 && n * k <= 48 << 20);
+    if (k <= 8192 && k % 16 == 0) return m <= 4 || n * k <= (m <= 6 ? 24 << 20 : 8 << 20);
+    if (m <= 4) return m < 4 || k > 10240 || n * k <= 96 << 20;
+    return k <= 2048 ? n * k <= 8 << 20 : n <= 1024;
 }
 // So little work that one launch of a wave per output is ahead (N = 1000, K = 100: 3.9
 // against 7.1 us at 16 tokens).
@@ -43,8 +50,7 @@ int launch_gemv(const float* x, int64_t m, const uint8_t* q, const float* s, con
 
 template <class T>
 int64_t workspace_bytes(int64_t m, int64_t n, int64_t k) {
-    constexpr bool kFp8 = __is_same(T, GemmF8W);
-    if (n <= 0 || k <= 0 || gemv_runs(m, n, k, kFp8) || tiny(m, n, k) || !tile_fits(m, n, k)) return 0;
+    if (n <= 0 || k <= 0 || gemv_runs(m, n, k) || tiny(m, n, k) || !tile_fits(m, n, k)) return 0;
     return tile_plan<T>(m, n, k, 0, true).part_bytes;
 }
 
@@ -52,13 +58,12 @@ template <class T>
 int weight_only(const float* x, int64_t m, const typename T::W::elem_t* q, const float* s, const float* bias,
                 int64_t n, int64_t k, void* workspace, int64_t workspace_bytes, float* y, tq_stream_t stream,
                 const char* what) {
-    constexpr bool kFp8 = __is_same(T, GemmF8W);
     TQ_REQUIRE(m >= 0 && n >= 0 && k >= 0, "%s: negative shape", what);
     if (m == 0 || n == 0) return TQ_OK;
     TQ_REQUIRE(y && s && (k == 0 || (x && q)), "%s: null pointer", what);
     TQ_REQUIRE(aligned(x, 4) && aligned(s, 4) && (!bias || aligned(bias, 4)) && aligned(y, 4),
                "%s: misaligned f32 pointer", what);
-    if (gemv_runs(m, n, k, kFp8)) return launch_gemv(x, m, q, s, bias, n, k, y, stream);
+    if (gemv_runs(m, n, k)) return launch_gemv(x, m, q, s, bias, n, k, y, stream);
     const hipStream_t st = as_hip(stream);
     if (tiny(m, n, k) || !tile_fits(m, n, k)) return launch_linear_8bit_generic(x, m, q, s, bias, n, k, y, st);
     const TilePlan plan = tile_plan<T>(m, n, k, 0, true);

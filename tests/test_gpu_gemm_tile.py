@@ -241,6 +241,32 @@ def test_w8_long_rows(tq, m, n, k):
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m,n,k,gemv", [(8, 12288, 512, True), (8, 12304, 512, False), (9, 512, 1024, False),
+                                        (6, 4096, 6144, True), (6, 4112, 6144, False), (8, 1024, 8192, True),
+                                        (7, 1040, 8192, False), (8, 8388, 1000, True), (5, 8389, 1000, False),
+                                        (8, 1024, 8208, True), (5, 1025, 8208, False), (4, 11183, 9001, True),
+                                        (4, 11184, 9001, False), (3, 11184, 9001, True), (4, 12288, 10241, True)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_weight_only_few_tokens(tq, m, n, k, gemv, fp8):
+    """Both sides of each line between the GEMV and the matrix cores."""
+    import torch
+
+    from theano_quantize import _abi
+    from theano_quantize._tensor import ptr, stream
+
+    x = torch.randn(m, k, generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+    qw = _codes(torch, (n, k), 14, fp8)
+    y, sw, b = _weight_only(torch, fp8, x, qw, m, n, k, True, 0)
+    ref = x.double() @ qw.double().t().contiguous() * sw.double() + b.double()
+    mag = (x.double().abs() @ qw.double().abs().t().contiguous()) * sw.double() + b.double().abs()
+    # as test_gemv_any_row_length
+    bound = 2.0 ** -24 * (k / 64 + 16) ** 0.5 * mag + 2.0 ** -22 * ref.abs()
+    assert bool(((y.double() - ref).abs() <= bound).all())
+    y2 = torch.empty_like(y)
+    _abi.call("tq_gemv_fp8" if fp8 else "tq_gemv_w8", ptr(x), m, ptr(qw), ptr(sw), ptr(b), n, k, ptr(y2), stream())
+    assert torch.equal(y, y2) == gemv  # the GEMV's bits where it runs; other sums elsewhere
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("n,k", [(48, 384), (33, 130), (1033, 130), (512, 2048)])
 def test_weight_only_rows_that_are_not_finite(tq, fp8, n, k):
