@@ -20,19 +20,21 @@ namespace {
 //    12288, K = 16384: 51 against 74);
 //  * 5 to 8 tokens of aligned rows up to 4096, two passes, while these are short (N = K =
 //    4096: 12.1-13.5 against 16; N = 12288: 25-28 against 28; N = 14336: 27-31 against
-//    28; N = 16384, K = 256: 14 against 8);
+//    28; N = 8192, K = 512 9.5 against 10; N = 16384, K = 256 14 against 8);
 //  * aligned rows up to 8192, three or four passes: N = 4096, K = 6144 at 6 tokens 19.4
 //    against 19.5, K = 8192 24 against 22; at 8 N = 1024, K = 8192 16.4 against 17.5, N =
 //    2048 22 against 18;
+//  * other rows up to 512, a wave per output: N = 15000, K = 300 21 against 9 at 5;
 //  * other rows up to 2048, one pass of 8: N = 8000, K = 1000 10.2 against 12.8; longer,
 //    two of 4: N = 1024, K = 14336 18.4 against 21.9 at 8, N = 4096, K = 4097 21 against
 //    18 at 5;
 //  * past 8 the matrix cores (N = K = 4096 at 12: 20 against 16).
 bool gemv_runs(int64_t m, int64_t n, int64_t k) {
     if (m > 8) return false;
-    if (k <= 4096 && k % 16 == 0) return m <= 4 || (n <= 12288 && n * k <= 48 << 20);
+    if (k <= 4096 && k % 16 == 0) return m <= 4 || (n <= (k < 1024 ? 8192 : 12288) && n * k <= 48 << 20);
     if (k <= 8192 && k % 16 == 0) return m <= 4 || n * k <= (m <= 6 ? 24 << 20 : 8 << 20);
     if (m <= 4) return m < 4 || k > 10240 || n * k <= 96 << 20;
+    if (k <= 512) return n * k <= 2 << 20;
     return k <= 2048 ? n * k <= 8 << 20 : n <= 1024;
 }
 // So little work that one launch of a wave per output is ahead (N = 1000, K = 100: 3.9

@@ -241,7 +241,8 @@ def test_w8_long_rows(tq, m, n, k):
     assert bool(((y.double() - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("m,n,k,gemv", [(8, 12288, 512, True), (8, 12304, 512, False), (9, 512, 1024, False),
+@pytest.mark.parametrize("m,n,k,gemv", [(8, 12288, 1024, True), (8, 12304, 1024, False), (8, 8192, 512, True),
+                                        (8, 8208, 512, False), (5, 8192, 250, True), (5, 8400, 250, False), (9, 512, 1024, False),
                                         (6, 4096, 6144, True), (6, 4112, 6144, False), (8, 1024, 8192, True),
                                         (7, 1040, 8192, False), (8, 8388, 1000, True), (5, 8389, 1000, False),
                                         (8, 1024, 8208, True), (5, 1025, 8208, False), (4, 11183, 9001, True),
