@@ -538,10 +538,11 @@ LinTiles lin_tiles(int64_t m, int64_t n, int64_t k) {
     return n % LinCfg::BN != 0 || narrow.cost < wide.cost ? narrow : wide;
 }
 
-// ns of a wide tile's (16384 outputs') group: gate/up 2.0 us, down 2.1 us, Linear (32768
-// outputs) 2.2 us at M = 512, D = K = 4096, F = N = 14336
+// ns of a wide tile's (16384 outputs') group: gate/up 2.0 us, down 2.1 us at M = 512, D =
+// 4096, F = 14336; the Linear's (32768 outputs) 1.8 us beside its stores at 5 TB/s, fitted
+// to where it and the tiles cross at M = 33 to 2048 (never 5 % behind the faster of the two)
 constexpr int64_t kUnit16384 = 16384 * kWideCost;
-constexpr int64_t kGuUnitNs = 2000, kDnUnitNs = 2100, kLinUnitNs = 1100;
+constexpr int64_t kGuUnitNs = 2000, kDnUnitNs = 2100, kLinUnitNs = 900;
 
 // Whether the pipelined kernels run an FFN of these sizes: they take D and F in
 // multiples of 256, and stay ahead of the register-staged tiles where their own tiles
@@ -559,7 +560,7 @@ bool lin_pipelined(int64_t m, int64_t n, int64_t k) {
     if (k == 0 || k % 256 != 0 || n % LinSCfg::BN != 0) return false;
     const W4TileCost tile = w4_linear_tile_cost(m, n, k);
     if (tile.ns == 0) return false;
-    return 9000 + lin_tiles(m, n, k).cost / 1000 * kLinUnitNs / (kUnit16384 / 1000) <= tile.ns;
+    return 10000 + lin_tiles(m, n, k).cost / 1000 * kLinUnitNs / (kUnit16384 / 1000) + m * n * 4 / 5000 <= tile.ns;
 }
 
 }  // namespace

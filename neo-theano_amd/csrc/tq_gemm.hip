@@ -12,7 +12,8 @@
 // the byte-to-lane assignment that suits its loads; integer accumulation makes
 // the order invisible in the result.
 //
-// Three kernels:
+// The kernels, by tile_plan's and wave_per_output_ns's estimates past the skinny ones:
+//  * k_gemm_w8a8_skinny, k_gemm_fp8_skinny (M <= 16, K <= 8192): N / 16 blocks.
 //  * k_gemm_w8a8_dma (K % 128 == 0): one 256-thread block per 128 (m) x 256 (n)
 //    tile.  K advances in 128-byte stages through a 3-deep LDS ring filled by
 //    global_load_lds_dwordx4 (global -> LDS without registers; one instruction
@@ -26,10 +27,11 @@
 //    goes through LDS to write 512-byte row segments.
 //  * k_gemm_tile (tq_gemm_tile.h; any M, N, K, any alignment): smaller tiles, K
 //    split over blocks where they leave CUs idle, for the M and N that do not fill
-//    the chip with 128 x 256 tiles and the shapes the LDS DMA cannot load.  Which
-//    one runs is tile_plan's estimate: at M = 64, N = 4096, K = 14336 the tiles
-//    take 15 us against 70 us for sixteen DMA blocks; at M = 2048, N = K = 4096
-//    the DMA kernel's 36 us stand against 51 us.
+//    the chip with 128 x 256 tiles and the shapes the LDS DMA cannot load: at M = 64,
+//    N = 4096, K = 14336 the tiles take 15 us against 70 us for sixteen DMA blocks;
+//    at M = 2048, N = K = 4096 the DMA kernel's 36 us stand against 51 us, at M = 1024
+//    25 against 33.
+//  * a wave per output (tq_generic.hip) on the smallest calls.
 #include "tq_internal.h"
 
 namespace tq {
@@ -304,8 +306,21 @@ bool i8_skinny(int64_t m, int64_t n, int64_t k) {
 }
 bool fp8_skinny(int64_t m, int64_t k) { return m <= 16 && k <= 8192; }
 
-// ns per 128-byte stage of the DMA kernels' 128 x 256 tiles (M = 2048, N = K = 4096)
-constexpr int kDmaStageI8 = 1000, kDmaStageF8 = 950;
+constexpr DmaCost kDmaI8{580, 400, 6200, 5500}, kDmaF8{640, 300, 6300, 6500};
+
+// The products of a wave per output (tq_generic.hip) in ns: 64 k a step, 105 ns each in
+// turn (N = 300, K = 4096 at one token 8.4 us) and up to 280 where several rows read the
+// same weights (15.3 us at two, 16.2 at three), 40 steps a ns over the chip (FP8, summed in
+// f64, 25), the weights at 1 TB/s for each of the first four rows; a quarter more for rows
+// off the 64-byte segments.  Ahead of the tiles' LDS fills and finishing launch on the
+// smallest calls (FP8 at one token, N = K = 1000: 5 against 8 us; 64 x 64 x 64: 3.0 against
+// 5.3).
+int64_t wave_per_output_ns(int64_t m, int64_t n, int64_t k, int steps_per_ns) {
+    const int64_t steps = (k + 63) / 64, step = m == 1 ? 105 : m == 2 ? 200 : 280;
+    const int64_t ns =
+        std::max({step * steps, m * n * (steps + 2) / steps_per_ns, n * k * std::min<int64_t>(m, 4) / 1000});
+    return 2700 + (k % 64 ? ns * 5 / 4 : ns);
+}
 
 TileArgs a8_args(const void* qa, const float* sa, const void* qw, const float* sw, const float* bias, int64_t m,
                  int64_t n, int64_t k, int32_t* acc, float* y, void* part) {
@@ -329,7 +344,7 @@ TileArgs a8_args(const void* qa, const float* sa, const void* qw, const float* s
 template <class T>
 int64_t a8_part_bytes(int64_t m, int64_t n, int64_t k) {
     if (m <= 0 || n <= 0 || k <= 0 || !tile_fits(m, n, k)) return 0;
-    return tile_plan<T>(m, n, k, 0, true).part_bytes;
+    return tile_plan<T>(m, n, k, nullptr, true).part_bytes;
 }
 
 // workspace of tq_linear_{w8a8,fp8}: codes [m, k], then scales [m], then partial sums
@@ -369,7 +384,9 @@ int gemm_w8a8(const int8_t* qa, const float* sa, const int8_t* qw, const float* 
         return check_launch(what);
     }
     if (!tile_fits(m, n, k)) return launch_gemm_w8a8_generic(qa, sa, qw, sw, bias, m, n, k, acc, y, st);
-    const TilePlan plan = tile_plan<GemmI8>(m, n, k, vec && k % kDmaBK == 0 ? kDmaStageI8 : 0, ws != nullptr);
+    const TilePlan plan = tile_plan<GemmI8>(m, n, k, vec && k % kDmaBK == 0 ? &kDmaI8 : nullptr, ws != nullptr);
+    if (wave_per_output_ns(m, n, k, 40) < plan.ns)
+        return launch_gemm_w8a8_generic(qa, sa, qw, sw, bias, m, n, k, acc, y, st);
     if (plan.shape == kTileDma) {
         const int tm = static_cast<int>((m + kDmaBM - 1) / kDmaBM), tn = static_cast<int>((n + kDmaBN - 1) / kDmaBN);
         k_gemm_w8a8_dma<false><<<static_cast<unsigned>(tm * tn), 256, 0, st>>>(
@@ -408,8 +425,10 @@ int gemm_fp8(const uint8_t* qa, const float* sa, const uint8_t* qw, const float*
     }
     if (!tile_fits(m, n, k)) return launch_gemm_fp8_generic(qa, sa, qw, sw, bias, m, n, k, y, st);
     const TileArgs args = a8_args(qa, sa, qw, sw, bias, m, n, k, nullptr, y, ws);
-    const TilePlan plan = native ? tile_plan<GemmF8>(m, n, k, kDmaStageF8, ws != nullptr)
-                                 : tile_plan<GemmF8b>(m, n, k, 0, ws != nullptr);
+    const TilePlan plan = native ? tile_plan<GemmF8>(m, n, k, &kDmaF8, ws != nullptr)
+                                 : tile_plan<GemmF8b>(m, n, k, nullptr, ws != nullptr);
+    if (wave_per_output_ns(m, n, k, 25) < plan.ns)
+        return launch_gemm_fp8_generic(qa, sa, qw, sw, bias, m, n, k, y, st);
     if (plan.shape == kTileDma) {
         const int tm = static_cast<int>((m + kDmaBM - 1) / kDmaBM), tn = static_cast<int>((n + kDmaBN - 1) / kDmaBN);
         k_gemm_fp8_dma<<<static_cast<unsigned>(tm * tn), 256, 0, st>>>(

@@ -664,11 +664,14 @@ __global__ __launch_bounds__(256) void k_gemm_tile_finish(TileArgs p) {
 }
 
 // ------------------------------------------------------------------ host side
-// Tile sizes and the time of one stage of one block in ns: with at most one block
-// on a CU (t1) and per block when several share it (t2), measured on M = 16 to
-// 2048 at N = K = 4096, N = 14336 and K = 14336.
+// Tile sizes and a launch's time in ns: of each stage with at most one block on a CU
+// (t1) and per block when several share it (t2), and apart from the stages (launch,
+// first loads, stores) with one round of blocks (f1) and per round (f2); `split` is the
+// finishing launch's.  Fitted to every tile and split at M = 1 to 2048 and 18 weights from
+// 64 x 64 to 14336 x 4096, 4096 x 14336, 16384 x 128 and 64 x 16384, read past the caches:
+// the chosen one takes 1.01 to 1.03 times the fastest's time on average.
 struct TileShape {
-    int bm, bn, t1, t2;
+    int bm, bn, t1, t2, f1, f2;
 };
 constexpr int kTileShapes = 4;
 enum { kTile128x128, kTile64x64, kTile32x128, kTile64x128 };
@@ -676,59 +679,72 @@ template <class T>
 struct TileCosts;
 template <>
 struct TileCosts<GemmI8> {
-    static constexpr TileShape shape[kTileShapes] = {{128, 128, 700, 800}, {64, 64, 270, 310}, {32, 128, 285, 325}, {64, 128, 500, 510}};
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 600, 640, 8000, 7500}, {64, 64, 270, 250, 4300, 1770}, {32, 128, 290, 250, 4500, 3770}, {64, 128, 430, 360, 6250, 4300}};
+    static constexpr int split = 2200;
 };
 template <>
 struct TileCosts<GemmF8> {
-    static constexpr TileShape shape[kTileShapes] = {{128, 128, 700, 760}, {64, 64, 270, 300}, {32, 128, 270, 295}, {64, 128, 430, 450}};
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 630, 600, 8000, 7000}, {64, 64, 270, 230, 4600, 1560}, {32, 128, 300, 230, 4760, 4070}, {64, 128, 300, 400, 6870, 2550}};
+    static constexpr int split = 2400;
 };
 template <>
 struct TileCosts<GemmF8b> {
-    static constexpr TileShape shape[kTileShapes] = {{128, 128, 850, 1060}, {64, 64, 420, 270}, {32, 128, 540, 300}, {64, 128, 600, 500}};
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 820, 1060, 8300, 8300}, {64, 64, 390, 260, 4770, 1190}, {32, 128, 550, 330, 4610, 1140}, {64, 128, 640, 500, 6430, 1450}};
+    static constexpr int split = 2600;
 };
-template <>
-struct TileCosts<GemmF8W> {
-    static constexpr TileShape shape[kTileShapes] = {{128, 128, 2100, 2400}, {64, 64, 840, 690}, {32, 128, 780, 600}, {64, 128, 1150, 960}};
+template <class Val>
+struct TileCosts<GemmF32<Val>> {
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 2050, 1800, 10800, 10800}, {64, 64, 785, 575, 5300, 2200}, {32, 128, 820, 535, 4650, 3150}, {64, 128, 1055, 840, 7200, 2770}};
+    static constexpr int split = 3000;
 };
-template <>
-struct TileCosts<GemmI8W> : TileCosts<GemmF8W> {};
 
 template <>
 struct TileCosts<GemmW4> {
-    static constexpr TileShape shape[kTileShapes] = {{128, 128, 900, 800}, {64, 64, 400, 300}, {32, 128, 640, 325}, {64, 128, 680, 490}};
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 830, 500, 7500, 6850}, {64, 64, 330, 230, 4870, 1170}, {32, 128, 580, 380, 5020, 1020}, {64, 128, 560, 410, 6810, 2460}};
+    static constexpr int split = 2200;
 };
 template <>
 struct TileCosts<GemmW4GateUp> {
-    static constexpr TileShape shape[kTileShapes] = {{128, 128, 820, 780}, {64, 64, 0, 0}, {32, 128, 0, 0}, {64, 128, 650, 525}};
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 820, 780, 3000, 0}, {64, 64, 0, 0, 0, 0}, {32, 128, 0, 0, 0, 0}, {64, 128, 650, 525, 3000, 0}};
+    static constexpr int split = 3000;
 };
 template <>
 struct TileCosts<GemmW4H> {
-    static constexpr TileShape shape[kTileShapes] = {{128, 128, 1500, 1900}, {64, 64, 720, 570}, {32, 128, 810, 475}, {64, 128, 1000, 815}};
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 1500, 1900, 3000, 0}, {64, 64, 720, 570, 3000, 0}, {32, 128, 810, 475, 3000, 0}, {64, 128, 1000, 815, 3000, 0}};
+    static constexpr int split = 3000;
 };
 
-constexpr int kTileDma = -1;  // the LDS-DMA kernels' 128 x 256 tiles
+// The LDS-DMA kernels' 128 x 256 tiles: a 128-byte stage takes t with up to half of the
+// CUs at work and t + busy with all of them (M = 1024, N = K = 4096, 128 blocks: 25.4 us;
+// M = 2048, 256 blocks: 37 us).
+constexpr int kTileDma = -1;
+struct DmaCost {
+    int t, busy, f1, f2;
+};
+
+inline int64_t dma_ns(const DmaCost& c, int64_t m, int64_t n, int64_t k) {
+    const int64_t cus = device_cu_count(), blocks = ((m + 127) / 128) * ((n + 255) / 256);
+    const int64_t full = blocks / cus, rest = blocks % cus, rounds = full + (rest > 0);
+    int64_t stage = full * (c.t + c.busy);
+    if (rest) stage += c.t + c.busy * std::max<int64_t>(0, 2 * rest - cus) / cus;
+    const int64_t ns = c.f1 + c.f2 * (rounds - 1) + k / 128 * stage;
+    // stores at 3.1 TB/s; weights past 16 MiB hold the loads up by some of their read
+    return std::max(ns, m * n * 4 / 3100) + std::max<int64_t>(0, n * k - (16 << 20)) / 6000;
+}
 
 struct TilePlan {
     int shape, split, tiles_m, tiles_n;
     int64_t part_bytes, ns;
 };
 
-// The shape and K split with the smallest estimate: rounds of blocks over the CUs
-// times the stages of a block times the stage's time; a split adds the finishing
-// launch (3 us) and its partial sums' traffic (4 TB/s) and is worth it where the
-// tiles alone leave CUs idle.  `dma_stage` > 0: the LDS-DMA kernel serves these
-// operands at that time per 128-byte stage.
+// The shape and K split with the smallest estimate; a split adds the finishing launch
+// and its partial sums' traffic (4 TB/s).  `dma`: the LDS-DMA kernel serves these operands.
 template <class T>
-TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int dma_stage, bool may_split) {
+TilePlan tile_plan(int64_t m, int64_t n, int64_t k, const DmaCost* dma, bool may_split) {
     const int64_t cus = device_cu_count();
     const int64_t stages = (k + 8 * T::A::kElems - 1) / (8 * T::A::kElems);
-    TilePlan best{kTile64x128, 1, 0, 0, 0, 0};
-    int64_t best_ns = INT64_MAX;
-    if (dma_stage > 0) {
-        const int64_t blocks = ((m + 127) / 128) * ((n + 255) / 256);
-        best.shape = kTileDma;
-        best_ns = (blocks + cus - 1) / cus * (k / 128) * dma_stage + 4000;
-    }
+    TilePlan best{kTile64x128, 1, 0, 0, 0, INT64_MAX};
+    if (dma) best = TilePlan{kTileDma, 1, 0, 0, 0, dma_ns(*dma, m, n, k)};
     for (int c = 0; c < kTileShapes; ++c) {
         if (T::kGateUp && (c == kTile64x64 || c == kTile32x128)) continue;  // two column tiles per wave
         const TileShape& t = TileCosts<T>::shape[c];
@@ -736,14 +752,11 @@ TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int dma_stage, bool may_spli
         for (int split : {1, 2, 3, 4, 6, 8, 12, 16}) {
             if (split > 1 && (!may_split || stages < 4 * split || tm * tn * split > 4 * cus)) break;
             const int64_t rounds = (tm * tn * split + cus - 1) / cus, per = (stages + split - 1) / split;
-            int64_t ns = rounds == 1 ? t.t1 * per : std::max<int64_t>(t.t1, rounds * t.t2) * per;
-            ns += 3000;
+            int64_t ns = rounds == 1 ? t.f1 + t.t1 * per
+                                     : std::max<int64_t>(t.f1, rounds * t.f2) + std::max<int64_t>(t.t1, rounds * t.t2) * per;
             const int64_t part = split * m * n * static_cast<int64_t>(sizeof(typename T::part_t));
-            if (split > 1) ns += 3000 + 2 * part / 4000;
-            if (ns < best_ns) {
-                best_ns = ns;
-                best = TilePlan{c, split, 0, 0, split > 1 ? part : 0, ns};
-            }
+            if (split > 1) ns += TileCosts<T>::split + 2 * part / 4000;
+            if (ns < best.ns) best = TilePlan{c, split, 0, 0, split > 1 ? part : 0, ns};
         }
     }
     if (best.shape != kTileDma) {

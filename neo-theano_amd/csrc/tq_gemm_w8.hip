@@ -53,7 +53,7 @@ int launch_gemv(const float* x, int64_t m, const uint8_t* q, const float* s, con
 template <class T>
 int64_t workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (n <= 0 || k <= 0 || gemv_runs(m, n, k) || tiny(m, n, k) || !tile_fits(m, n, k)) return 0;
-    return tile_plan<T>(m, n, k, 0, true).part_bytes;
+    return tile_plan<T>(m, n, k, nullptr, true).part_bytes;
 }
 
 template <class T>
@@ -68,7 +68,7 @@ int weight_only(const float* x, int64_t m, const typename T::W::elem_t* q, const
     if (gemv_runs(m, n, k)) return launch_gemv(x, m, q, s, bias, n, k, y, stream);
     const hipStream_t st = as_hip(stream);
     if (tiny(m, n, k) || !tile_fits(m, n, k)) return launch_linear_8bit_generic(x, m, q, s, bias, n, k, y, st);
-    const TilePlan plan = tile_plan<T>(m, n, k, 0, true);
+    const TilePlan plan = tile_plan<T>(m, n, k, nullptr, true);
     TQ_REQUIRE(plan.part_bytes == 0 || (workspace && aligned(workspace, 8) && workspace_bytes >= plan.part_bytes),
                "%s: workspace of %lld bytes, %lld needed", what, (long long)workspace_bytes,
                (long long)plan.part_bytes);

@@ -93,7 +93,8 @@ __global__ __launch_bounds__(kGenBlock) void k_gemm_w8a8_generic(const int8_t* _
     }
 }
 
-// FP8 (e4m3) codes: products exact in f32, f32 sum over K, then the scales.
+// FP8 (e4m3) codes: products exact in f32, f64 sum over K (as the tiles of tq_gemm_tile.h
+// that take the larger sizes), then the scales.
 __global__ __launch_bounds__(kGenBlock) void k_gemm_fp8_generic(const uint8_t* __restrict__ qa,
                                                                 const float* __restrict__ sa,
                                                                 const uint8_t* __restrict__ qw,
@@ -106,11 +107,12 @@ __global__ __launch_bounds__(kGenBlock) void k_gemm_fp8_generic(const uint8_t* _
     const int64_t i = out / n, j = out % n;
     const uint8_t* ar = qa + i * k;
     const uint8_t* wr = qw + j * k;
-    float acc = 0.f;
+    double acc = 0.0;
     for (int64_t p = lane; p < k; p += kWave)
-        acc += code_value(ar[p]) * code_value(wr[p]);
-    acc = wave_sum(acc);
-    if (lane == 0) y[out] = fmaf(acc * sa[i], sw[j], bias ? bias[j] : 0.f);
+        acc += static_cast<double>(code_value(ar[p]) * code_value(wr[p]));
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kWave);
+    if (lane == 0) y[out] = fmaf(static_cast<float>(acc) * sa[i], sw[j], bias ? bias[j] : 0.f);
 }
 
 unsigned generic_grid(int64_t outputs) { return static_cast<unsigned>((outputs + kGenWaves - 1) / kGenWaves); }

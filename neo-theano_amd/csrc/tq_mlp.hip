@@ -41,7 +41,7 @@ bool tiny(int64_t m, int64_t n, int64_t k) { return m * n <= 1 << 22 && m * n * 
 
 W4TileCost w4_linear_tile_cost(int64_t m, int64_t n, int64_t k) {
     if (k == 0 || tiny(m, n, k) || !tile_fits(m, n, k)) return W4TileCost{0, 0};
-    const TilePlan plan = tile_plan<GemmW4>(m, n, k, 0, true);
+    const TilePlan plan = tile_plan<GemmW4>(m, n, k, nullptr, true);
     return W4TileCost{plan.ns, plan.part_bytes};
 }
 
@@ -50,13 +50,13 @@ int launch_w4_linear_tile(const uint16_t* x_bf16, int64_t m, const uint8_t* pack
                           const char* what) {
     if (k == 0 || tiny(m, n, k) || !tile_fits(m, n, k))
         return launch_linear_w4_generic(x_bf16, m, packed, s_f16, bias, n, k, y, st);
-    const TilePlan plan = tile_plan<GemmW4>(m, n, k, 0, part != nullptr);
+    const TilePlan plan = tile_plan<GemmW4>(m, n, k, nullptr, part != nullptr);
     return launch_tile<GemmW4>(plan, w4_args(x_bf16, packed, s_f16, bias, m, n, k, y, part), st, what);
 }
 
 W4TileCost mlp_tile_cost(int64_t m, int64_t d, int64_t f) {
     if (!tile_fits(m, 2 * f, d) || !tile_fits(m, d, f)) return W4TileCost{INT64_MAX, 0};
-    const TilePlan gu = tile_plan<GemmW4GateUp>(m, 2 * f, d, 0, true), dn = tile_plan<GemmW4H>(m, d, f, 0, true);
+    const TilePlan gu = tile_plan<GemmW4GateUp>(m, 2 * f, d, nullptr, true), dn = tile_plan<GemmW4H>(m, d, f, nullptr, true);
     return W4TileCost{gu.ns + dn.ns, align256(4 * m * f) + std::max(gu.part_bytes, dn.part_bytes)};
 }
 
@@ -69,10 +69,10 @@ int launch_mlp_tile(const uint16_t* x_bf16, int64_t m, int64_t d, int64_t f, con
     TileArgs gu = w4_args(x_bf16, gate_packed, gate_s, nullptr, m, 2 * f, d, h, part);
     gu.w2 = up_packed;
     gu.sg2 = up_s;
-    const int rc = launch_tile<GemmW4GateUp>(tile_plan<GemmW4GateUp>(m, 2 * f, d, 0, may_split), gu, st,
+    const int rc = launch_tile<GemmW4GateUp>(tile_plan<GemmW4GateUp>(m, 2 * f, d, nullptr, may_split), gu, st,
                                              "tq_mlp_w4g128 (gate/up)");
     if (rc != TQ_OK) return rc;
-    return launch_tile<GemmW4H>(tile_plan<GemmW4H>(m, d, f, 0, may_split),
+    return launch_tile<GemmW4H>(tile_plan<GemmW4H>(m, d, f, nullptr, may_split),
                                 w4_args(h, down_packed, down_s, nullptr, m, d, f, y, part), st,
                                 "tq_mlp_w4g128 (down)");
 }

@@ -89,6 +89,37 @@ def test_fp8_any_shape(tq, m, n, k, with_ws):
     assert rel < 1e-6, rel  # the fp8 matrix instructions' own sums would be 1.5e-5 off
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 1000, 1000), (1, 5000, 777), (64, 64, 64), (200, 64, 64), (3, 17, 100)])
+@pytest.mark.parametrize("with_ws", [False, True])
+def test_a8_smallest_calls(tq, m, n, k, with_ws):
+    """The smallest products, a wave per output: exact sums for INT8, FP8 summed in f64."""
+    import torch
+
+    y, acc, prod, _ = _run(torch, False, _codes(torch, (m, k), 17, False), _codes(torch, (n, k), 18, False), m, n, k,
+                           True, 1, with_ws)
+    assert torch.equal(acc.double(), prod)
+    y, _, _, ref = _run(torch, True, _codes(torch, (m, k), 19, True), _codes(torch, (n, k), 20, True), m, n, k, False, 1,
+                        with_ws)
+    # the sum to f32 and the products with the two scales: three roundings
+    assert bool(((y - ref).abs() <= 3.01 * 2.0 ** -24 * ref.abs()).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(700, 4096, 256), (700, 4096, 384), (256, 16384, 128), (1024, 1008, 256),
+                                   (130, 2064, 512), (512, 528, 2048)])
+@pytest.mark.parametrize("with_ws", [False, True])
+def test_a8_aligned_shapes(tq, m, n, k, with_ws):
+    """Sizes that the LDS-DMA kernels and the tiles share (K % 128, N % 16, 16-byte aligned)."""
+    import torch
+
+    y, acc, prod, ref = _run(torch, False, _codes(torch, (m, k), 17, False), _codes(torch, (n, k), 18, False), m, n, k,
+                             True, 0, with_ws)
+    assert torch.equal(acc.double(), prod)
+    assert bool(((y - ref).abs() <= 4 * 2.0 ** -24 * (ref.abs() + 1.0)).all())
+    y, _, _, ref = _run(torch, True, _codes(torch, (m, k), 19, True), _codes(torch, (n, k), 20, True), m, n, k, True, 0,
+                        with_ws)
+    assert ((y - ref).norm() / ref.norm()).item() < 6e-5  # the fp8 matrix instructions' own sums, 1.5e-5 measured
+
+
 def test_fp8_nan_code_stays_in_its_row_and_column(tq):
     import torch
 
