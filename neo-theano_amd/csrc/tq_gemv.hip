@@ -694,9 +694,9 @@ int gemv_8bit(const float* x, int64_t m, const typename Code::code_t* q, const f
     // short rows: the tokens' x still fits the registers).  A wave per output stays
     // ahead where a row is too short for a wave's 1024 k (N = 1000, K = 100: 2.1 to 2.8
     // us at 1 to 8 tokens against 3.1 to 8.1; N = 1003, K = 1000: 4.7 to 6.6 against 3.2
-    // to 5.7 at 1 to 4 tokens, 7.3 against 9.2 at 8; N = 300, K = 5000: 22 against 11 at 8).
+    // to 5.7 at 1 to 4 tokens, 7.3 against 9.2 at 8, 11 against 19 at 16; N = 300, K = 5000: 22 against 11 at 8).
     const bool vec16 = k % 16 == 0 && k <= 8 * 1024 && aligned(x, 16) && aligned(q, 16);
-    if (k < 16 || k > 16 * 1024 || (!vec16 && (k <= 512 || (m > 4 && m <= 8 && k <= 2048 && n * k <= 2 << 20))))
+    if (k < 16 || k > 16 * 1024 || (!vec16 && (k <= 512 || (m > 4 && k <= 2048 && n * k <= 2 << 20))))
         return launch_linear_8bit_generic(x, m, q, s, bias, n, k, y, st);
     if (!vec16) {
         const int64_t per = k <= 2048 ? 8 : 4;
