@@ -34,10 +34,10 @@
 // along d across the wave), both stored to LDS as 8-byte runs, with offsets
 // fixed per thread and a uniform step per item, so whole tiles load without
 // clamps; it fits two waves per SIMD in 256 registers.  Other head dimensions
-// keep the per-element loads (k_attention, one wave per SIMD).  At head dim 128
-// a launch with a block per CU or more takes 8-wave blocks (256 queries, each
-// key tile loaded and split once for all of them).  All forms give the same
-// bits.
+// keep the per-element loads (k_attention, one wave per SIMD).  Head dims past 64
+// run blocks of 3 or 6 waves (96 wide) and 4 or 8 (128 wide; up to 256 queries, each
+// key tile loaded and split once for all of them), as tq_attention_f32 picks by the
+// rounds of blocks over the CUs.  All forms give the same bits.
 #include <cmath>
 
 #include "tq_internal.h"
@@ -392,9 +392,8 @@ __device__ __forceinline__ void attention_block(const float* __restrict__ q, int
 }
 
 // Two waves per SIMD where the quad loads leave the registers for them (256 per
-// lane); the scalar form keeps one (its element loads need more).  kW = 8: the
-// wide form, 256 queries per block, each key tile loaded and split once for
-// twice as many queries.
+// lane); the scalar form keeps one (its element loads need more).  kW: waves, 32
+// queries each.
 template <int kDP, int kW>
 __global__ __launch_bounds__(kW * kWave) __attribute__((amdgpu_waves_per_eu(2))) void k_attention_vec(
     const float* __restrict__ q, int64_t ldq, const float* __restrict__ k, int64_t ldk, const float* __restrict__ v,
@@ -443,11 +442,17 @@ extern "C" int tq_attention_f32(const float* q, int64_t ldq, const float* k, int
                      kKT * std::max(ldk, ldv) + e < (int64_t(1) << 31);
     // Waves per block (32 queries each).  Head dims past 64: 8 (6 at up to 96, where a
     // thread's tile items then share a column), each key tile split once for all of them
-    // (S = 2048, 32 heads of 128: 237 us against 267 with 4), unless half as many already
-    // give at most one block per CU.
-    const int most = head_dim > 96 ? 8 : 6;
-    const int64_t half_blocks = (seq + most / 2 * kQW - 1) / (most / 2 * kQW) * heads * batch;
-    const int waves = !vec || head_dim <= 64 ? kWaves : half_blocks > device_cu_count() ? most : most / 2;
+    // (S = 2048, 32 heads of 128: 218 us against 247 with 4), unless half as many already
+    // give at most one block per CU (S = 129, 16 heads of 80: 18.7 against 21.4).  The
+    // 6-wave blocks run one to a CU, of 3/4 of the time of the 8-wave ones padded to 128,
+    // which take head dims up to 96 where they need that much fewer rounds over the CUs
+    // (S = 2048, 32 heads of 80: 196 us against 290; S = 1500: 138 against 118).
+    const int64_t cus = device_cu_count();
+    auto blocks = [&](int w) { return (seq + w * kQW - 1) / (w * kQW) * heads * batch; };
+    auto rounds = [&](int w) { return (blocks(w) + cus - 1) / cus; };
+    const bool pad = head_dim > 96 || 4 * rounds(8) < 3 * rounds(6);
+    const int most = pad ? 8 : 6;
+    const int waves = !vec || head_dim <= 64 ? kWaves : blocks(most / 2) > cus ? most : most / 2;
     const dim3 grid(static_cast<unsigned>((seq + waves * kQW - 1) / (waves * kQW)), static_cast<unsigned>(heads),
                     static_cast<unsigned>(batch));
 #define TQ_ATT(KERNEL, ...)                                                                                     \
@@ -457,7 +462,7 @@ extern "C" int tq_attention_f32(const float* q, int64_t ldq, const float* k, int
         if (vec) TQ_ATT(k_attention_vec, 32, kWaves); else TQ_ATT(k_attention, 32);
     } else if (head_dim <= 64) {
         if (vec) TQ_ATT(k_attention_vec, 64, kWaves); else TQ_ATT(k_attention, 64);
-    } else if (vec && head_dim <= 96) {
+    } else if (vec && !pad) {
         if (waves == 6) TQ_ATT(k_attention_vec, 96, 6); else TQ_ATT(k_attention_vec, 96, 3);
     } else if (vec) {
         if (waves == 8) TQ_ATT(k_attention_vec, 128, 8); else TQ_ATT(k_attention_vec, 128, kWaves);

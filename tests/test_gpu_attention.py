@@ -240,10 +240,12 @@ def test_mha_quantized_activations_stagewise(tq, oracle, mode):
 
 
 @pytest.mark.parametrize("B,S,H,D", [(1, 70, 2, 80), (2, 193, 3, 96), (1, 97, 3, 68), (1, 192, 180, 96), (1, 33, 260, 72),
-                                     (1, 257, 129, 100), (2, 31, 5, 124)])
+                                     (1, 257, 129, 100), (2, 31, 5, 124), (1, 193, 140, 80),
+                                     (2, 200, 70, 96)])
 @pytest.mark.parametrize("masked", [False, True])
 def test_attention_core_block_shapes(tq, B, S, H, D, masked):
-    """Head dims past 64 in 3- and 6-wave (up to 96) and 4- and 8-wave blocks, partial
+    """Head dims past 64 in 3- and 6-wave (up to 96) and 4- and 8-wave blocks (from 96 down to
+    80 where these take fewer rounds), partial
     query blocks and key tiles, mask rows that are not 16-byte aligned, a row masked
     everywhere: against float64."""
     import torch
