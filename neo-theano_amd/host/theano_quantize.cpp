@@ -577,9 +577,13 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
     const auto ts = reinterpret_cast<tq_stream_t>(stream);
     const float* b = bias_ ? bias_->data() : nullptr;
     const int64_t n = static_cast<int64_t>(out_), k = static_cast<int64_t>(in_);
-    // the workspace forms: a smaller or misaligned workspace is not used
-    const bool has_ws = workspace && workspace_bytes >= this->workspace_bytes(m) &&
-                        reinterpret_cast<uintptr_t>(workspace) % 256 == 0;
+    // the workspace forms: a smaller or misaligned workspace is not used, and none is
+    // needed where workspace_bytes(m) is 0
+    const size_t need = this->workspace_bytes(m);
+    const bool has_ws =
+        need == 0 || (workspace && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 256 == 0);
+    void* const ws = need ? workspace : nullptr;
+    const int64_t ws_bytes = need ? static_cast<int64_t>(workspace_bytes) : 0;
     int st = TQ_OK;
     switch (mode_) {
         case Mode::W4: {
@@ -602,8 +606,7 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
         case Mode::W8: {
             const auto* xf = static_cast<const float*>(x);
             if (has_ws) {
-                st = tq_gemm_w8(xf, m, w8_.codes.data(), w8_.scales.data(), b, n, k, workspace,
-                                static_cast<int64_t>(workspace_bytes), y, ts);
+                st = tq_gemm_w8(xf, m, w8_.codes.data(), w8_.scales.data(), b, n, k, ws, ws_bytes, y, ts);
                 break;
             }
             for (int64_t m0 = 0; m0 < m && st == TQ_OK; m0 += 16) {
@@ -626,7 +629,7 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
             st = tq_quantize_i8_rowwise(static_cast<const float*>(x), m, k, act_codes, act_scales, ts);
             if (st == TQ_OK)
                 st = has_ws ? tq_gemm_w8a8_ws(act_codes, act_scales, w8_.codes.data(), w8_.scales.data(), b, m, n, k,
-                                                 nullptr, workspace, static_cast<int64_t>(workspace_bytes), y, ts)
+                                                 nullptr, ws, ws_bytes, y, ts)
                                : tq_gemm_w8a8(act_codes, act_scales, w8_.codes.data(), w8_.scales.data(), b, m, n, k,
                                               nullptr, y, ts);
             break;
@@ -644,7 +647,7 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
                 st = tq_quantize_fp8_rowwise(static_cast<const float*>(x), m, k, qa, act_scales, ts);
                 if (st == TQ_OK)
                     st = has_ws ? tq_gemm_fp8_ws(qa, act_scales, fp8_.codes.data(), fp8_.scales.data(), b, m, n, k,
-                                                    workspace, static_cast<int64_t>(workspace_bytes), y, ts)
+                                                    ws, ws_bytes, y, ts)
                                    : tq_gemm_fp8(qa, act_scales, fp8_.codes.data(), fp8_.scales.data(), b, m, n, k, y,
                                                  ts);
                 break;
@@ -661,8 +664,7 @@ Result<void> QuantizedLinear::forward_device(const void* x, int64_t m, float* y,
         case Mode::FP8Weight: {
             const auto* xf = static_cast<const float*>(x);
             if (has_ws) {
-                st = tq_gemm_fp8_weight(xf, m, fp8_.codes.data(), fp8_.scales.data(), b, n, k, workspace,
-                                        static_cast<int64_t>(workspace_bytes), y, ts);
+                st = tq_gemm_fp8_weight(xf, m, fp8_.codes.data(), fp8_.scales.data(), b, n, k, ws, ws_bytes, y, ts);
                 break;
             }
             for (int64_t m0 = 0; m0 < m && st == TQ_OK; m0 += 16) {

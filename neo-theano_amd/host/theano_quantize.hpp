@@ -351,8 +351,10 @@ class QuantizedLinear : public Module {
                                 void* workspace = nullptr, size_t workspace_bytes = 0) const;
     static constexpr int64_t kTiledPassesMaxM = 32;
     static constexpr int64_t kFusedA8MaxM = 2;
-    // device scratch for m tokens: the w4 prefill path and the fp8 GEMV on
-    // fake-quantized activations (m <= kFusedA8MaxM); 0 otherwise
+    // device scratch for m tokens (may be 0): the w4 prefill path, the fp8 GEMV on
+    // fake-quantized activations (m <= kFusedA8MaxM), and the sizes at which the 8-bit
+    // modes split K over blocks.  Without it (256-byte aligned) w8 and fp8_weight run
+    // those sizes in GEMV passes of 16 tokens, w8a8 and fp8 unsplit.
     size_t workspace_bytes(int64_t m) const;
     // Quantized checkpoint entries under `name` (layout in theano_serialize.hpp):
     // codes and scales as stored on the device, loaded back without re-quantizing.

@@ -426,6 +426,37 @@ TEST_GPU(test_parity_quantized_linear_w8) {
     assert_close(y, ref, "w8 linear");
 }
 
+TEST_GPU(test_quantized_linear_w8_needs_no_workspace_where_it_asks_for_none) {
+    // sizes that the matrix cores run unsplit: no workspace asked for, none needed
+    const size_t m = 100, n = 1000, k = 384;
+    const auto wv = randn(n * k, 0.02, 34), xv = randn(m * k, 1.0, 35);
+    const auto w32 = f32(wv), x32 = f32(xv);
+    rocm::DeviceBuffer<float> x(m * k), y(m * n), y2(m * n), s(n);
+    x.upload(x32.data(), m * k, nullptr);
+    std::vector<float> got(m * n), want(m * n), sv(n);
+    for (bool fp8 : {false, true}) {
+        const QConfig cfg = fp8 ? QConfig{QuantDType::FP8, QuantDType::UInt8, true, true} : QConfig::default_int8();
+        const QuantizedLinear layer =
+            QuantizedLinear::from_tensors(Tensor::from_slice(wv, {n, k}), std::nullopt, cfg).unwrap();
+        ASSERT(layer.workspace_bytes(m) == 0);
+        ASSERT(layer.forward_device(x.data(), m, y.data(), nullptr).is_ok());
+        rocm::DeviceBuffer<uint8_t> q(n * k);
+        std::vector<uint8_t> qv(n * k);
+        if (fp8)
+            tqo_quantize_fp8_rowwise(w32.data(), n, k, qv.data(), sv.data());
+        else
+            tqo_quantize_i8_rowwise(w32.data(), n, k, reinterpret_cast<int8_t*>(qv.data()), sv.data());
+        q.upload(qv.data(), n * k, nullptr);
+        s.upload(sv.data(), n, nullptr);
+        ASSERT((fp8 ? tq_gemm_fp8_weight(x.data(), m, q.data(), s.data(), nullptr, n, k, nullptr, 0, y2.data(), nullptr)
+                    : tq_gemm_w8(x.data(), m, reinterpret_cast<int8_t*>(q.data()), s.data(), nullptr, n, k, nullptr, 0,
+                                 y2.data(), nullptr)) == TQ_OK);
+        y.download(got.data(), m * n, nullptr);
+        y2.download(want.data(), m * n, nullptr);
+        ASSERT(std::memcmp(got.data(), want.data(), m * n * sizeof(float)) == 0);
+    }
+}
+
 TEST_GPU(test_parity_quantized_linear_w4) {
     const size_t n = 200, k = 1024;
     const auto wv = randn(n * k, 0.02, 41);
