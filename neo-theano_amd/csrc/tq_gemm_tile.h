@@ -669,7 +669,9 @@ __global__ __launch_bounds__(256) void k_gemm_tile_finish(TileArgs p) {
 // first loads, stores) with one round of blocks (f1) and per round (f2); `split` is the
 // finishing launch's.  Fitted to every tile and split at M = 1 to 2048 and 18 weights from
 // 64 x 64 to 14336 x 4096, 4096 x 14336, 16384 x 128 and 64 x 16384, read past the caches:
-// the chosen one takes 1.01 to 1.03 times the fastest's time on average.
+// the chosen one takes 1.01 to 1.03 times the fastest's time on average.  t1 = 0: not built
+// (GateUp holds two column tiles per wave; GemmF32's three planes at 128 x 128 were the
+// fastest at none of 680 sizes).
 struct TileShape {
     int bm, bn, t1, t2, f1, f2;
 };
@@ -694,7 +696,7 @@ struct TileCosts<GemmF8b> {
 };
 template <class Val>
 struct TileCosts<GemmF32<Val>> {
-    static constexpr TileShape shape[kTileShapes] = {{128, 128, 2050, 1800, 10800, 10800}, {64, 64, 785, 575, 5300, 2200}, {32, 128, 820, 535, 4650, 3150}, {64, 128, 1055, 840, 7200, 2770}};
+    static constexpr TileShape shape[kTileShapes] = {{128, 128, 0, 0, 0, 0}, {64, 64, 785, 575, 5300, 2200}, {32, 128, 820, 535, 4650, 3150}, {64, 128, 1055, 840, 7200, 2770}};
     static constexpr int split = 3000;
 };
 
@@ -713,6 +715,11 @@ struct TileCosts<GemmW4H> {
     static constexpr TileShape shape[kTileShapes] = {{128, 128, 1500, 1900, 3000, 0}, {64, 64, 720, 570, 3000, 0}, {32, 128, 810, 475, 3000, 0}, {64, 128, 1000, 815, 3000, 0}};
     static constexpr int split = 3000;
 };
+
+template <class T>
+constexpr bool tile_built(int shape) {
+    return TileCosts<T>::shape[shape].t1 > 0;
+}
 
 // The LDS-DMA kernels' 128 x 256 tiles: a 128-byte stage takes t with up to half of the
 // CUs at work and t + busy with all of them (M = 1024, N = K = 4096, 128 blocks: 25.4 us;
@@ -746,7 +753,7 @@ TilePlan tile_plan(int64_t m, int64_t n, int64_t k, const DmaCost* dma, bool may
     TilePlan best{kTile64x128, 1, 0, 0, 0, INT64_MAX};
     if (dma) best = TilePlan{kTileDma, 1, 0, 0, 0, dma_ns(*dma, m, n, k)};
     for (int c = 0; c < kTileShapes; ++c) {
-        if (T::kGateUp && (c == kTile64x64 || c == kTile32x128)) continue;  // two column tiles per wave
+        if (!tile_built<T>(c)) continue;
         const TileShape& t = TileCosts<T>::shape[c];
         const int64_t tm = (m + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn;
         for (int split : {1, 2, 3, 4, 6, 8, 12, 16}) {
@@ -781,15 +788,16 @@ int launch_tile(const TilePlan& plan, TileArgs p, hipStream_t st, const char* wh
     p.split = plan.split;
     const unsigned grid = static_cast<unsigned>(static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.split);
     switch (plan.shape) {
-    case kTile128x128: k_gemm_tile<T, 128, 128, 2, 2, 1><<<grid, 256, 0, st>>>(p); break;
-    case kTile64x128: k_gemm_tile<T, 64, 128, 2, 2, 2><<<grid, 256, 0, st>>>(p); break;
-    default:
-        if constexpr (!T::kGateUp) {
-            if (plan.shape == kTile64x64)
-                k_gemm_tile<T, 64, 64, 2, 2, 2><<<grid, 256, 0, st>>>(p);
-            else
-                k_gemm_tile<T, 32, 128, 1, 4, 2><<<grid, 256, 0, st>>>(p);
-        }
+    case kTile128x128:
+        if constexpr (tile_built<T>(kTile128x128)) k_gemm_tile<T, 128, 128, 2, 2, 1><<<grid, 256, 0, st>>>(p);
+        break;
+    case kTile64x64:
+        if constexpr (tile_built<T>(kTile64x64)) k_gemm_tile<T, 64, 64, 2, 2, 2><<<grid, 256, 0, st>>>(p);
+        break;
+    case kTile32x128:
+        if constexpr (tile_built<T>(kTile32x128)) k_gemm_tile<T, 32, 128, 1, 4, 2><<<grid, 256, 0, st>>>(p);
+        break;
+    default: k_gemm_tile<T, 64, 128, 2, 2, 2><<<grid, 256, 0, st>>>(p);
     }
     if (p.split > 1) {
         const int rc = check_launch(what);
