@@ -58,8 +58,16 @@ def _run(torch, fp8, qa, qw, m, n, k, bias, off, with_ws):
     return y.double(), acc, prod, ref
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
-@pytest.mark.parametrize("with_ws", [False, True])
+# with a workspace, each tile form unsplit and with K split (the estimates' choices on 256
+# CUs: 128 x 128, 32 x 128, 64 x 128, 64 x 64), for INT8 and for codes widened to bf16
+I8_FORMS = [(1980, 1553, 257), (69, 6035, 10460), (67, 8784, 34), (9, 4100, 1937), (297, 10913, 699), (38, 9416, 11275),
+            (9, 37, 453), (10, 33, 1828)]
+F8B_FORMS = [(1579, 1958, 1083), (99, 8692, 5231), (75, 8718, 32), (9, 1428, 3068), (521, 9749, 33), (258, 4029, 8036),
+             (12, 1381, 33), (9, 35, 1256)]
+
+
+@pytest.mark.parametrize("m,n,k,with_ws", [(*s, ws) for s in SHAPES for ws in (False, True)] +
+                         [(*s, True) for s in I8_FORMS])
 def test_w8a8_any_shape_exact(tq, m, n, k, with_ws):
     import torch
 
@@ -72,8 +80,8 @@ def test_w8a8_any_shape_exact(tq, m, n, k, with_ws):
         assert bool(((y - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
-@pytest.mark.parametrize("with_ws", [False, True])
+@pytest.mark.parametrize("m,n,k,with_ws", [(*s, ws) for s in SHAPES for ws in (False, True)] +
+                         [(*s, True) for s in F8B_FORMS])
 def test_fp8_any_shape(tq, m, n, k, with_ws):
     import torch
 
@@ -105,10 +113,13 @@ def test_a8_smallest_calls(tq, m, n, k, with_ws):
 
 
 @pytest.mark.parametrize("m,n,k", [(700, 4096, 256), (700, 4096, 384), (256, 16384, 128), (1024, 1008, 256),
-                                   (130, 2064, 512), (512, 528, 2048)])
+                                   (130, 2064, 512), (512, 528, 2048), (265, 9808, 128), (306, 10528, 2560),
+                                   (67, 8528, 256), (10, 1392, 9344), (642, 10880, 128), (33, 8256, 6016), (17, 32, 896),
+                                   (21, 32, 1792), (64, 4096, 14336)])
 @pytest.mark.parametrize("with_ws", [False, True])
 def test_a8_aligned_shapes(tq, m, n, k, with_ws):
-    """Sizes that the LDS-DMA kernels and the tiles share (K % 128, N % 16, 16-byte aligned)."""
+    """Sizes that the LDS-DMA kernels and the tiles share (K % 128, N % 16, 16-byte aligned),
+    among them every tile form of the fp8 matrix instructions, unsplit and with K split."""
     import torch
 
     y, acc, prod, ref = _run(torch, False, _codes(torch, (m, k), 17, False), _codes(torch, (n, k), 18, False), m, n, k,
@@ -118,6 +129,39 @@ def test_a8_aligned_shapes(tq, m, n, k, with_ws):
     y, _, _, ref = _run(torch, True, _codes(torch, (m, k), 19, True), _codes(torch, (n, k), 20, True), m, n, k, True, 0,
                         with_ws)
     assert ((y - ref).norm() / ref.norm()).item() < 6e-5  # the fp8 matrix instructions' own sums, 1.5e-5 measured
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 5, 17), (17, 1003, 1000), (77, 130, 4099), (33, 528, 2048), (64, 4096, 14336),
+                                   (12, 272, 1024), (300, 4112, 256)])
+@pytest.mark.parametrize("mode", ["w8a8", "fp8"])
+def test_linear_in_one_call(tq, m, n, k, mode):
+    """Quantize and GEMM of one call: the bits of the two calls, nothing past the workspace
+    that it asks for."""
+    import torch
+
+    from theano_quantize import _abi
+    from theano_quantize._tensor import ptr, stream
+
+    fp8 = mode == "fp8"
+    x = torch.randn(m, k, generator=torch.Generator(device="cuda").manual_seed(m), device="cuda")
+    qw = _codes(torch, (n, k), 15, fp8)
+    sw, b = torch.rand(n, device="cuda") + 0.5, torch.randn(n, device="cuda")
+    need = int(getattr(_abi.lib(), f"tq_linear_{mode}_workspace_bytes")(m, n, k))
+    ws = torch.empty(need + 256, dtype=torch.uint8, device="cuda").fill_(0xA5)
+    y, y2 = (torch.full((m, n), float("nan"), device="cuda") for _ in range(2))
+    _abi.call(f"tq_linear_{mode}", ptr(x), m, ptr(qw), ptr(sw), ptr(b), n, k, ptr(ws), need, ptr(y), stream())
+    assert bool((ws[need:] == 0xA5).all())
+    qa = torch.empty(m, k, dtype=torch.uint8, device="cuda")
+    sa = torch.empty(m, device="cuda")
+    _abi.call("tq_quantize_fp8_rowwise" if fp8 else "tq_quantize_i8_rowwise", ptr(x), m, k, ptr(qa), ptr(sa), stream())
+    nb = int(getattr(_abi.lib(), f"tq_gemm_{mode}_workspace_bytes")(m, n, k))
+    part = torch.empty(max(nb, 8) + 256, dtype=torch.uint8, device="cuda").fill_(0xA5)
+    args = [ptr(qa), ptr(sa), ptr(qw), ptr(sw), ptr(b), m, n, k] + ([] if fp8 else [None])
+    _abi.call(f"tq_gemm_{mode}_ws", *args, ptr(part), nb, ptr(y2), stream())
+    assert bool((part[nb:] == 0xA5).all())
+    assert torch.equal(y, y2)
+    with pytest.raises(tq.InvalidArgument):
+        _abi.call(f"tq_linear_{mode}", ptr(x), m, ptr(qw), ptr(sw), ptr(b), n, k, ptr(ws), need - 1, ptr(y), stream())
 
 
 def test_fp8_nan_code_stays_in_its_row_and_column(tq):
@@ -154,7 +198,8 @@ def _weight_only(torch, fp8, x, qw, m, n, k, bias, off):
 # the same edges with enough work (more than 4 Mi products) for the matrix-core kernels;
 # the smaller shapes above run a wave per output, summed in f32
 WEIGHT_SHAPES = [(17, 4160, 63), (31, 2200, 64), (33, 1025, 129), (64, 300, 255), (128, 300, 128), (65, 129, 1023),
-                 (9, 4096, 4096), (6, 1003, 4100), (512, 512, 1024), (300, 4096, 256)]
+                 (9, 4096, 4096), (6, 1003, 4100), (512, 512, 1024), (300, 4096, 256), (39, 310, 347), (18, 426, 547),
+                 (266, 9904, 34), (33, 4359, 4395), (74, 11047, 34), (543, 34, 4051)]
 
 
 @pytest.mark.parametrize("m,n,k", [s for s in SHAPES if s[0] > 8] + WEIGHT_SHAPES)
