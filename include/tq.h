@@ -279,8 +279,9 @@ int tq_gemv_w4g128_tiled(const uint16_t* x_bf16, int64_t m, const uint8_t* packe
  * bit-exact); y = fma(f32(acc) * sa[i], sw[j], bias[j] or 0).  acc may be NULL.
  * Any M, N, K and any alignment of the codes, all on the i8 MFMA.  M <= 16 with
  * N % 16 == 0, K % 64 == 0 and K <= 8192 (16-byte aligned operands): a skinny
- * kernel of N/16 blocks, 16 weight rows each; the LDS-DMA kernel's 128 x 256 tiles
- * where K % 128 == 0 and they fill the chip; register-staged tiles otherwise. */
+ * kernel of N/16 blocks, 16 weight rows each; else the LDS-DMA kernel's 128 x 256
+ * tiles (K % 128 == 0) or register-staged tiles, whichever is estimated ahead, and a
+ * wave per output for the smallest products. */
 int tq_gemm_w8a8(const int8_t* qa, const float* sa, const int8_t* qw, const float* sw,
                  const float* bias, int64_t m, int64_t n, int64_t k, int32_t* acc,
                  float* y, tq_stream_t stream);
@@ -300,7 +301,8 @@ int tq_gemm_w8a8_ws(const int8_t* qa, const float* sa, const int8_t* qw, const f
  * dequantized operands (linear.rs:111-121, tensor_ops.rs:379-410).  Any M, N, K
  * and alignment.  The FP8 MFMA kernels serve K % 128 == 0 and N % 16 == 0 with
  * 16-byte aligned qa, qw, sw, bias and y (M <= 16 with K <= 8192: a skinny kernel of
- * N/16 blocks); other cases widen the codes to bf16 (exact) for the bf16 MFMA. */
+ * N/16 blocks); other cases widen the codes to bf16 (exact) for the bf16 MFMA
+ * or, the smallest, sum them in f64 in a wave per output. */
 int tq_gemm_fp8(const uint8_t* qa, const float* sa, const uint8_t* qw, const float* sw,
                 const float* bias, int64_t m, int64_t n, int64_t k, float* y, tq_stream_t stream);
 

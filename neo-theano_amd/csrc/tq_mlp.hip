@@ -9,9 +9,10 @@
 //
 // The INT4 codes widen to bf16 exactly, so a group's 128 products are exact and its
 // f32 sum is scaled once; the down projection takes the f32 h = SiLU(gate) * up as
-// bf16 hi + lo planes.  M = 389, N = 5827, K = 256: 8.8 us, against 300 us for a wave
-// per output (N % 16 != 0 had no other kernel); FFN at M = 889, D = 4096, F = 384: 30
-// us, against 170 us for 128-row tiles that ran K unsplit.
+// bf16 hi + lo planes.  M = 389, N = 5827, K = 256: 8.3 us, against 300 us for a wave
+// per output (N % 16 != 0 had no other kernel); FFN at M = 889, D = 4096, F = 384: 44
+// us with its weights read past the caches, against 170 us for 128-row tiles that ran K
+// unsplit.
 #include "tq_gemm_tile.h"
 
 namespace tq {
