@@ -311,7 +311,7 @@ constexpr DmaCost kDmaI8{580, 400, 6200, 5500}, kDmaF8{640, 300, 6300, 6500};
 // The products of a wave per output (tq_generic.hip) in ns: 64 k a step, 105 ns each in
 // turn (N = 300, K = 4096 at one token 8.4 us) and up to 280 where several rows read the
 // same weights (15.3 us at two, 16.2 at three), 40 steps a ns over the chip (FP8, summed in
-// f64, 25), the weights at 1 TB/s for each of the first four rows; a quarter more for rows
+// f64, 30), the weights at 1 TB/s for each of the first four rows; a quarter more for rows
 // off the 64-byte segments.  Ahead of the tiles' LDS fills and finishing launch on the
 // smallest calls (FP8 at one token, N = K = 1000: 5 against 8 us; 64 x 64 x 64: 3.0 against
 // 5.3).
@@ -427,7 +427,7 @@ int gemm_fp8(const uint8_t* qa, const float* sa, const uint8_t* qw, const float*
     const TileArgs args = a8_args(qa, sa, qw, sw, bias, m, n, k, nullptr, y, ws);
     const TilePlan plan = native ? tile_plan<GemmF8>(m, n, k, &kDmaF8, ws != nullptr)
                                  : tile_plan<GemmF8b>(m, n, k, nullptr, ws != nullptr);
-    if (wave_per_output_ns(m, n, k, 25) < plan.ns)
+    if (wave_per_output_ns(m, n, k, 30) < plan.ns)
         return launch_gemm_fp8_generic(qa, sa, qw, sw, bias, m, n, k, y, st);
     if (plan.shape == kTileDma) {
         const int tm = static_cast<int>((m + kDmaBM - 1) / kDmaBM), tn = static_cast<int>((n + kDmaBN - 1) / kDmaBN);
